@@ -12,6 +12,9 @@
 // Column ranges are split across workgroups (split-K, XCD-aware) to fill all 256 CUs;
 // partial results go to a workspace and a reduction kernel sums them in a fixed order
 // and writes Y in the caller's column-major layout.
+#include <algorithm>
+#include <cmath>
+
 #include "context.hpp"
 #include "cplx.hpp"
 #include "mfma.hpp"
@@ -22,13 +25,13 @@ namespace {
 
 constexpr int kVec = kBlockVectors;
 
-// Xt[j][n] = X[j + n N] for n < nvec, 0 otherwise (j < N, n < 32).
-template <typename Rin, typename R>
+// Xt[j][n] = X[j + n N] for n < nvec, 0 otherwise (j < N, n < VT).
+template <typename Rin, typename R, int VT>
 __global__ void stage_vectors_kernel(const cx_t<Rin>* __restrict__ X, int64_t N, int nvec, cx_t<R>* __restrict__ Xt) {
     const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (idx >= N * kVec) return;
-    const int64_t j = idx / kVec;
-    const int n = static_cast<int>(idx % kVec);
+    if (idx >= N * VT) return;
+    const int64_t j = idx / VT;
+    const int n = static_cast<int>(idx % VT);
     cx_t<R> v = mk(R(0), R(0));
     if (n < nvec) {
         const cx_t<Rin> x = X[j + n * N];
@@ -54,14 +57,14 @@ struct ProductTiling<double> {
     static constexpr bool G3M = false;
 };
 
-template <typename R, bool G3M, int TW>
-__device__ inline void product_step(const cx_t<R> (&h)[TW], const cx_t<R> (&x)[2],
-                                    typename Mfma<R>::acc_t (&acc)[TW][2][G3M ? 3 : 2]) {
+template <typename R, bool G3M, int TW, int UT>
+__device__ inline void product_step(const cx_t<R> (&h)[TW], const cx_t<R> (&x)[UT],
+                                    typename Mfma<R>::acc_t (&acc)[TW][UT][G3M ? 3 : 2]) {
     using M = Mfma<R>;
 #pragma unroll
     for (int t = 0; t < TW; ++t)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < UT; ++u) {
             const cx_t<R> hv = h[t], xv = x[u];
             if (G3M) {
                 acc[t][u][0] = M::mma(hv.x + hv.y, xv.x, acc[t][u][0]);
@@ -78,12 +81,14 @@ __device__ inline void product_step(const cx_t<R> (&h)[TW], const cx_t<R> (&x)[2
 
 // 1-D grid of row_blocks * splits workgroups, block 256. Workgroup id -> (split = id %
 // splits, row block = id / splits): with splits a multiple of 8 every split, and with
-// it its slice of Xt, lives on one XCD and its L2. Partial sums to Yp[split][row][32].
+// it its slice of Xt, lives on one XCD and its L2. Partial sums to Yp[split][row][16 UT]: UT
+// 16-vector tiles, one for blocks of at most 16 vectors (half the matrix instructions, staged
+// vectors and partial sums; the kernel then streams H: N = 5184, 8 vectors, 143 -> 94 us).
 // The main loop has no conditional loads: rows past N are clamped to row N-1 once (they
 // only feed outputs that are never stored) and whole 4U-column groups are loaded
 // unconditionally, so the compiler can issue all loads of a group together; only the
 // column tail of a split is masked.
-template <typename R>
+template <typename R, int UT>
 __global__ __launch_bounds__(256, 3) void dense_product_kernel(const cx_t<R>* __restrict__ H, const cx_t<R>* __restrict__ Xt,
                                                             int64_t N, int64_t kchunk, int splits,
                                                             cx_t<R>* __restrict__ Yp) {
@@ -93,6 +98,7 @@ __global__ __launch_bounds__(256, 3) void dense_product_kernel(const cx_t<R>* __
     constexpr int TW = T::TW, U = T::U;
     constexpr bool G3 = T::G3M;
     constexpr int NACC = G3 ? 3 : 2;
+    constexpr int VT = 16 * UT;
     const int sp = blockIdx.x % splits;
     const int rb = blockIdx.x / splits;
     const int lane = threadIdx.x & 63;
@@ -103,11 +109,11 @@ __global__ __launch_bounds__(256, 3) void dense_product_kernel(const cx_t<R>* __
     const int li = lane & 15;  // row within a 16-row tile / vector within a 16-vector tile
     const int lk = lane >> 4;  // column offset 0..3 within a 4-column step
 
-    acc_t acc[TW][2][NACC];
+    acc_t acc[TW][UT][NACC];
 #pragma unroll
     for (int t = 0; t < TW; ++t)
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < UT; ++u)
 #pragma unroll
             for (int a = 0; a < NACC; ++a) acc[t][u][a] = acc_t{0, 0, 0, 0};
 
@@ -117,40 +123,40 @@ __global__ __launch_bounds__(256, 3) void dense_product_kernel(const cx_t<R>* __
         const int64_t r = row0 + 16 * t + li;
         hrow[t] = H + (r < N ? r : N - 1) + static_cast<int64_t>(lk) * N;
     }
-    const cx_t<R>* xl = Xt + static_cast<int64_t>(lk) * kVec + li;
+    const cx_t<R>* xl = Xt + static_cast<int64_t>(lk) * VT + li;
 
     const int64_t kmain = kbeg + (kend > kbeg ? (kend - kbeg) / (4 * U) * (4 * U) : 0);
     int64_t j = kbeg;
     for (; j < kmain; j += 4 * U) {
-        cx_t<R> h[U][TW], x[U][2];
+        cx_t<R> h[U][TW], x[U][UT];
 #pragma unroll
         for (int s = 0; s < U; ++s) {
             const int64_t col = j + 4 * s;
 #pragma unroll
             for (int t = 0; t < TW; ++t) h[s][t] = hrow[t][col * N];
 #pragma unroll
-            for (int u = 0; u < 2; ++u) x[s][u] = xl[col * kVec + 16 * u];
+            for (int u = 0; u < UT; ++u) x[s][u] = xl[col * VT + 16 * u];
         }
 #pragma unroll
-        for (int s = 0; s < U; ++s) product_step<R, G3, TW>(h[s], x[s], acc);
+        for (int s = 0; s < U; ++s) product_step<R, G3, TW, UT>(h[s], x[s], acc);
     }
     for (; j < kend; j += 4) {  // masked tail, fewer than 4U columns
         const bool cok = j + lk < kend;
         const int64_t col = cok ? j : kend - 1 - lk;  // keeps the lane's address inside the split
-        cx_t<R> h[TW], x[2];
+        cx_t<R> h[TW], x[UT];
 #pragma unroll
         for (int t = 0; t < TW; ++t) {
             const cx_t<R> v = hrow[t][col * N];
             h[t] = cok ? v : mk(R(0), R(0));
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const cx_t<R> v = xl[col * kVec + 16 * u];
+        for (int u = 0; u < UT; ++u) {
+            const cx_t<R> v = xl[col * VT + 16 * u];
             x[u] = cok ? v : mk(R(0), R(0));
         }
-        product_step<R, G3, TW>(h, x, acc);
+        product_step<R, G3, TW, UT>(h, x, acc);
     }
-    cx_t<R>* out = Yp + static_cast<int64_t>(sp) * N * kVec;
+    cx_t<R>* out = Yp + static_cast<int64_t>(sp) * N * VT;
 #pragma unroll
     for (int t = 0; t < TW; ++t)
 #pragma unroll
@@ -158,7 +164,7 @@ __global__ __launch_bounds__(256, 3) void dense_product_kernel(const cx_t<R>* __
             const int64_t r = row0 + 16 * t + M::out_row(lk, v);
             if (r < N) {
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
+                for (int u = 0; u < UT; ++u) {
                     R re, im;
                     if (G3) {
                         re = acc[t][u][0][v] - acc[t][u][2][v];
@@ -167,45 +173,59 @@ __global__ __launch_bounds__(256, 3) void dense_product_kernel(const cx_t<R>* __
                         re = acc[t][u][0][v];
                         im = acc[t][u][1][v];
                     }
-                    out[r * kVec + 16 * u + li] = mk(re, im);
+                    out[r * VT + 16 * u + li] = mk(re, im);
                 }
             }
         }
 }
 
 // Y[r + n N] = sum_s Yp[s][r][n] for n < nvec, summed in the output precision in a fixed
-// order. A workgroup owns 64 rows: the partial rows are read
-// with consecutive threads on consecutive (row, vector) pairs, the sums are transposed
-// through LDS and written column by column.
-template <typename R, typename Rout>
+// order (eight interleaved partial sums, so that eight loads are in flight). One output per
+// thread, 256 / VT rows per workgroup, so that a small matrix with many splits still has
+// workgroups on most CUs; the sums are transposed through LDS and written column by column.
+// Bound by the latency of its loads when small, by HBM when large: N = 900, 64 splits:
+// 129 -> 18 us (64 rows per workgroup, one load at a time, left 15 workgroups); N = 36864,
+// 8 splits of 32 vectors: 42 -> 29 us (5.2 TB/s).
+template <typename R, typename Rout, int VT>
 __global__ __launch_bounds__(256) void reduce_product_kernel(const cx_t<R>* __restrict__ Yp, int64_t N, int nvec,
                                                              int splits, cx_t<Rout>* __restrict__ Y) {
-    constexpr int kRows = 64;
-    __shared__ cx_t<Rout> tile[kRows][kVec + 1];
+    constexpr int kRows = 256 / VT, kDeep = 8;
+    __shared__ cx_t<Rout> tile[kRows][VT + 1];
     const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kRows;
-#pragma unroll
-    for (int j = 0; j < kRows * kVec / 256; ++j) {
-        const int f = threadIdx.x + 256 * j;
-        const int rr = f / kVec, n = f % kVec;
+    {
+        const int rr = threadIdx.x / VT, n = threadIdx.x % VT;
         const int64_t r = r0 + rr;
-        Rout sr = 0, si = 0;
+        Rout ar[kDeep], ai[kDeep];
+#pragma unroll
+        for (int j = 0; j < kDeep; ++j) ar[j] = ai[j] = Rout(0);
         if (r < N && n < nvec) {
-            for (int s = 0; s < splits; ++s) {
-                const cx_t<R> v = Yp[(static_cast<int64_t>(s) * N + r) * kVec + n];
-                sr += static_cast<Rout>(v.x);
-                si += static_cast<Rout>(v.y);
+            const int64_t stride = N * VT;
+            const cx_t<R>* p = Yp + r * VT + n;
+            int s = 0;
+            for (; s + kDeep <= splits; s += kDeep, p += kDeep * stride) {
+#pragma unroll
+                for (int j = 0; j < kDeep; ++j) {
+                    const cx_t<R> v = p[j * stride];
+                    ar[j] += static_cast<Rout>(v.x);
+                    ai[j] += static_cast<Rout>(v.y);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < kDeep - 1; ++j) {
+                if (s + j < splits) {
+                    const cx_t<R> v = p[j * stride];
+                    ar[j] += static_cast<Rout>(v.x);
+                    ai[j] += static_cast<Rout>(v.y);
+                }
             }
         }
-        tile[rr][n] = mk(sr, si);
+        tile[rr][n] = mk(((ar[0] + ar[4]) + (ar[1] + ar[5])) + ((ar[2] + ar[6]) + (ar[3] + ar[7])),
+                         ((ai[0] + ai[4]) + (ai[1] + ai[5])) + ((ai[2] + ai[6]) + (ai[3] + ai[7])));
     }
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kRows * kVec / 256; ++j) {
-        const int f = threadIdx.x + 256 * j;
-        const int rr = f % kRows, n = f / kRows;
-        const int64_t r = r0 + rr;
-        if (r < N && n < nvec) Y[r + static_cast<int64_t>(n) * N] = tile[rr][n];
-    }
+    const int rr = threadIdx.x % kRows, n = threadIdx.x / kRows;
+    const int64_t r = r0 + rr;
+    if (r < N && n < nvec) Y[r + static_cast<int64_t>(n) * N] = tile[rr][n];
 }
 
 // C (N x nb) = alpha A B + beta C (beta = 0: C is not read) for a tall A (N x m,
@@ -369,37 +389,73 @@ __global__ __launch_bounds__(kRedOut* kRedSlices) void gram_reduce_kernel(const 
     }
 }
 
-// Column splits of the dense product: enough workgroups to fill 256 CUs a few times over,
-// a multiple of the XCD count, at most max_splits (>= 1).
+// Vectors per tile row of a product launch: one 16-vector matrix tile for up to 16 vectors.
+int vector_tile(int nvec) { return nvec <= 16 ? 16 : kVec; }
+
+// Column splits of the dense product, at most max_splits (>= 1): the count with the smallest
+// estimated time: whole rounds of resident workgroups (three per CU) at about the product's
+// rate, or the latency of their column groups when these are few, plus the partial sums
+// written and read back, or the latency of the reduction's batches of loads. Up to N = 8192 the staged vectors fit in
+// one XCD's L2 and any count will do; beyond, a multiple of the XCD count keeps a split's
+// slice of them on one XCD. (A fixed aim of 2048 workgroups wrote 56 partial sums of every
+// row at N = 5184, as many bytes as a third of the matrix.)
 template <typename R>
-int product_splits(int64_t N, int max_splits) {
+int product_splits(int64_t N, int vt, int max_splits) {
     using T = ProductTiling<R>;
+    constexpr double kResident = 768.0;
+    const double rate = (sizeof(R) == 8 ? 55e12 : 120e12), bandwidth = 4e12;
     const int rows_wg = 64 * T::TW;
-    const int row_blocks = static_cast<int>((N + rows_wg - 1) / rows_wg);
-    int splits = std::max(1, std::min(64, (2048 + row_blocks - 1) / row_blocks));
-    splits = (splits + kXcds - 1) / kXcds * kXcds;
-    return std::max(1, std::min(splits, max_splits));
+    const double row_blocks = static_cast<double>((N + rows_wg - 1) / rows_wg);
+    const int step = (N <= 8192 || max_splits < kXcds) ? 1 : kXcds;
+    int best = 1;
+    double best_t = 1e300;
+    for (int s = step; s <= std::min(64, max_splits); s += step) {
+        const double rounds = std::ceil(row_blocks * s / kResident);
+        const double cols = std::ceil(static_cast<double>(N) / s / (4 * T::U)) * (4 * T::U);
+        // one round: every resident workgroup's columns, at the matrix cores' or at HBM's rate
+        const double per = std::max(std::max(8.0 * vt / rate, 2.0 * sizeof(R) / bandwidth) * kResident * rows_wg * cols,
+                                    1e-6 * cols / (4 * T::U));
+        const double t = rounds * per + std::max(2.0 * s * N * vt * 2.0 * sizeof(R) / bandwidth, 2e-6 * ((s + 7) / 8));
+        if (t < best_t) {
+            best_t = t;
+            best = s;
+        }
+    }
+    return best;
 }
 
-// Y = H X through the staging buffer xt (N x 32) and the partial sums yp (splits x N x 32).
-template <typename Rin, typename R, typename Rout>
-void dense_product_into(int64_t N, const cx_t<R>* H, const cx_t<Rin>* X, cx_t<Rout>* Y, int nvec, hipStream_t s,
+// Y = H X for up to 16 UT vectors through the staging buffer xt (N x 16 UT) and the partial
+// sums yp (splits x N x 16 UT).
+template <typename Rin, typename R, typename Rout, int UT>
+void dense_product_tile(int64_t N, const cx_t<R>* H, const cx_t<Rin>* X, cx_t<Rout>* Y, int nv, hipStream_t s,
                         cx_t<R>* xt, cx_t<R>* yp, int splits) {
     using T = ProductTiling<R>;
+    constexpr int VT = 16 * UT;
     const int rows_wg = 64 * T::TW;
     const int row_blocks = static_cast<int>((N + rows_wg - 1) / rows_wg);
     const int step = 4 * T::U;
     const int64_t kchunk = ((N + splits - 1) / splits + step - 1) / step * step;
     // every split owns a (possibly empty) column range and writes its partial rows
+    const int64_t tot = N * VT;
+    hipLaunchKernelGGL((stage_vectors_kernel<Rin, R, VT>), dim3((tot + 255) / 256), dim3(256), 0, s, X, N, nv, xt);
+    hipLaunchKernelGGL((dense_product_kernel<R, UT>), dim3(row_blocks * splits), dim3(256), 0, s, H, xt, N, kchunk,
+                       splits, yp);
+    hipLaunchKernelGGL((reduce_product_kernel<R, Rout, VT>), dim3((tot + 255) / 256), dim3(256), 0, s, yp, N, nv,
+                       splits, Y);
+}
+
+// max_splits: what the partial-sum buffer holds for 32 vectors per row.
+template <typename Rin, typename R, typename Rout>
+void dense_product_into(int64_t N, const cx_t<R>* H, const cx_t<Rin>* X, cx_t<Rout>* Y, int nvec, hipStream_t s,
+                        cx_t<R>* xt, cx_t<R>* yp, int max_splits) {
     for (int v0 = 0; v0 < nvec; v0 += kVec) {
         const int nv = std::min(kVec, nvec - v0);
-        const int64_t tot = N * kVec;
-        hipLaunchKernelGGL((stage_vectors_kernel<Rin, R>), dim3((tot + 255) / 256), dim3(256), 0, s, X + v0 * N, N, nv,
-                           xt);
-        hipLaunchKernelGGL((dense_product_kernel<R>), dim3(row_blocks * splits), dim3(256), 0, s, H, xt, N, kchunk,
-                           splits, yp);
-        hipLaunchKernelGGL((reduce_product_kernel<R, Rout>), dim3((N + 63) / 64), dim3(256), 0, s, yp, N, nv, splits,
-                           Y + v0 * N);
+        const int vt = vector_tile(nv);
+        const int splits = product_splits<R>(N, vt, max_splits);
+        if (vt == 16)
+            dense_product_tile<Rin, R, Rout, 1>(N, H, X + v0 * N, Y + v0 * N, nv, s, xt, yp, splits);
+        else
+            dense_product_tile<Rin, R, Rout, 2>(N, H, X + v0 * N, Y + v0 * N, nv, s, xt, yp, splits);
     }
     XATU_HIP(hipGetLastError());
 }
@@ -408,10 +464,14 @@ template <typename Rin, typename R, typename Rout>
 void dense_product(const Context& c, const cx_t<R>* H, const cx_t<Rin>* X, cx_t<Rout>* Y, int nvec, hipStream_t s,
                    DevBuf<cx_t<R>>& xt, DevBuf<cx_t<R>>& yp) {
     const int64_t N = c.N;
-    const int splits = product_splits<R>(N, 64);
-    xt.alloc(std::max<size_t>(xt.n, static_cast<size_t>(N) * kVec));
-    yp.alloc(std::max<size_t>(yp.n, static_cast<size_t>(splits) * N * kVec));
-    dense_product_into<Rin, R, Rout>(N, H, X, Y, nvec, s, xt.p, yp.p, splits);
+    size_t room = 0;  // partial sums of the largest vector block of the call
+    for (int v0 = 0; v0 < nvec; v0 += kVec) {
+        const int vt = vector_tile(std::min(kVec, nvec - v0));
+        room = std::max(room, static_cast<size_t>(product_splits<R>(N, vt, 64)) * N * vt);
+    }
+    xt.reserve(static_cast<size_t>(N) * kVec);
+    yp.reserve(room);
+    dense_product_into<Rin, R, Rout>(N, H, X, Y, nvec, s, xt.p, yp.p, 64);
 }
 
 }  // namespace
@@ -420,19 +480,14 @@ void launch_matvec64(Context& c, const double2* X, double2* Y, int nvec, hipStre
     dense_product<double, double, double>(c, c.d_H64.p, X, Y, nvec, s, c.s_xt64, c.s_yp64);
 }
 
-int64_t matvec64_scratch_elems(int64_t N, int max_splits) {
-    return N * kVec * (1 + product_splits<double>(N, max_splits));
-}
-
 void launch_matvec64_scratch(const Context& c, const double2* X, double2* Y, int nvec, double2* scratch,
                              int64_t scratch_elems, hipStream_t s) {
     const int64_t N = c.N;
-    // as many splits as the scratch holds beside the staged vectors (same kernels and, when
-    // they fit, the same splits as the allocating product)
+    // as many splits as the scratch holds beside the staged vectors, 32 vectors wide (same
+    // kernels and, when they fit, the same splits as the allocating product)
     const int max_splits = static_cast<int>(std::min<int64_t>(64, scratch_elems / (N * kVec) - 1));
     if (max_splits < 1) throw Error(XATU_ERR_INVALID_ARGUMENT, "scratch too small for the product");
-    const int splits = product_splits<double>(N, max_splits);
-    dense_product_into<double, double, double>(N, c.d_H64.p, X, Y, nvec, s, scratch, scratch + N * kVec, splits);
+    dense_product_into<double, double, double>(N, c.d_H64.p, X, Y, nvec, s, scratch, scratch + N * kVec, max_splits);
 }
 
 // Product with the FP32 matrix: on the FP16 matrix cores with split operands where the
@@ -448,19 +503,19 @@ void launch_matvec32(Context& c, const double2* X, double2* Y, int nvec, hipStre
 }
 
 void launch_stage_vectors(const double2* X, int64_t N, int nvec, double2* Xt, hipStream_t s) {
-    hipLaunchKernelGGL((stage_vectors_kernel<double, double>), dim3((N * kVec + 255) / 256), dim3(256), 0, s, X, N,
+    hipLaunchKernelGGL((stage_vectors_kernel<double, double, kVec>), dim3((N * kVec + 255) / 256), dim3(256), 0, s, X, N,
                        nvec, Xt);
 }
 void launch_stage_vectors(const double2* X, int64_t N, int nvec, float2* Xt, hipStream_t s) {
-    hipLaunchKernelGGL((stage_vectors_kernel<double, float>), dim3((N * kVec + 255) / 256), dim3(256), 0, s, X, N,
+    hipLaunchKernelGGL((stage_vectors_kernel<double, float, kVec>), dim3((N * kVec + 255) / 256), dim3(256), 0, s, X, N,
                        nvec, Xt);
 }
 void launch_reduce_partials(const double2* Yp, int64_t N, int nvec, int splits, double2* Y, hipStream_t s) {
-    hipLaunchKernelGGL((reduce_product_kernel<double, double>), dim3((N + 63) / 64), dim3(256), 0, s, Yp, N, nvec,
+    hipLaunchKernelGGL((reduce_product_kernel<double, double, kVec>), dim3((N * kVec + 255) / 256), dim3(256), 0, s, Yp, N, nvec,
                        splits, Y);
 }
 void launch_reduce_partials(const float2* Yp, int64_t N, int nvec, int splits, double2* Y, hipStream_t s) {
-    hipLaunchKernelGGL((reduce_product_kernel<float, double>), dim3((N + 63) / 64), dim3(256), 0, s, Yp, N, nvec,
+    hipLaunchKernelGGL((reduce_product_kernel<float, double, kVec>), dim3((N * kVec + 255) / 256), dim3(256), 0, s, Yp, N, nvec,
                        splits, Y);
 }
 

@@ -219,6 +219,7 @@ struct Context {
     DevBuf<float2> s_pt32;            // partial sums of the transposed-block products (split product)
     DevBuf<int2> d_herm_items;        // (row block, column chunk) work items of the split product
     int herm_items = 0;
+    int herm_chunk = 0;               // columns per work item (a multiple of kSplitRowBlock)
     int64_t herm_n = 0;               // matrix dimension the work items were laid out for
     DevBuf<float> s_colmax, s_xscale; // column maxima and power-of-two scales of the staged vectors
     DevBuf<double> s_xinv;            // inverse combined scales applied by the split-product reduction

@@ -25,14 +25,16 @@
 // parts pass through a per-wave LDS buffer so that a lane holds one k and eight i, the
 // vectors being staged a second time in that i order (Xt). Complex products use two FP32
 // accumulators per tile, the negated imaginary parts of H supplying the minus signs.
-// The columns are cut into chunks of 2048 (work items (b, chunk) for the chunks at or
-// below b's diagonal block); the direct sums go to one slot per chunk, the transposed
+// The columns are cut into chunks (work items (b, chunk) for the chunks at or below b's
+// diagonal block, the chunk length chosen per dimension by lay_out_items); the direct sums go to one slot per chunk, the transposed
 // sums (the four waves' added in LDS) to one slot per row block, and a reduction adds
 // the slots of each row in a fixed order. The last step of a column may read up to 31
 // entries past its end: the staged vectors are zero there and the entries read are finite
 // (32 zero entries of padding after the matrix, zeroed heads of the unbuilt columns).
 #include <algorithm>
 #include <cmath>
+#include <functional>
+#include <queue>
 #include <vector>
 
 #include "context.hpp"
@@ -202,7 +204,6 @@ __device__ inline HFrag16 split_h(const float4 (&r)[4], float sH) {
 constexpr int kHermTiles = 4;
 constexpr int kHermRows = 4 * 16 * kHermTiles;
 static_assert(kHermRows == kSplitRowBlock, "row block of the split product");
-constexpr int kHermChunk = 4096;   // columns per work item, a multiple of kHermRows
 constexpr int kTrRow = 72;         // FP16 entries per row of the transposition buffer (64 + 8 padding)
 constexpr int kCbRow = 34;         // complex entries per row of the combine buffer (32 + 2 padding)
 
@@ -234,7 +235,7 @@ template <int TW, bool PRESPLIT>
 __global__ __launch_bounds__(256, 1) void herm_product_kernel(const float2* __restrict__ H,
                                                               const XFrag16* __restrict__ Xs,
                                                               const XFrag16* __restrict__ Xt,
-                                                              const int2* __restrict__ items, int64_t N, float sH,
+                                                              const int2* __restrict__ items, int chunk, int64_t N, float sH,
                                                               float2* __restrict__ Pn, float2* __restrict__ Pt) {
     static_assert(TW == 4, "the transposed fragments assume 64 rows per wave");
     __shared__ HermLds lds;
@@ -244,8 +245,8 @@ __global__ __launch_bounds__(256, 1) void herm_product_kernel(const float2* __re
     const int li = lane & 15, g = lane >> 4;
     const int64_t rb0 = static_cast<int64_t>(b) * kHermRows;
     const int64_t row0 = rb0 + wave * (16 * TW);
-    const int64_t cbeg = static_cast<int64_t>(c) * kHermChunk;
-    const int64_t kend = min(N, cbeg + kHermChunk);
+    const int64_t cbeg = static_cast<int64_t>(c) * chunk;
+    const int64_t kend = min(N, cbeg + chunk);
     const bool diag = cbeg <= rb0;
     const int64_t kbeg = diag ? rb0 : cbeg;
     const int nd = diag ? static_cast<int>((min(kend, rb0 + kHermRows) - rb0 + 31) / 32) : 0;
@@ -482,7 +483,7 @@ struct Herm2Lds {
 __global__ __launch_bounds__(256, 1) void herm_product_wave_kernel(const float2* __restrict__ H,
                                                                    const XFrag16* __restrict__ Xs,
                                                                    const XFrag16* __restrict__ Xt,
-                                                                   const int2* __restrict__ items, int64_t N,
+                                                                   const int2* __restrict__ items, int chunk, int64_t N,
                                                                    float2* __restrict__ Pn, float2* __restrict__ Pt) {
     __shared__ Herm2Lds lds;
     const int2 bc = items[blockIdx.x];
@@ -490,8 +491,8 @@ __global__ __launch_bounds__(256, 1) void herm_product_wave_kernel(const float2*
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int li = lane & 15, g = lane >> 4;
     const int64_t rb0 = static_cast<int64_t>(b) * kHermRows;
-    const int64_t cbeg = static_cast<int64_t>(c) * kHermChunk;
-    const int64_t kend = min(N, cbeg + kHermChunk);
+    const int64_t cbeg = static_cast<int64_t>(c) * chunk;
+    const int64_t kend = min(N, cbeg + chunk);
     const bool diag = cbeg <= rb0;
     const int64_t kbeg = diag ? rb0 : cbeg;
     const int nd = diag ? static_cast<int>((min(kend, rb0 + kHermRows) - rb0 + 31) / 32) : 0;
@@ -699,14 +700,14 @@ __global__ __launch_bounds__(256, 1) void herm_product_wave_kernel(const float2*
 constexpr int kReduceRows = 8;  // rows per workgroup of the reduction (256 threads = 8 rows x 32 vectors)
 __global__ __launch_bounds__(256) void herm_reduce_kernel(const float2* __restrict__ Pn,
                                                           const float2* __restrict__ Pt, int64_t N, int nvec,
-                                                          int nchunks, const double* __restrict__ scale,
+                                                          int nchunks, int chunk, const double* __restrict__ scale,
                                                           double2* __restrict__ Y) {
     constexpr int kRows = kReduceRows;  // one output (row, vector) per thread
     __shared__ double2 tile[kRows][kVec + 1];
     // the last rows (the most transposed-block slots) first
     const int64_t r0 = static_cast<int64_t>(gridDim.x - 1 - blockIdx.x) * kRows;
     const int b = static_cast<int>(r0 / kHermRows);
-    const int c0 = static_cast<int>(static_cast<int64_t>(b) * kHermRows / kHermChunk);
+    const int c0 = static_cast<int>(static_cast<int64_t>(b) * kHermRows / chunk);
 #pragma unroll
     for (int j = 0; j < kRows * kVec / 256; ++j) {
         const int f = threadIdx.x + 256 * j;
@@ -858,27 +859,56 @@ void split_product_scale(Context& c) {
     if (c.h16_scale > 0.0f) lay_out_items(c);
 }
 
-// Work items (row block, column chunk) of the split product, the longest first; laid out
-// once per matrix dimension.
+// Work items (row block, column chunk) of the split product, the longest first, laid out once
+// per matrix dimension. The chunk is the multiple of the row block with the shortest schedule
+// of its items on the CUs (one workgroup each; about 22 us per 256 x 256 block and 8 us to
+// start and end an item, both measured) plus the direct partial sums an item writes and the
+// reduction reads back: at small N short chunks, so that every CU has work (a fixed 4096
+// left 84 items, the longest 16 blocks, at N = 9216), at N = 36864 chunks of 1536. Products
+// with staging and reduction, 4096 -> now: N = 2304 217 -> 58 us, 5184 361 -> 67, 9216
+// 387 -> 136, 14400 414 -> 280, 20736 517 -> 517, 36864 1572 -> 1571.
 static void lay_out_items(Context& c) {
     const int64_t N = c.N;
     if (c.herm_n == N && c.herm_items > 0) return;
-    const int B = static_cast<int>((N + kHermRows - 1) / kHermRows);
-    const int C = static_cast<int>((N + kHermChunk - 1) / kHermChunk);
-    std::vector<int2> it;
-    std::vector<int64_t> len;
-    for (int ch = 0; ch < C; ++ch)
-        for (int b = 0; b < B; ++b) {
-            const int64_t rb0 = static_cast<int64_t>(b) * kHermRows, cb = static_cast<int64_t>(ch) * kHermChunk;
-            if (rb0 >= cb + kHermChunk) continue;
-            it.push_back(make_int2(b, ch));
-            len.push_back(std::min<int64_t>(N, cb + kHermChunk) - std::max(rb0, cb));
+    const int64_t B = (N + kHermRows - 1) / kHermRows;
+    constexpr int kCus = 256, kMaxItems = 2048;
+    struct Item {
+        int2 at;
+        int64_t len;
+    };
+    std::vector<Item> best;
+    double best_us = 1e300;
+    for (int blocks : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        const int64_t chunk = static_cast<int64_t>(blocks) * kHermRows;
+        // skip layouts of far more items than CUs while a longer chunk remains
+        if (blocks < 16 && B * B / (2 * blocks) > kMaxItems) continue;
+        std::vector<Item> it;
+        for (int64_t ch = 0; ch * chunk < N; ++ch)
+            for (int64_t b = 0; b < B; ++b) {
+                const int64_t rb0 = b * kHermRows, cb = ch * chunk;
+                if (rb0 >= cb + chunk) continue;
+                it.push_back({make_int2(static_cast<int>(b), static_cast<int>(ch)), std::min(N, cb + chunk) - std::max(rb0, cb)});
+            }
+        std::stable_sort(it.begin(), it.end(), [](const Item& x, const Item& y) { return x.len > y.len; });
+        std::priority_queue<double, std::vector<double>, std::greater<double>> cu(std::greater<double>(),
+                                                                                 std::vector<double>(kCus, 0.0));
+        double last = 0.0;
+        for (const Item& i : it) {
+            const double t = cu.top() + 8.0 + 22.0 * static_cast<double>(i.len) / kHermRows;
+            cu.pop();
+            cu.push(t);
+            last = std::max(last, t);
         }
-    std::vector<size_t> order(it.size());
-    for (size_t i = 0; i < order.size(); ++i) order[i] = i;
-    std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return len[x] > len[y]; });
-    std::vector<int2> sorted(it.size());
-    for (size_t i = 0; i < order.size(); ++i) sorted[i] = it[order[i]];
+        // microseconds for the direct partial sums, 64 KB per item written and read
+        const double us = last + it.size() * 2.0 * kHermRows * kVec * sizeof(float2) / 5e6;
+        if (us < best_us) {
+            best_us = us;
+            best.swap(it);
+            c.herm_chunk = static_cast<int>(chunk);
+        }
+    }
+    std::vector<int2> sorted(best.size());
+    for (size_t i = 0; i < best.size(); ++i) sorted[i] = best[i].at;
     c.d_herm_items.alloc(sorted.size());
     XATU_HIP(hipMemcpy(c.d_herm_items.p, sorted.data(), sorted.size() * sizeof(int2), hipMemcpyHostToDevice));
     c.herm_items = static_cast<int>(sorted.size());
@@ -916,7 +946,7 @@ bool split_product_available(const Context& c) {
 void launch_matvec_split16(Context& c, const double2* X, double2* Y, int nvec, hipStream_t s) {
     const int64_t N = c.N;
     const int B = static_cast<int>((N + kHermRows - 1) / kHermRows);
-    const int C = static_cast<int>((N + kHermChunk - 1) / kHermChunk);
+    const int C = static_cast<int>((N + c.herm_chunk - 1) / c.herm_chunk);
     const int64_t nsteps = (N + 31) / 32;
     const int64_t ngroups = 4 * static_cast<int64_t>(B);
     const int64_t rows = (N + kMaxChunks - 1) / kMaxChunks;
@@ -944,13 +974,13 @@ void launch_matvec_split16(Context& c, const double2* X, double2* Y, int nvec, h
                            c.s_xscale.p, xs, xt);
         if (c.h32_presplit) {
             hipLaunchKernelGGL(herm_product_wave_kernel, dim3(c.herm_items), dim3(256), 0, s, c.d_H32.p, xs, xt,
-                               c.d_herm_items.p, N, c.s_yp32.p, c.s_pt32.p);
+                               c.d_herm_items.p, c.herm_chunk, N, c.s_yp32.p, c.s_pt32.p);
         } else {
             hipLaunchKernelGGL((herm_product_kernel<kHermTiles, false>), dim3(c.herm_items), dim3(256), 0, s,
-                               c.d_H32.p, xs, xt, c.d_herm_items.p, N, sH, c.s_yp32.p, c.s_pt32.p);
+                               c.d_H32.p, xs, xt, c.d_herm_items.p, c.herm_chunk, N, sH, c.s_yp32.p, c.s_pt32.p);
         }
         hipLaunchKernelGGL(herm_reduce_kernel, dim3((N + kReduceRows - 1) / kReduceRows), dim3(256), 0, s, c.s_yp32.p, c.s_pt32.p, N, nv, C,
-                           c.s_xinv.p, Y + static_cast<int64_t>(v0) * N);
+                           c.herm_chunk, c.s_xinv.p, Y + static_cast<int64_t>(v0) * N);
     }
     XATU_HIP(hipGetLastError());
 }

@@ -38,6 +38,10 @@ DEVICE_SOURCES = [
     "device/hf.hip",
     "device/band_adjoint.hip",
     "device/convolution.hip",
+    "device/conv_rows_in64.hip",
+    "device/conv_rows_out64.hip",
+    "device/conv_rows_in32.hip",
+    "device/conv_rows_out32.hip",
     "device/split_product.hip",
     "device/projected_eigen.hip",
     "device/capi.hip",

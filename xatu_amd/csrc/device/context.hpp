@@ -348,6 +348,10 @@ void launch_conv64(Context& c, const double2* X, double2* Y, int nvec, hipStream
 void launch_conv32(Context& c, const double2* X, double2* Y, int nvec, hipStream_t s);
 // S[(n nmesh + q) NA^2 + a + NA b] = sum_k G_ab(k, k+q) for ns <= 32 states (FFT autocorrelation).
 void conv_pair_density(Context& c, const double2* psi, int ns, double2* S);
+// On meshes of the row and column transforms (conv_rows_available): the adjoint of the lattice sums
+// on the cells, shat[(s npairs + p) nR + R], for ns <= 32 states.
+bool conv_rows_available(Context& c);
+void conv_cell_density(Context& c, const double2* psi, int ns, double* shat);
 // Matrix-free products Y = H X (complex FP64 vectors) with tiles of H recomputed in
 // FP64 / FP32 arithmetic inside the product (FP32: FP32 tiles, FP32 accumulation).
 void launch_matfree64(Context& c, const double2* X, double2* Y, int nvec, hipStream_t s);

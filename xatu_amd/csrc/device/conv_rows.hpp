@@ -1,0 +1,404 @@
+// Transforms of the convolution product on 2-D meshes with sides n = A B (fft_stages.hpp): three
+// kernels between which the correlation buffer holds only the window of first-axis frequencies
+// where the kernel spectrum is not zero.
+//
+// The spectrum of the lattice-sum table on the mesh is the potential itself: the table is
+// M_ab(Delta) = (1/T) sum_R V_ab(R) e^{i Delta R}, so its transform at frequency xi is
+// V_ab(R)/T for the cells R = -xi (a < b) or R = +xi (a >= b, stored conjugated), real, and
+// zero outside the cutoff: |xi_0| <= w of the n frequencies of an axis matter (N = 36864,
+// cutoff 25 cells: 57 of 96). The buffer is
+//   G[(o1 batch + b) W + j],  o1 the mesh row, b = (al norb + be) nvec + v, xi_0 = (w0 + j) mod n.
+//  conv_rows_in_kernel   z_{al be}(k) = sum_c C_k[al, c] u[v][c][be][k] along a mesh row and its
+//                        transform, in registers, the window to G
+//  conv_columns_kernel   per (b, j): transform along o1, times the spectrum, inverse (in place)
+//  conv_rows_out_kernel  inverse transform along a row from the window, contracted at once with
+//                        the band coefficients: t[v][c][be][k] = sum_al conj(C_k[al, c]) w(k)
+// so that z and w at the mesh points never go to memory: the buffer is written and read twice
+// at W / n of its size. Measured against one kernel that held whole planes in LDS between a
+// contraction that wrote z and one that read w (32 FP32 vectors, 36 orbitals, 120 x 120; 16 FP64
+// vectors, 18 orbitals, 96 x 96): 1.77 + 4.12 + 1.65 -> 1.55 + 1.14 + 1.72 + 0.16 ms and
+// 0.17 + 0.56 + 0.25 -> 0.18 + 0.19 + 0.24 + 0.02 ms. The columns run at 4 TB/s; the rows are
+// bound by the latency of the loop over l (LDS reads, exchange, two DFTs) at two waves per
+// SIMD: their vector instructions alone take about half the time.
+#pragma once
+#include <cstdint>
+
+#include "context.hpp"
+#include "cplx.hpp"
+#include "fft_stages.hpp"
+
+namespace xatu_dev {
+
+constexpr int kRowWaves = 4;   // waves per workgroup of the row kernels
+constexpr int kColGroup = 32;  // adjacent columns per workgroup of the column kernel
+
+// Waves per SIMD of the row kernels (three made the FP32 ones spill: 1.72 -> 1.84 ms).
+constexpr int kRowOccupancy = 2;
+
+// Arguments of the row kernels. A group of B lanes owns one (fixed orbital f, vector v) of one
+// mesh row and loops over the other orbital l; its row of G starts at
+// (o1 batch + f sf + l sl + v) W.
+struct RowsArgs {
+    int n;
+    int W, w0;           // window of the first-axis frequencies
+    int nk, nvec;
+    int nfix, nloop;     // fixed and looped orbitals
+    int lchunk, stage;   // looped orbitals per workgroup (grid z) and per LDS stage
+    int conj;            // rows_out: conjugate the coefficients
+    int64_t batch, sf, sl;
+};
+
+// LDS: twiddles, staged coefficients [l][channel][o0], then a buffer per wave for the exchange
+// between the two steps (8-byte words; FP64 exchanges real and imaginary parts in turn).
+template <typename R, int A, int B, int NCH>
+constexpr size_t rows_lds_bytes(int stage) {
+    constexpr int n = A * B;
+    return sizeof(cx_t<R>) * (static_cast<size_t>(n) + static_cast<size_t>(stage) * NCH * n) +
+           8 * static_cast<size_t>(kRowWaves) * (64 / B) * B * (A | 1);
+}
+
+// Orders the LDS accesses of one wave (the groups of a row never cross a wave).
+__device__ inline void rows_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Exchange of a group through its LDS buffer: lane `wl` (if wr) writes v[i] to slot(i), lane
+// `rl` (if rd) reads x[i] from its slots.
+template <typename R, int NW, int NR, typename WS, typename RS>
+__device__ inline void rows_exchange(void* buf, bool wr, const cx_t<R> (&v)[NW], WS&& ws, bool rd, cx_t<R> (&x)[NR],
+                                     RS&& rs) {
+    if constexpr (sizeof(R) == 8) {
+        double* e = static_cast<double*>(buf);
+        if (wr) {
+#pragma unroll
+            for (int i = 0; i < NW; ++i) e[ws(i)] = v[i].x;
+        }
+        rows_wave_sync();
+        if (rd) {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) x[i].x = e[rs(i)];
+        }
+        rows_wave_sync();
+        if (wr) {
+#pragma unroll
+            for (int i = 0; i < NW; ++i) e[ws(i)] = v[i].y;
+        }
+        rows_wave_sync();
+        if (rd) {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) x[i].y = e[rs(i)];
+        }
+        rows_wave_sync();
+    } else {
+        float2* e = static_cast<float2*>(buf);
+        if (wr) {
+#pragma unroll
+            for (int i = 0; i < NW; ++i) e[ws(i)] = v[i];
+        }
+        rows_wave_sync();
+        if (rd) {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) x[i] = e[rs(i)];
+        }
+        rows_wave_sync();
+    }
+}
+
+// Coefficients Coef[(c nloop + l) nk + k] of the looped orbitals l0 .. l0 + count - 1 on mesh row
+// o1 to sc[(l NCH + c) n + o0] (zero where the mesh point has no k-point).
+template <typename R, int NCH>
+__device__ inline void stage_row_coefficients(cx_t<R>* sc, const cx_t<R>* __restrict__ Coef, const int* __restrict__ kmap,
+                                              const RowsArgs& a, int o1, int l0, int count) {
+    const int total = count * NCH * a.n;
+    for (int e = threadIdx.x; e < total; e += 64 * kRowWaves) {
+        const int o0 = e % a.n, lc = e / a.n;
+        const int c = lc % NCH, l = l0 + lc / NCH;
+        const int k = kmap[o0 + a.n * o1];
+        sc[e] = k >= 0 ? Coef[(static_cast<size_t>(c) * a.nloop + l) * a.nk + k] : mk(R(0), R(0));
+    }
+}
+
+// Offsets within a mesh row of G of a lane's frequencies s + A k2, from `at` on; -1 outside the
+// window or for an idle lane.
+template <int A, int B>
+__device__ inline void row_offsets(const RowsArgs& a, int s, int at, bool on, int (&off)[B]) {
+#pragma unroll
+    for (int k2 = 0; k2 < B; ++k2) {
+        int j = s + A * k2 - a.w0;
+        if (j < 0) j += A * B;
+        off[k2] = (on && j < a.W) ? at + j : -1;
+    }
+}
+
+// Twiddles e^{-2 pi i k / n} from the lattice sums' table of e^{i pi p / n}.
+template <typename R>
+__device__ inline void load_twiddles(cx_t<R>* tw, const double2* __restrict__ root, int n, int nthreads) {
+    for (int k = threadIdx.x; k < n; k += nthreads) {
+        const double2 r = root[2 * k];
+        tw[k] = mk(static_cast<R>(r.x), static_cast<R>(-r.y));
+    }
+}
+
+// Forward rows. U[((v NCH + c) nfix + f) nk + k]. grid (row groups, n, chunks of l), block 256.
+template <typename R, int A, int B, int NCH>
+__global__ __launch_bounds__(64 * kRowWaves, kRowOccupancy) void conv_rows_in_kernel(RowsArgs a, const int* __restrict__ kmap,
+                                                                      const double2* __restrict__ root,
+                                                                      const cx_t<R>* __restrict__ Coef,
+                                                                      const cx_t<R>* __restrict__ U,
+                                                                      cx_t<R>* __restrict__ G) {
+    using C = cx_t<R>;
+    constexpr int n = A * B, GW = 64 / B, AP = A | 1;
+    extern __shared__ unsigned char rows_raw[];
+    C* tw = reinterpret_cast<C*>(rows_raw);
+    C* sc = tw + n;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int gi = lane / B, s = lane - gi * B;
+    const int o1 = blockIdx.y;
+    const int task = (blockIdx.x * kRowWaves + wave) * GW + gi;
+    const bool live = gi < GW && task < a.nfix * a.nvec;
+    const int f = live ? task / a.nvec : 0, v = live ? task - f * a.nvec : 0;
+    unsigned char* xb = rows_raw + sizeof(C) * (n + static_cast<size_t>(a.stage) * NCH * n) +
+                        8 * static_cast<size_t>(wave * GW + (gi < GW ? gi : 0)) * B * AP;
+    load_twiddles<R>(tw, root, n, 64 * kRowWaves);
+    C u[A][NCH];
+#pragma unroll
+    for (int j = 0; j < A; ++j) {
+        const int k = live ? kmap[B * j + s + n * o1] : -1;
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+            u[j][c] = k >= 0 ? U[((static_cast<size_t>(v) * NCH + c) * a.nfix + f) * a.nk + k] : mk(R(0), R(0));
+    }
+    const int l0 = blockIdx.z * a.lchunk, l1 = min(a.nloop, l0 + a.lchunk);
+    // uniform base of the mesh row, 32-bit offsets of the lane's window entries (-1: outside)
+    C* grow = G + static_cast<int64_t>(o1) * a.batch * a.W;
+    int off[B];
+    row_offsets<A, B>(a, s, static_cast<int>(f * a.sf + v) * a.W, live && s < A, off);
+    for (int ls = l0; ls < l1; ls += a.stage) {
+        const int count = min(a.stage, l1 - ls);
+        __syncthreads();
+        stage_row_coefficients<R, NCH>(sc, Coef, kmap, a, o1, ls, count);
+        __syncthreads();
+        for (int l = 0; l < count; ++l) {
+            C z[A];
+#pragma unroll
+            for (int j = 0; j < A; ++j) {
+                z[j] = mk(R(0), R(0));
+#pragma unroll
+                for (int c = 0; c < NCH; ++c) cfma(z[j], sc[(l * NCH + c) * n + B * j + s], u[j][c]);
+            }
+            dft_len<R, A, -1>(z);
+#pragma unroll
+            for (int k1 = 1; k1 < A; ++k1) z[k1] = cmul(z[k1], tw[s * k1]);
+            C x[B];
+            rows_exchange<R, A, B>(
+                xb, gi < GW, z, [&](int i) { return s * AP + i; }, gi < GW && s < A, x, [&](int i) { return i * AP + s; });
+            if (live && s < A) {
+                dft_len<R, B, -1>(x);
+                C* out = grow + static_cast<int64_t>(ls + l) * a.sl * a.W;
+#pragma unroll
+                for (int k2 = 0; k2 < B; ++k2)
+                    if (off[k2] >= 0) out[static_cast<unsigned>(off[k2])] = x[k2];
+            }
+        }
+    }
+}
+
+// Inverse rows and contraction: T[(((part nvec + v) NCH + c) nfix + f) nk + k] = sum over the l of
+// this chunk (part) of Coef_l (conjugated if a.conj) times the row. grid as above, block 256.
+template <typename R, int A, int B, int NCH>
+__global__ __launch_bounds__(64 * kRowWaves, kRowOccupancy) void conv_rows_out_kernel(RowsArgs a, const int* __restrict__ kmap,
+                                                                       const double2* __restrict__ root,
+                                                                       const cx_t<R>* __restrict__ Coef,
+                                                                       const cx_t<R>* __restrict__ G,
+                                                                       cx_t<R>* __restrict__ T) {
+    using C = cx_t<R>;
+    constexpr int n = A * B, GW = 64 / B, AP = A | 1;
+    extern __shared__ unsigned char rows_raw[];
+    C* tw = reinterpret_cast<C*>(rows_raw);
+    C* sc = tw + n;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int gi = lane / B, s = lane - gi * B;
+    const int o1 = blockIdx.y;
+    const int task = (blockIdx.x * kRowWaves + wave) * GW + gi;
+    const bool live = gi < GW && task < a.nfix * a.nvec;
+    const int f = live ? task / a.nvec : 0, v = live ? task - f * a.nvec : 0;
+    unsigned char* xb = rows_raw + sizeof(C) * (n + static_cast<size_t>(a.stage) * NCH * n) +
+                        8 * static_cast<size_t>(wave * GW + (gi < GW ? gi : 0)) * B * AP;
+    load_twiddles<R>(tw, root, n, 64 * kRowWaves);
+    C t[A][NCH];
+#pragma unroll
+    for (int j = 0; j < A; ++j)
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) t[j][c] = mk(R(0), R(0));
+    const int l0 = blockIdx.z * a.lchunk, l1 = min(a.nloop, l0 + a.lchunk);
+    const C* grow = G + static_cast<int64_t>(o1) * a.batch * a.W;
+    const R cs = a.conj ? R(-1) : R(1);
+    int off[B];
+    row_offsets<A, B>(a, s, static_cast<int>(f * a.sf + v) * a.W, live && s < A, off);
+    // the next row's window is loaded one row ahead where the registers allow it
+    constexpr bool kAhead = sizeof(R) * (A * NCH + 3 * B) <= 8 * 56;
+    C x[B];
+    auto load = [&](int l) {
+        const C* in = grow + static_cast<int64_t>(l) * a.sl * a.W;
+#pragma unroll
+        for (int k2 = 0; k2 < B; ++k2) x[k2] = off[k2] >= 0 ? in[static_cast<unsigned>(off[k2])] : mk(R(0), R(0));
+    };
+    if (kAhead && l0 < l1) load(l0);
+    for (int ls = l0; ls < l1; ls += a.stage) {
+        const int count = min(a.stage, l1 - ls);
+        __syncthreads();
+        stage_row_coefficients<R, NCH>(sc, Coef, kmap, a, o1, ls, count);
+        __syncthreads();
+        for (int l = 0; l < count; ++l) {
+            if (!kAhead) load(ls + l);
+            C y[B];
+#pragma unroll
+            for (int i = 0; i < B; ++i) y[i] = x[i];
+            if (kAhead && ls + l + 1 < l1) load(ls + l + 1);
+            dft_len<R, B, 1>(y);
+            if (s < A) {
+#pragma unroll
+                for (int i = 1; i < B; ++i) y[i] = cmul(y[i], cconj(tw[i * s]));
+            }
+            C w[A];
+            rows_exchange<R, B, A>(
+                xb, gi < GW && s < A, y, [&](int i) { return i * AP + s; }, gi < GW, w, [&](int i) { return s * AP + i; });
+            dft_len<R, A, 1>(w);
+#pragma unroll
+            for (int j = 0; j < A; ++j)
+#pragma unroll
+                for (int c = 0; c < NCH; ++c) {
+                    C q = sc[(l * NCH + c) * n + B * j + s];
+                    q.y *= cs;
+                    cfma(t[j][c], q, w[j]);
+                }
+        }
+    }
+    if (live) {
+        const size_t base = (static_cast<size_t>(blockIdx.z) * a.nvec + v) * NCH;
+#pragma unroll
+        for (int j = 0; j < A; ++j) {
+            const int k = kmap[B * j + s + n * o1];
+            if (k < 0) continue;
+#pragma unroll
+            for (int c = 0; c < NCH; ++c) T[((base + c) * a.nfix + f) * a.nk + k] = t[j][c];
+        }
+    }
+}
+
+// Columns u = b W + j of G (length n, stride count = batch W): transform along o1, times the real
+// spectrum P[(pa n + xi_1) W + j] of the atom pair of b, inverse; in place. SPECTRUM false:
+// forward transform only, frequency xi_1 left at row xi_1. Lane (s, column) holds rows B j2 + s,
+// then frequency k1 = s of the first step. grid ceil(count / 32), block 32 B, dynamic LDS
+// (n + 32 n) entries.
+template <typename R, int A, int B, bool SPECTRUM>
+__global__ __launch_bounds__(kColGroup* B) void conv_columns_kernel(LatticeDesc lat, int W, int64_t count, int nvec,
+                                                                    const double2* __restrict__ root,
+                                                                    const R* __restrict__ P, cx_t<R>* __restrict__ G) {
+    using C = cx_t<R>;
+    constexpr int n = A * B, T = kColGroup;
+    extern __shared__ unsigned char rows_raw[];
+    C* tw = reinterpret_cast<C*>(rows_raw);
+    C* ex = tw + n;
+    const int c = threadIdx.x % T, s = threadIdx.x / T;
+    const int64_t u = static_cast<int64_t>(blockIdx.x) * T + c;
+    const bool live = u < count;
+    C* g = G + (live ? u : count - 1);
+    load_twiddles<R>(tw, root, n, T * B);
+    {
+        C v[A];
+#pragma unroll
+        for (int j = 0; j < A; ++j) v[j] = g[static_cast<int64_t>(B * j + s) * count];
+        __syncthreads();  // the twiddles
+        dft_len<R, A, -1>(v);
+#pragma unroll
+        for (int k = 0; k < A; ++k) ex[(s * A + k) * T + c] = k ? cmul(v[k], tw[s * k]) : v[k];
+    }
+    __syncthreads();
+    C v[B];
+    if (s < A) {
+#pragma unroll
+        for (int i = 0; i < B; ++i) v[i] = ex[(i * A + s) * T + c];
+        dft_len<R, B, -1>(v);
+        if constexpr (SPECTRUM) {
+            const int64_t uu = live ? u : count - 1;
+            const int64_t b = uu / W;
+            const int j = static_cast<int>(uu - b * W);
+            const int ab = static_cast<int>(b / nvec);
+            const int al = ab / lat.norb, be = ab - al * lat.norb;
+            int pa = 0, pb = 0;
+            while (al >= lat.orb_begin[pa + 1]) ++pa;
+            while (be >= lat.orb_begin[pb + 1]) ++pb;
+            const R* p = P + static_cast<int64_t>(pa + lat.natoms * pb) * n * W + j;
+#pragma unroll
+            for (int k = 0; k < B; ++k) {
+                const R q = p[static_cast<int64_t>(s + A * k) * W];
+                v[k].x *= q;
+                v[k].y *= q;
+            }
+            dft_len<R, B, 1>(v);
+#pragma unroll
+            for (int i = 1; i < B; ++i) v[i] = cmul(v[i], cconj(tw[i * s]));
+        } else if (live) {
+#pragma unroll
+            for (int k = 0; k < B; ++k) g[static_cast<int64_t>(s + A * k) * count] = v[k];
+        }
+    }
+    if constexpr (SPECTRUM) {
+        // a lane writes the slots that it read itself
+        if (s < A) {
+#pragma unroll
+            for (int i = 0; i < B; ++i) ex[(i * A + s) * T + c] = v[i];
+        }
+        __syncthreads();
+        C w[A];
+#pragma unroll
+        for (int k = 0; k < A; ++k) w[k] = ex[(s * A + k) * T + c];
+        dft_len<R, A, 1>(w);
+        if (live) {
+#pragma unroll
+            for (int j = 0; j < A; ++j) g[static_cast<int64_t>(B * j + s) * count] = w[j];
+        }
+    }
+}
+
+// Launchers (one source file per precision and kernel, to build them in parallel). A side
+// without a factor pair or more than four channels throws.
+template <typename R>
+void launch_rows_in(RowsArgs a, int nch, const int* kmap, const double2* root, const cx_t<R>* Coef, const cx_t<R>* U,
+                    cx_t<R>* G, hipStream_t s);
+// chunks: chunks of the looped orbitals, each with its own part of T (see rows_out_chunks).
+template <typename R>
+void launch_rows_out(RowsArgs a, int nch, int chunks, const int* kmap, const double2* root, const cx_t<R>* Coef,
+                     const cx_t<R>* G, cx_t<R>* T, hipStream_t s);
+template <typename R>
+void launch_columns(const LatticeDesc& lat, int W, int64_t count, int nvec, const double2* root, const R* P,
+                    cx_t<R>* G, bool spectrum, hipStream_t s);
+
+// Chunks of the looped orbitals for about `aim` workgroups.
+inline int rows_chunks(const RowsArgs& a, int aim, int most) {
+    int A = 0, B = 0;
+    fft_factors(a.n, A, B);
+    const int per = kRowWaves * (64 / B);
+    const int64_t wgs = static_cast<int64_t>((a.nfix * a.nvec + per - 1) / per) * a.n;
+    const int c = static_cast<int>((aim + wgs - 1) / wgs);
+    const int chunks = c < 1 ? 1 : (c > most ? most : c);
+    const int len = (a.nloop + chunks - 1) / chunks;
+    return (a.nloop + len - 1) / len;
+}
+// Parts of T: one per chunk, so few.
+inline int rows_out_chunks(const RowsArgs& a) { return rows_chunks(a, 512, a.nloop < 6 ? a.nloop : 6); }
+
+// Stages of the looped orbitals that keep the LDS near 40 KB (four workgroups per CU).
+template <typename R, int A, int B, int NCH>
+int rows_stage(int lchunk) {
+    const size_t fixed = rows_lds_bytes<R, A, B, NCH>(0), per = sizeof(cx_t<R>) * NCH * A * B;
+    const size_t room = fixed < 40 * 1024 ? 40 * 1024 - fixed : 0;
+    const int fit = static_cast<int>(room / per);
+    const int most = fit < 1 ? 1 : (fit < lchunk ? fit : lchunk);
+    const int stages = (lchunk + most - 1) / most;
+    return (lchunk + stages - 1) / stages;
+}
+
+}  // namespace xatu_dev

@@ -1,0 +1,5 @@
+// conv_rows_out.inc in FP64.
+#include "conv_rows.hpp"
+
+#define XATU_REAL double
+#include "conv_rows_out.inc"

@@ -25,8 +25,12 @@
 // partial sums from a blocked scan in a fixed order. The diagonal energies enter as
 // e_i x_i, so H x = e x - D x + X_tri x exactly as the assembled matrix.
 //
-// FFTs: rocFFT (batched, in place, interleaved complex); plans are cached per
-// precision and batch size. The exchange part runs in FP64 for both precisions.
+// FFTs: on 2-D meshes with sides A B (fft_stages.hpp) the row and column kernels of
+// conv_rows.hpp, which never store z or w on the mesh; otherwise rocFFT (batched, in place,
+// interleaved complex; plans cached per precision and batch size). The exchange part runs in
+// FP64 for both precisions.
+#include <algorithm>
+#include <cstdlib>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -37,6 +41,7 @@
 #include <rocfft/rocfft.h>
 
 #include "context.hpp"
+#include "conv_rows.hpp"
 #include "cplx.hpp"
 #include "mfma.hpp"
 
@@ -98,6 +103,33 @@ template <typename R>
 __global__ void scale_spectrum_kernel(const double2* __restrict__ in, int64_t n, double scale, cx_t<R>* __restrict__ out) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n) out[i] = mk(static_cast<R>(in[i].x * scale), static_cast<R>(in[i].y * scale));
+}
+
+// Kernel spectrum of the atom pair (a, b) on the window of the first axis, real:
+// P[((a + NA b) n + xi_1) W + j] = sum of V_ab(R) / T over the cells R = -xi (a < b) or R = xi
+// (a >= b) modulo the mesh, xi_0 = (w0 + j) mod n. head[xi_0 + n xi_1] is the first cell of a
+// residue, next[R] the following one (-1: none).
+template <typename R>
+__global__ void window_spectrum_kernel(LatticeDesc lat, int W, int w0, const int* __restrict__ head,
+                                       const int* __restrict__ next, int nR, const double* __restrict__ vtab,
+                                       double inv_total, R* __restrict__ P) {
+    const int n = lat.mesh_n;
+    const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (idx >= static_cast<int64_t>(lat.natoms) * lat.natoms * n * W) return;
+    const int j = static_cast<int>(idx % W);
+    const int x1 = static_cast<int>((idx / W) % n);
+    const int ab = static_cast<int>(idx / (static_cast<int64_t>(W) * n));
+    const int a = ab % lat.natoms, b = ab / lat.natoms;
+    int m0 = (w0 + j) % n, m1 = x1;
+    if (a < b) {
+        m0 = m0 ? n - m0 : 0;
+        m1 = m1 ? n - m1 : 0;
+    }
+    const int lo = min(a, b), hi = max(a, b);
+    const int p = lo * lat.natoms - lo * (lo - 1) / 2 + hi - lo;  // pairs (lo, hi >= lo), row by row
+    double sum = 0.0;
+    for (int r = head[m0 + n * m1]; r >= 0; r = next[r]) sum += vtab[static_cast<size_t>(p) * nR + r];
+    P[idx] = static_cast<R>(sum * inv_total);
 }
 
 // Band stacks transposed for coalesced access across k: Ct[(c norb + al) nk + k] =
@@ -229,399 +261,6 @@ __global__ void conv_multiply_kernel(LatticeDesc lat, int nvec, int64_t M, GLayo
     G[i] = cmul(G[i], P[static_cast<int64_t>(pa) * M + xi]);
 }
 
-// ---- fused transform along the second mesh axis (row-interleaved layout) ----
-// For 2-D meshes whose side n = A B factors into two of the lengths 1, 2, 3, 4, 5, 6, 8, 9,
-// 10, 12, 15, 16 (n <= kColMax), the transform along o1, the product with the spectrum and
-// the inverse transform along o1 run in one kernel: a workgroup holds 32 adjacent columns
-// u = b mesh_n + xi0 (each a length-n vector of stride batch mesh_n) and does a four-step
-// transform in registers with two LDS exchanges, so G is read and written once instead of
-// twice per direction with a transposition in between.
-constexpr int kColMax = 128;
-
-// In-register DFT of length RD; sg = -1 forward (e^{-2 pi i / RD}), +1 inverse.
-template <typename R, int RD>
-__device__ inline void small_dft(cx_t<R> (&v)[RD], R sg) {
-    using C = cx_t<R>;
-    auto isc = [&](C z, R f) { return mk(-sg * f * z.y, sg * f * z.x); };  // i sg f z
-    if constexpr (RD == 2) {
-        const C a = v[0], b = v[1];
-        v[0] = cadd(a, b);
-        v[1] = csub(a, b);
-    } else if constexpr (RD == 3) {
-        const R h3 = R(0.86602540378443864676);  // sin(2 pi / 3)
-        const C a = cadd(v[1], v[2]), d = csub(v[1], v[2]);
-        const C m = mk(v[0].x - R(0.5) * a.x, v[0].y - R(0.5) * a.y);
-        const C t = isc(d, h3);
-        v[0] = cadd(v[0], a);
-        v[1] = cadd(m, t);
-        v[2] = csub(m, t);
-    } else if constexpr (RD == 4) {
-        const C t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]), t2 = cadd(v[1], v[3]), t3 = isc(csub(v[1], v[3]), R(1));
-        v[0] = cadd(t0, t2);
-        v[1] = cadd(t1, t3);
-        v[2] = csub(t0, t2);
-        v[3] = csub(t1, t3);
-    } else {
-        static_assert(RD == 5, "radix");
-        // cos and sin of 2 pi / 5 and 4 pi / 5
-        const R c1 = R(0.30901699437494742410), s1 = R(0.95105651629515357212);
-        const R c2 = R(-0.80901699437494742410), s2 = R(0.58778525229247312917);
-        const C a1 = cadd(v[1], v[4]), d1 = csub(v[1], v[4]), a2 = cadd(v[2], v[3]), d2 = csub(v[2], v[3]);
-        const C p1 = mk(v[0].x + c1 * a1.x + c2 * a2.x, v[0].y + c1 * a1.y + c2 * a2.y);
-        const C p2 = mk(v[0].x + c2 * a1.x + c1 * a2.x, v[0].y + c2 * a1.y + c1 * a2.y);
-        const C q1 = isc(mk(s1 * d1.x + s2 * d2.x, s1 * d1.y + s2 * d2.y), R(1));
-        const C q2 = isc(mk(s2 * d1.x - s1 * d2.x, s2 * d1.y - s1 * d2.y), R(1));
-        v[0] = cadd(v[0], cadd(a1, a2));
-        v[1] = cadd(p1, q1);
-        v[4] = csub(p1, q1);
-        v[2] = cadd(p2, q2);
-        v[3] = csub(p2, q2);
-    }
-}
-
-// Twiddle e^{sg 2 pi i k / n} from the table of e^{-2 pi i k / n}.
-template <typename R>
-__device__ inline cx_t<R> twiddle(const cx_t<R>* tw, int k, R sg) {
-    const cx_t<R> w = tw[k];
-    return mk(w.x, sg < R(0) ? w.y : -w.y);
-}
-
-// DFT of length A B in registers as two Stockham stages (radix A, then radix B with the
-// twiddles e^{sg 2 pi i j r / (A B)} read from the n-point table).
-template <typename R, int A, int B>
-__device__ inline void composite_dft(cx_t<R> (&v)[A * B], R sg, const cx_t<R>* tw, int n) {
-    using C = cx_t<R>;
-    constexpr int RD = A * B;
-    C t[RD];
-#pragma unroll
-    for (int j = 0; j < B; ++j) {
-        C x[A];
-#pragma unroll
-        for (int r = 0; r < A; ++r) x[r] = v[j + r * B];
-        small_dft<R, A>(x, sg);
-#pragma unroll
-        for (int r = 0; r < A; ++r) t[j * A + r] = x[r];
-    }
-    const int unit = n / RD;
-#pragma unroll
-    for (int j = 0; j < A; ++j) {
-        C x[B];
-#pragma unroll
-        for (int r = 0; r < B; ++r) x[r] = (j * r) ? cmul(t[j + r * A], twiddle(tw, j * r * unit, sg)) : t[j + r * A];
-        small_dft<R, B>(x, sg);
-#pragma unroll
-        for (int r = 0; r < B; ++r) v[j + r * A] = x[r];
-    }
-}
-
-// DFT of one of the lengths 1, 2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16.
-template <typename R, int RD>
-__device__ inline void dft_len(cx_t<R> (&a)[RD], R sg, const cx_t<R>* tw, int n) {
-    if constexpr (RD == 1) {
-    } else if constexpr (RD <= 5) {
-        small_dft<R, RD>(a, sg);
-    } else if constexpr (RD == 6) {
-        composite_dft<R, 3, 2>(a, sg, tw, n);
-    } else if constexpr (RD == 8) {
-        composite_dft<R, 4, 2>(a, sg, tw, n);
-    } else if constexpr (RD == 9) {
-        composite_dft<R, 3, 3>(a, sg, tw, n);
-    } else if constexpr (RD == 10) {
-        composite_dft<R, 5, 2>(a, sg, tw, n);
-    } else if constexpr (RD == 12) {
-        composite_dft<R, 3, 4>(a, sg, tw, n);
-    } else if constexpr (RD == 15) {
-        composite_dft<R, 5, 3>(a, sg, tw, n);
-    } else {
-        static_assert(RD == 16, "length");
-        composite_dft<R, 4, 4>(a, sg, tw, n);
-    }
-}
-
-constexpr int kFourStepCols = 32; // columns per workgroup (512 threads: 16 per column)
-
-// Stage 1 (thread s < B): rows B j2 + s, A-point DFT, twiddle, Y[s][k1] to LDS.
-template <typename R, int A, int T>
-__device__ inline void four_step_in(const cx_t<R>* gcol, bool live, int64_t count, int B, int s, int c, int n,
-                                    const cx_t<R>* tw, cx_t<R>* ex) {
-    cx_t<R> v[A];
-#pragma unroll
-    for (int j2 = 0; j2 < A; ++j2) v[j2] = live ? gcol[static_cast<int64_t>(B * j2 + s) * count] : mk(R(0), R(0));
-    dft_len<R, A>(v, R(-1), tw, n);
-#pragma unroll
-    for (int k1 = 0; k1 < A; ++k1) ex[(s * A + k1) * T + c] = k1 ? cmul(v[k1], tw[s * k1]) : v[k1];
-}
-
-// Stage 2 (threads with act, s < A): Y[j1][s], B-point DFT (xi1 = s + A k2), times the
-// spectrum column pc, inverse B-point DFT, twiddle back, Z[s][j1] to LDS. Every thread of
-// the workgroup calls it (B is uniform) and passes its barrier between the reads and the
-// writes of the shared buffer.
-template <typename R, int B, int T>
-__device__ inline void four_step_mid(bool act, const cx_t<R>* pc, int A, int s, int c, int n, const cx_t<R>* tw,
-                                     cx_t<R>* ex) {
-    cx_t<R> v[B];
-    if (act) {
-#pragma unroll
-        for (int j1 = 0; j1 < B; ++j1) v[j1] = ex[(j1 * A + s) * T + c];
-    }
-    __syncthreads();
-    if (!act) return;
-    dft_len<R, B>(v, R(-1), tw, n);
-    if (pc) {
-#pragma unroll
-        for (int k2 = 0; k2 < B; ++k2) v[k2] = cmul(v[k2], pc[static_cast<int64_t>(n) * (s + A * k2)]);
-    }
-    dft_len<R, B>(v, R(1), tw, n);
-#pragma unroll
-    for (int j1 = 0; j1 < B; ++j1) {
-        const cx_t<R> w = tw[j1 * s];
-        ex[(s * B + j1) * T + c] = (j1 * s) ? cmul(v[j1], mk(w.x, -w.y)) : v[j1];
-    }
-}
-
-// Stage 3 (thread s < B): Z[k1][s], inverse A-point DFT, rows B j2 + s to G.
-template <typename R, int A, int T>
-__device__ inline void four_step_out(cx_t<R>* gcol, bool live, int64_t count, int B, int s, int c, int n,
-                                     const cx_t<R>* tw, const cx_t<R>* ex) {
-    cx_t<R> v[A];
-#pragma unroll
-    for (int k1 = 0; k1 < A; ++k1) v[k1] = ex[(k1 * B + s) * T + c];
-    dft_len<R, A>(v, R(1), tw, n);
-    if (live) {
-#pragma unroll
-        for (int j2 = 0; j2 < A; ++j2) gcol[static_cast<int64_t>(B * j2 + s) * count] = v[j2];
-    }
-}
-
-#define XATU_FOUR_STEP_LENGTHS(X) X(1) X(2) X(3) X(4) X(5) X(6) X(8) X(9) X(10) X(12) X(15) X(16)
-
-// The same fused column transform for n = A B (A >= B, both lengths of dft_len) as a
-// four-step transform in registers: thread (s, c) of column c loads rows B j2 + s (j2 < A)
-// and does the A-point DFTs, twiddles by e^{-2 pi i s k1 / n} and stores Y[s][k1] to LDS;
-// thread (s, c) then takes Y[j1][s] (j1 < B), does the B-point DFT (outputs xi1 = s + A k2),
-// multiplies by the spectrum, inverts the B-point DFT, twiddles back and stores Z[s][j1];
-// thread (s, c) finally takes Z[k1][s] (k1 < A), inverts the A-point DFT and stores rows
-// B j2 + s. Two LDS exchanges instead of a pass per radix. grid ceil(count / 32), block 512.
-template <typename R>
-__global__ __launch_bounds__(512) void conv_columns4_kernel(LatticeDesc lat, int n, int A, int B, int64_t count,
-                                                            int nvec, int64_t M, const cx_t<R>* __restrict__ P,
-                                                            cx_t<R>* __restrict__ G) {
-    using C = cx_t<R>;
-    constexpr int T = kFourStepCols;
-    __shared__ C ex[kColMax * T];
-    __shared__ C tw[kColMax];
-    const int c = threadIdx.x % T, s = threadIdx.x / T;
-    const int64_t u = static_cast<int64_t>(blockIdx.x) * T + c;
-    const bool live = u < count;
-    for (int k = threadIdx.x; k < n; k += blockDim.x) {
-        double sn, cs;
-        sincospi(2.0 * k / n, &sn, &cs);
-        tw[k] = mk(static_cast<R>(cs), static_cast<R>(-sn));  // e^{-2 pi i k / n}
-    }
-    __syncthreads();
-    C* gcol = G + u;
-    if (s < B) {
-        switch (A) {
-#define XATU_IN(L) \
-    case L: four_step_in<R, L, T>(gcol, live, count, B, s, c, n, tw, ex); break;
-            XATU_FOUR_STEP_LENGTHS(XATU_IN)
-#undef XATU_IN
-        }
-    }
-    __syncthreads();
-    const C* pc = nullptr;
-    if (live) {
-        const int64_t b = u / n;
-        const int xi0 = static_cast<int>(u - b * n);
-        const int ab = static_cast<int>(b / nvec);
-        const int al = ab / lat.norb, be = ab % lat.norb;
-        pc = P + static_cast<int64_t>(atom_of(lat, al) + lat.natoms * atom_of(lat, be)) * M + xi0;
-    }
-    // B is the same for the whole workgroup: every thread takes the same case and passes the
-    // barrier inside four_step_mid once
-    switch (B) {
-#define XATU_MID(L) \
-    case L: four_step_mid<R, L, T>(s < A, pc, A, s, c, n, tw, ex); break;
-        XATU_FOUR_STEP_LENGTHS(XATU_MID)
-#undef XATU_MID
-    }
-    __syncthreads();
-    if (s < B) {
-        switch (A) {
-#define XATU_OUT(L) \
-    case L: four_step_out<R, L, T>(gcol, live, count, B, s, c, n, tw, ex); break;
-            XATU_FOUR_STEP_LENGTHS(XATU_OUT)
-#undef XATU_OUT
-        }
-    }
-}
-
-// Whole-plane form of the same transform, for 2-D meshes whose n x n plane (FP64 up to n = 100,
-// FP32 up to 128) fits in LDS: one workgroup per batch entry b loads its plane once,
-// transforms the rows, transforms the columns with the spectrum product between the forward
-// and inverse column transforms, inverts the rows and stores the plane, so G is read and
-// written once per product instead of once per pass (row transform, column kernel, inverse
-// row transform). Every stage is a four-step stage done in place: a task reads the positions
-// B j + s (or B t + j) of its row or column and writes the same positions, so only the
-// barriers between stages are needed. The forward A-point stage stores its output k1 at
-// B k1 + s; after the forward B-point stage, position B t + k2 of a row holds the frequency
-// t + A k2 (the columns are transformed in that order and the spectrum read accordingly).
-// Rows are ldp = n + 1 entries apart in LDS so that tasks on consecutive rows use different
-// banks. grid batch, block plane_threads<R>() (FP64: 512, whose 256 registers per thread hold
-// the 16-point stages without spilling; one FP64 plane takes most of the LDS anyway),
-// dynamic LDS (kColMax + n (n + 1)) entries.
-template <typename R>
-constexpr int plane_threads() { return sizeof(R) == 8 ? 512 : 1024; }
-
-// A-point stage, forward (from positions B j2 + s to B k1 + s, times e^{-2 pi i s k1 / n}) or
-// inverse (from B k1 + s to B j2 + s, no twiddle); in and out may be the same.
-template <typename R, int A>
-__device__ inline void plane_stage_a(const cx_t<R>* in, int istr, cx_t<R>* out, int ostr, int B, int s, int n,
-                                     const cx_t<R>* tw, bool forward) {
-    cx_t<R> v[A];
-#pragma unroll
-    for (int j = 0; j < A; ++j) v[j] = in[static_cast<int64_t>(B * j + s) * istr];
-    dft_len<R, A>(v, forward ? R(-1) : R(1), tw, n);
-#pragma unroll
-    for (int k = 0; k < A; ++k)
-        out[static_cast<int64_t>(B * k + s) * ostr] = (forward && k) ? cmul(v[k], tw[s * k]) : v[k];
-}
-
-// B-point stage in place at positions B t + j (j < B): forward (output k2 at B t + k2), or
-// inverse then times e^{+2 pi i j t / n}; with spec, forward, times spec[(t + A k2) n],
-// inverse and twiddle back (the column stage between the forward and inverse transforms).
-template <typename R, int B>
-__device__ inline void plane_stage_b(cx_t<R>* base, int str, int t, int A, int n, const cx_t<R>* tw, int mode,
-                                     const cx_t<R>* spec) {
-    using C = cx_t<R>;
-    C v[B];
-#pragma unroll
-    for (int j = 0; j < B; ++j) v[j] = base[(B * t + j) * str];
-    if (mode >= 0) dft_len<R, B>(v, R(-1), tw, n);  // 0: forward; 1: forward, spectrum, inverse
-    if (mode == 1) {
-#pragma unroll
-        for (int k = 0; k < B; ++k) v[k] = cmul(v[k], spec[static_cast<int64_t>(n) * (t + A * k)]);
-    }
-    if (mode != 0) dft_len<R, B>(v, R(1), tw, n);  // -1: inverse only
-#pragma unroll
-    for (int j = 0; j < B; ++j) {
-        const C w = tw[j * t];
-        base[(B * t + j) * str] = (mode != 0 && j * t) ? cmul(v[j], mk(w.x, -w.y)) : v[j];
-    }
-}
-
-template <typename R, int NT>
-__global__ __launch_bounds__(NT) void conv_plane_kernel(LatticeDesc lat, int n, int A, int B, int batch,
-                                                                   int nvec, int64_t M, const cx_t<R>* __restrict__ P,
-                                                                   cx_t<R>* __restrict__ G) {
-    using C = cx_t<R>;
-    extern __shared__ unsigned char plane_raw[];
-    C* tw = reinterpret_cast<C*>(plane_raw);
-    C* pl = tw + kColMax;
-    const int ldp = n + 1;
-    const int tid = threadIdx.x;
-    const int b = blockIdx.x;
-    for (int k = tid; k < n; k += NT) {
-        double sn, cs;
-        sincospi(2.0 * k / n, &sn, &cs);
-        tw[k] = mk(static_cast<R>(cs), static_cast<R>(-sn));  // e^{-2 pi i k / n}
-    }
-    const int ab = b / nvec;
-    const int al = ab / lat.norb, be = ab % lat.norb;
-    const C* pp = P + static_cast<int64_t>(atom_of(lat, al) + lat.natoms * atom_of(lat, be)) * M;
-    C* g = G + static_cast<int64_t>(b) * n;  // row o1 of the plane at g + o1 gs
-    const int64_t gs = static_cast<int64_t>(batch) * n;
-    __syncthreads();
-    // A and B are the same for the whole workgroup: every thread takes the same case
-#define XATU_SWITCH_A switch (A) { XATU_FOUR_STEP_LENGTHS(XATU_CASE_A) }
-#define XATU_SWITCH_B switch (B) { XATU_FOUR_STEP_LENGTHS(XATU_CASE_B) }
-    // rows, forward A-point stage from G (s fastest: a row's 16-byte entries together)
-    for (int task = tid; task < n * B; task += NT) {
-        const int s = task % B, o1 = task / B;
-#define XATU_CASE_A(L) \
-    case L: plane_stage_a<R, L>(g + o1 * gs, 1, pl + o1 * ldp, 1, B, s, n, tw, true); break;
-        XATU_SWITCH_A
-#undef XATU_CASE_A
-    }
-    __syncthreads();
-    // rows, forward B-point stage (o1 fastest: rows ldp entries apart)
-    for (int task = tid; task < n * A; task += NT) {
-        const int o1 = task % n, t = task / n;
-#define XATU_CASE_B(L) \
-    case L: plane_stage_b<R, L>(pl + o1 * ldp, 1, t, A, n, tw, 0, nullptr); break;
-        XATU_SWITCH_B
-#undef XATU_CASE_B
-    }
-    __syncthreads();
-    // columns (position p of every row), forward A-point stage
-    for (int task = tid; task < n * B; task += NT) {
-        const int p = task % n, s = task / n;
-#define XATU_CASE_A(L) \
-    case L: plane_stage_a<R, L>(pl + p, ldp, pl + p, ldp, B, s, n, tw, true); break;
-        XATU_SWITCH_A
-#undef XATU_CASE_A
-    }
-    __syncthreads();
-    // columns: forward B-point stage, spectrum of row frequency p / B + A (p % B), inverse
-    for (int task = tid; task < n * A; task += NT) {
-        const int p = task % n, t = task / n;
-        const C* spec = pp + (p / B + A * (p % B));
-#define XATU_CASE_B(L) \
-    case L: plane_stage_b<R, L>(pl + p, ldp, t, A, n, tw, 1, spec); break;
-        XATU_SWITCH_B
-#undef XATU_CASE_B
-    }
-    __syncthreads();
-    // columns, inverse A-point stage
-    for (int task = tid; task < n * B; task += NT) {
-        const int p = task % n, s = task / n;
-#define XATU_CASE_A(L) \
-    case L: plane_stage_a<R, L>(pl + p, ldp, pl + p, ldp, B, s, n, tw, false); break;
-        XATU_SWITCH_A
-#undef XATU_CASE_A
-    }
-    __syncthreads();
-    // rows, inverse B-point stage
-    for (int task = tid; task < n * A; task += NT) {
-        const int o1 = task % n, t = task / n;
-#define XATU_CASE_B(L) \
-    case L: plane_stage_b<R, L>(pl + o1 * ldp, 1, t, A, n, tw, -1, nullptr); break;
-        XATU_SWITCH_B
-#undef XATU_CASE_B
-    }
-    __syncthreads();
-    // rows, inverse A-point stage to G
-    for (int task = tid; task < n * B; task += NT) {
-        const int s = task % B, o1 = task / B;
-#define XATU_CASE_A(L) \
-    case L: plane_stage_a<R, L>(pl + o1 * ldp, 1, g + o1 * gs, 1, B, s, n, tw, false); break;
-        XATU_SWITCH_A
-#undef XATU_CASE_A
-    }
-#undef XATU_SWITCH_A
-#undef XATU_SWITCH_B
-}
-
-// LDS bytes of conv_plane_kernel for mesh side n.
-template <typename R>
-size_t conv_plane_lds(int n) {
-    return (static_cast<size_t>(kColMax) + static_cast<size_t>(n) * (n + 1)) * sizeof(cx_t<R>);
-}
-
-// Factors (A, B) of the four-step column transform for mesh side n <= kColMax, A >= B, both
-// lengths of dft_len, B as large as possible; A = 0 if none.
-void four_step_factors(int n, int& A, int& B) {
-    static const int len[] = {1, 2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16};
-    A = B = 0;
-    if (n < 1 || n > kColMax) return;  // the LDS tile and twiddle table hold kColMax rows
-    for (int b : len)
-        for (int a : len)
-            if (a >= b && a * b == n && b > B) {
-                A = a;
-                B = b;
-            }
-}
-
 // Y[k NCV + c NV + v, n] = e(kcv) x - sum_be V_k[be, v] sum_al conj(C_k[al, c]) w[(al norb + be) nvec + n][g(k)]
 // thread per k, blockIdx.y = group of vectors (the band coefficients are loaded once per group)
 template <typename R, int NC, int NV>
@@ -709,6 +348,52 @@ __global__ __launch_bounds__(256) void conv_y_kernel(int nk, int norb, int nvec,
                 }
         }
     }
+}
+
+// Y[k NCV + c NV + v, n] = e(kcv) x - sum_be V_k[be, v] t[n][c][be][k] with t the sum of the
+// parts that conv_rows_out_kernel left (T[((part nvec + n) NC + c) norb + be][k]); thread per k,
+// blockIdx.y = vector n
+template <typename R, int NC, int NV>
+__global__ __launch_bounds__(256) void conv_bands_y_kernel(int nk, int norb, int nvec, int parts,
+                                                           const cx_t<R>* __restrict__ Vt,
+                                                           const double* __restrict__ eval_k,
+                                                           const double* __restrict__ eval_kq, double scissor,
+                                                           const cx_t<R>* __restrict__ T,
+                                                           const double2* __restrict__ X, int64_t N,
+                                                           double2* __restrict__ Y) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    const int n = blockIdx.y;
+    if (k >= nk) return;
+    constexpr int nb = NV + NC, ncv = NC * NV;
+    cx_t<R> acc[NC][NV];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) acc[c][v] = mk(R(0), R(0));
+    const size_t part_stride = static_cast<size_t>(nvec) * NC * norb * nk;
+    const cx_t<R>* tn = T + static_cast<size_t>(n) * NC * norb * nk + k;
+    for (int be = 0; be < norb; ++be) {
+        cx_t<R> vb[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) vb[v] = Vt[(static_cast<size_t>(v) * norb + be) * nk + k];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const cx_t<R>* tc = tn + (static_cast<size_t>(c) * norb + be) * nk;
+            cx_t<R> t = tc[0];
+            for (int q = 1; q < parts; ++q) t = cadd(t, tc[q * part_stride]);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) cfma(acc[c][v], vb[v], t);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int64_t row = static_cast<int64_t>(k) * ncv + c * NV + v;
+            const double e = (scissor + eval_kq[static_cast<size_t>(k) * nb + NV + c]) - eval_k[static_cast<size_t>(k) * nb + v];
+            const double2 x = X[row + n * N];
+            Y[row + n * N] = mk(e * x.x - static_cast<double>(acc[c][v].x), e * x.y - static_cast<double>(acc[c][v].y));
+        }
 }
 
 // Launch the contraction kernels for the context's band counts (nc, nv in 1..4).
@@ -844,6 +529,38 @@ __global__ void power_sum_kernel(LatticeDesc lat, int ns, int64_t M, const doubl
     Pw[(static_cast<int64_t>(n) * lat.natoms * lat.natoms + ab) * M + xi] = mk(sum, 0.0);
 }
 
+// shat[(s npairs + p) nR + R] from the forward transforms G[(xi_1 batch + (al norb + be) ns + s) W + j]
+// (see conv_cell_density); grid (ceil(nR / 256), npairs, ns)
+__global__ void cell_power_kernel(LatticeDesc lat, int W, int w0, const int* __restrict__ cells, int nR, int npairs,
+                                  int ns, const double2* __restrict__ G, double* __restrict__ shat) {
+    const int R = blockIdx.x * blockDim.x + threadIdx.x;
+    const int p = blockIdx.y, st = blockIdx.z;
+    if (R >= nR) return;
+    int a = 0, rem = p;
+    while (rem >= lat.natoms - a) {
+        rem -= lat.natoms - a;
+        ++a;
+    }
+    const int b = a + rem;
+    const int n = lat.mesh_n, norb = lat.norb;
+    const int64_t batch = static_cast<int64_t>(norb) * norb * ns;
+    auto power = [&](int ra, int rb, int sign) {  // sum over al in ra, be in rb at xi = sign R
+        int x[2];
+        for (int j = 0; j < 2; ++j) x[j] = (((sign * cells[3 * R + j]) % n) + n) % n;
+        int j = x[0] - w0;
+        if (j < 0) j += n;
+        const double2* g = G + (x[1] * batch + st) * W + j;
+        double sum = 0.0;
+        for (int al = lat.orb_begin[ra]; al < lat.orb_begin[ra + 1]; ++al)
+            for (int be = lat.orb_begin[rb]; be < lat.orb_begin[rb + 1]; ++be) {
+                const double2 z = g[static_cast<int64_t>(al * norb + be) * ns * W];
+                sum += z.x * z.x + z.y * z.y;
+            }
+        return sum;
+    };
+    shat[(static_cast<size_t>(st) * npairs + p) * nR + R] = a < b ? power(a, b, -1) + power(b, a, 1) : power(a, a, 1);
+}
+
 // S[(n nmesh + q) NA^2 + ab] = W[(n NA^2 + ab) M + g(Delta(q))] / M with Delta_j = (q_j - m/2) mod m
 __global__ void scatter_pair_density_kernel(LatticeDesc lat, int ns, const double2* __restrict__ W,
                                             double2* __restrict__ S) {
@@ -884,7 +601,16 @@ struct ConvState {
     DevBuf<float2> G32, U32, Ct32, Vt32;
     DevBuf<double2> part, total;
     DevBuf<double2> Mt;  // interaction table on the mesh (set-up scratch, kept between set-ups)
-    size_t lds_limit = 0;  // LDS bytes a workgroup may use on this device (0: not queried yet)
+    // row and column transforms (2-D meshes with a supported side): window of the first axis, real
+    // spectra on it, cell lists of the spectrum, k-point of each mesh point (-1: none)
+    bool rows = false;
+    bool full = false;  // every mesh point has a k-point
+    int W = 0, w0 = 0;
+    DevBuf<double> Pw64;
+    DevBuf<float> Pw32;
+    DevBuf<int> d_head, d_next, d_kmap;
+    DevBuf<double2> T64;
+    DevBuf<float2> T32;
     // A transform over the whole mesh: one rocFFT plan per direction (entry-major layout),
     // or for the row-interleaved layout two batched 1-D plans per direction (along o0,
     // then along o1)
@@ -905,17 +631,6 @@ struct ConvState {
 };
 
 void destroy_conv_state(ConvState* s) { delete s; }
-
-// LDS a workgroup may use on the current device (queried once per state).
-size_t conv_lds_limit(ConvState& cs) {
-    if (cs.lds_limit == 0) {
-        int dev = 0, v = 0;
-        XATU_HIP(hipGetDevice(&dev));
-        XATU_HIP(hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-        cs.lds_limit = static_cast<size_t>(std::max(v, 1));
-    }
-    return cs.lds_limit;
-}
 
 namespace {
 
@@ -980,8 +695,16 @@ ConvState::Plan& get_plan(Context& c, ConvState& cs, int batch, bool interleaved
     return cs.plans.emplace(key, p).first->second;
 }
 
-// Kernel spectra P_ab = (1/M) backward FFT of the table on the mesh, and the grid
-// index of every k-point; rebuilt after each preparation of the operator.
+// Largest correlation buffer of one pass of the row and column transforms: a product takes its
+// vectors in chunks that keep the buffer within it (N = 129600, 32 FP32 vectors, 2.3 GB in one
+// pass: 16.0 ms a call; passes of 512 MB 16.6 ms, of 128 MB, which the last-level cache
+// holds, 19.7 ms: the kernels are not bound by that traffic).
+constexpr size_t kRowsBufferBytes = size_t(4) << 30;
+
+// Band stacks transposed, the mesh point of every k-point, and the kernel spectra: on 2-D
+// meshes with a supported side directly from the potential on the window of the transforms,
+// otherwise P_ab = (1/M) backward FFT of the table on the mesh; rebuilt after each preparation
+// of the operator.
 void ensure_conv(Context& c) {
     if (!c.conv) c.conv = std::unique_ptr<ConvState, void (*)(ConvState*)>(new ConvState, destroy_conv_state);
     ConvState& cs = *c.conv;
@@ -990,7 +713,10 @@ void ensure_conv(Context& c) {
     const int64_t M = c.lat.nmesh;
     cs.M = M;
     const int m = c.lat.mesh_n;
-    std::vector<int> gk(c.nk);
+    const int norb = c.lat.norb;
+    const int na2 = c.lat.natoms * c.lat.natoms;
+    std::vector<int> gk(c.nk), kmap(M, -1);
+    bool distinct = true;
     for (int k = 0; k < c.nk; ++k) {
         int64_t g = 0, mul = 1;
         for (int j = 0; j < c.lat.ndim; ++j) {
@@ -1000,10 +726,9 @@ void ensure_conv(Context& c) {
             mul *= m;
         }
         gk[k] = static_cast<int>(g);
+        distinct = distinct && kmap[g] < 0;
+        kmap[g] = k;
     }
-    cs.d_gk.alloc(c.nk);
-    XATU_HIP(hipMemcpyAsync(cs.d_gk.p, gk.data(), gk.size() * sizeof(int), hipMemcpyHostToDevice, c.stream));
-    const int norb = c.lat.norb;
     cs.Ct64.alloc(static_cast<size_t>(c.nc) * norb * c.nk);
     cs.Vt64.alloc(static_cast<size_t>(c.nv) * norb * c.nk);
     cs.Ct32.alloc(cs.Ct64.n);
@@ -1014,7 +739,47 @@ void ensure_conv(Context& c) {
     hipLaunchKernelGGL((transpose_stacks_kernel<float>), tg, dim3(256), 0, c.stream, c.nk, c.nv, c.nc, norb,
                        c.d_evec_k.p, c.d_evec_kq.p, cs.Ct32.p, cs.Vt32.p);
     XATU_HIP(hipGetLastError());
-    const int na2 = c.lat.natoms * c.lat.natoms;
+    int fa = 0, fb = 0;
+    fft_factors(m, fa, fb);
+    cs.full = distinct && static_cast<int64_t>(c.nk) == M;
+    // k-points that share a mesh point (offsets that differ by whole periods) stay on the general path
+    cs.rows = c.lat.ndim == 2 && fa > 0 && distinct;
+    if (cs.rows) {
+        int w = 0;
+        std::vector<int> head(M, -1), next(c.nR, -1);
+        for (int r = c.nR - 1; r >= 0; --r) {
+            int o[2];
+            for (int j = 0; j < 2; ++j) {
+                const int mj = c.h_cells[2 * static_cast<size_t>(r) + j];
+                w = std::max(w, j == 0 ? std::abs(mj) : 0);
+                o[j] = ((mj % m) + m) % m;
+            }
+            const int g = o[0] + m * o[1];
+            next[r] = head[g];
+            head[g] = r;
+        }
+        cs.W = std::min(m, 2 * w + 1);
+        cs.w0 = cs.W == m ? 0 : m - w;
+        cs.d_head.alloc(head.size());
+        cs.d_next.alloc(next.size());
+        cs.d_kmap.alloc(kmap.size());
+        XATU_HIP(hipMemcpyAsync(cs.d_head.p, head.data(), head.size() * sizeof(int), hipMemcpyHostToDevice, c.stream));
+        XATU_HIP(hipMemcpyAsync(cs.d_next.p, next.data(), next.size() * sizeof(int), hipMemcpyHostToDevice, c.stream));
+        XATU_HIP(hipMemcpyAsync(cs.d_kmap.p, kmap.data(), kmap.size() * sizeof(int), hipMemcpyHostToDevice, c.stream));
+        const size_t np = static_cast<size_t>(na2) * m * cs.W;
+        cs.Pw64.alloc(np);
+        cs.Pw32.alloc(np);
+        const double inv_total = 1.0 / static_cast<double>(c.inter.total_cells);
+        hipLaunchKernelGGL((window_spectrum_kernel<double>), dim3((np + 255) / 256), dim3(256), 0, c.stream, c.lat, cs.W,
+                           cs.w0, cs.d_head.p, cs.d_next.p, c.nR, c.d_vtab.p, inv_total, cs.Pw64.p);
+        hipLaunchKernelGGL((window_spectrum_kernel<float>), dim3((np + 255) / 256), dim3(256), 0, c.stream, c.lat, cs.W,
+                           cs.w0, cs.d_head.p, cs.d_next.p, c.nR, c.d_vtab.p, inv_total, cs.Pw32.p);
+        XATU_HIP(hipGetLastError());
+        cs.gen = c.prep_gen;
+        return;
+    }
+    cs.d_gk.alloc(c.nk);
+    XATU_HIP(hipMemcpyAsync(cs.d_gk.p, gk.data(), gk.size() * sizeof(int), hipMemcpyHostToDevice, c.stream));
     DevBuf<double2>& Mt = cs.Mt;
     Mt.alloc(static_cast<size_t>(na2) * M);
     hipLaunchKernelGGL(table_grid_kernel, dim3((Mt.n + 255) / 256), dim3(256), 0, c.stream, c.lat, c.d_ft.p, Mt.p);
@@ -1033,89 +798,192 @@ void ensure_conv(Context& c) {
     cs.gen = c.prep_gen;
 }
 
+// The precision's buffers of a ConvState.
 template <typename R>
-void conv_product(Context& c, const double2* X, double2* Y, int nvec, hipStream_t s, DevBuf<cx_t<R>>& G,
-                  DevBuf<cx_t<R>>& U, const cx_t<R>* P, const cx_t<R>* Ct, const cx_t<R>* Vt) {
-    ConvState& cs = *c.conv;
+struct ConvBuffers;
+template <>
+struct ConvBuffers<double> {
+    DevBuf<double2>&G, &U, &T;
+    const double2 *P, *Ct, *Vt;
+    const double* Pw;
+    explicit ConvBuffers(ConvState& s) : G(s.G64), U(s.U64), T(s.T64), P(s.P64.p), Ct(s.Ct64.p), Vt(s.Vt64.p), Pw(s.Pw64.p) {}
+};
+template <>
+struct ConvBuffers<float> {
+    DevBuf<float2>&G, &U, &T;
+    const float2 *P, *Ct, *Vt;
+    const float* Pw;
+    explicit ConvBuffers(ConvState& s) : G(s.G32), U(s.U32), T(s.T32), P(s.P32.p), Ct(s.Ct32.p), Vt(s.Vt32.p), Pw(s.Pw32.p) {}
+};
+
+// u of nv vectors (band contraction with the valence vectors) to b.U.
+template <typename R>
+void conv_bands_in(Context& c, ConvBuffers<R>& b, const double2* X, int nv, hipStream_t s) {
+    const int norb = c.lat.norb;
+    b.U.reserve(static_cast<size_t>(nv) * c.nc * norb * c.nk);
+    const unsigned kb = (c.nk + 255) / 256;
+    const int vg = (nv + conv_vec_group<R>() - 1) / conv_vec_group<R>();
+    with_bands<R>(c, [&](auto ncc, auto nvc) {
+        constexpr int NC = decltype(ncc)::value, NV = decltype(nvc)::value;
+        hipLaunchKernelGGL((conv_u_kernel<R, NC, NV>), dim3(kb, vg), dim3(256), 0, s, c.nk, norb, nv, b.Vt, X, c.N, b.U.p);
+    });
+    XATU_HIP(hipGetLastError());
+}
+
+// Arguments of the row kernels for nv vectors: fixed orbital be, looped orbital al.
+RowsArgs rows_args(const Context& c, const ConvState& cs, int nv) {
+    const int norb = c.lat.norb;
+    RowsArgs a{};
+    a.n = c.lat.mesh_n;
+    a.W = cs.W;
+    a.w0 = cs.w0;
+    a.nk = c.nk;
+    a.nvec = nv;
+    a.nfix = a.nloop = norb;
+    a.conj = 1;
+    a.batch = static_cast<int64_t>(norb) * norb * nv;
+    a.sl = static_cast<int64_t>(norb) * nv;
+    a.sf = nv;
+    return a;
+}
+
+// The transformed z of nv vectors (b.U) on the window: rows, then columns (with the spectrum and
+// back, or forward only) in b.G.
+template <typename R>
+void conv_rows_forward(Context& c, ConvState& cs, ConvBuffers<R>& b, int nv, bool spectrum, hipStream_t s) {
+    const RowsArgs a = rows_args(c, cs, nv);
+    const int64_t count = a.batch * cs.W;
+    b.G.reserve(static_cast<size_t>(count) * a.n);
+    launch_rows_in<R>(a, c.nc, cs.d_kmap.p, c.d_twiddle.p, b.Ct, b.U.p, b.G.p, s);
+    launch_columns<R>(c.lat, cs.W, count, nv, c.d_twiddle.p, b.Pw, b.G.p, spectrum, s);
+}
+
+// Direct term and energies of nv vectors by row and column transforms.
+template <typename R>
+void conv_rows_product(Context& c, ConvState& cs, ConvBuffers<R>& b, const double2* X, double2* Y, int nv, hipStream_t s) {
+    conv_bands_in<R>(c, b, X, nv, s);
+    conv_rows_forward<R>(c, cs, b, nv, true, s);
+    const RowsArgs a = rows_args(c, cs, nv);
+    const int parts = rows_out_chunks(a);
+    b.T.reserve(static_cast<size_t>(parts) * nv * c.nc * c.lat.norb * c.nk);
+    launch_rows_out<R>(a, c.nc, parts, cs.d_kmap.p, c.d_twiddle.p, b.Ct, b.G.p, b.T.p, s);
+    with_bands<R>(c, [&](auto ncc, auto nvc) {
+        constexpr int NC = decltype(ncc)::value, NV = decltype(nvc)::value;
+        hipLaunchKernelGGL((conv_bands_y_kernel<R, NC, NV>), dim3((c.nk + 255) / 256, nv), dim3(256), 0, s, c.nk,
+                           c.lat.norb, nv, parts, b.Vt, c.d_eval_k.p, c.d_eval_kq.p, c.scissor, b.T.p, X, c.N, Y);
+    });
+    XATU_HIP(hipGetLastError());
+}
+
+// The same with whole meshes in the buffer and rocFFT: 1-D meshes, sides without a factor pair,
+// k-points that share a mesh point.
+template <typename R>
+void conv_mesh_product(Context& c, ConvState& cs, ConvBuffers<R>& b, const double2* X, double2* Y, int nv, hipStream_t s) {
     const int norb = c.lat.norb;
     const int64_t M = cs.M;
+    const int batch = norb * norb * nv;
+    // 2-D meshes: row-interleaved layout, two 1-D passes without transpositions
+    const bool inter = c.lat.ndim == 2;
+    const GLayout lay = inter ? GLayout{c.lat.mesh_n, c.lat.mesh_n, static_cast<int64_t>(batch) * c.lat.mesh_n}
+                              : GLayout{M, 0, 0};
+    b.G.reserve(static_cast<size_t>(batch) * M);
+    if (!cs.full) XATU_HIP(hipMemsetAsync(b.G.p, 0, static_cast<size_t>(batch) * M * sizeof(cx_t<R>), s));
+    conv_bands_in<R>(c, b, X, nv, s);
+    const dim3 kb((c.nk + 255) / 256);
+    with_bands<R>(c, [&](auto ncc, auto nvc) {
+        constexpr int NC = decltype(ncc)::value, NV = decltype(nvc)::value;
+        (void)NV;
+        hipLaunchKernelGGL((conv_z_kernel<R, NC>), dim3(kb.x, (norb + conv_orb_group<R>() - 1) / conv_orb_group<R>(), nv),
+                           dim3(256), 0, s, c.nk, norb, nv, lay, cs.d_gk.p, b.Ct, b.U.p, b.G.p);
+    });
+    XATU_HIP(hipGetLastError());
+    ConvState::Plan& p = get_plan<R>(c, cs, batch, inter);
+    void* buf[1] = {b.G.p};
+    XATU_FFT(rocfft_execute(p.fwd, buf, nullptr, p.info));
+    if (p.fwd2) XATU_FFT(rocfft_execute(p.fwd2, buf, nullptr, p.info));
+    hipLaunchKernelGGL((conv_multiply_kernel<R>), dim3((M + 255) / 256, batch), dim3(256), 0, s, c.lat, nv, M, lay, b.P,
+                       b.G.p);
+    XATU_HIP(hipGetLastError());
+    if (p.bwd2) XATU_FFT(rocfft_execute(p.bwd2, buf, nullptr, p.info));
+    XATU_FFT(rocfft_execute(p.bwd, buf, nullptr, p.info));
+    with_bands<R>(c, [&](auto ncc, auto nvc) {
+        constexpr int NC = decltype(ncc)::value, NV = decltype(nvc)::value;
+        const int yg = (nv + conv_y_group<R>() - 1) / conv_y_group<R>();
+        hipLaunchKernelGGL((conv_y_kernel<R, NC, NV>), dim3(kb.x, yg), dim3(256), 0, s, c.nk, norb, nv, lay, cs.d_gk.p,
+                           b.Ct, b.Vt, c.d_eval_k.p, c.d_eval_kq.p, c.scissor, b.G.p, X, c.N, Y);
+    });
+    XATU_HIP(hipGetLastError());
+}
+
+// Vectors per pass of the row and column transforms (their buffer within kRowsBufferBytes).
+template <typename R>
+int rows_vectors(const Context& c, const ConvState& cs, int nvec) {
+    const size_t per = sizeof(cx_t<R>) * static_cast<size_t>(c.lat.norb) * c.lat.norb * cs.W * c.lat.mesh_n;
+    const int most = static_cast<int>(std::max<size_t>(1, std::min<size_t>(kBlockVectors, kRowsBufferBytes / per)));
+    const int passes = (nvec + most - 1) / most;
+    return (nvec + passes - 1) / passes;
+}
+
+template <typename R>
+void conv_product(Context& c, const double2* X, double2* Y, int nvec, hipStream_t s) {
+    ConvState& cs = *c.conv;
+    ConvBuffers<R> b(cs);
     const int64_t N = c.N;
-    const bool full = (static_cast<int64_t>(c.nk) == M);
+    const int step = cs.rows ? rows_vectors<R>(c, cs, nvec) : kBlockVectors;
+    for (int v0 = 0; v0 < nvec; v0 += step) {
+        const int nv = std::min(step, nvec - v0);
+        const double2* Xb = X + static_cast<int64_t>(v0) * N;
+        double2* Yb = Y + static_cast<int64_t>(v0) * N;
+        if (cs.rows) conv_rows_product<R>(c, cs, b, Xb, Yb, nv, s);
+        else conv_mesh_product<R>(c, cs, b, Xb, Yb, nv, s);
+    }
+    if (!c.inter.exchange) return;
     for (int v0 = 0; v0 < nvec; v0 += kBlockVectors) {
         const int nv = std::min(kBlockVectors, nvec - v0);
         const double2* Xb = X + static_cast<int64_t>(v0) * N;
         double2* Yb = Y + static_cast<int64_t>(v0) * N;
-        const int batch = norb * norb * nv;
-        // 2-D meshes: row-interleaved layout, two 1-D passes without transpositions
-        const bool inter = c.lat.ndim == 2;
-        const GLayout lay = inter ? GLayout{c.lat.mesh_n, c.lat.mesh_n, static_cast<int64_t>(batch) * c.lat.mesh_n}
-                                  : GLayout{M, 0, 0};
-        G.alloc(std::max<size_t>(G.n, static_cast<size_t>(batch) * M));
-        U.alloc(std::max<size_t>(U.n, static_cast<size_t>(nv) * c.nc * norb * c.nk));
-        if (!full) XATU_HIP(hipMemsetAsync(G.p, 0, static_cast<size_t>(batch) * M * sizeof(cx_t<R>), s));
-        const dim3 kb((c.nk + 255) / 256);
-        const int vg = (nv + conv_vec_group<R>() - 1) / conv_vec_group<R>();
-        with_bands<R>(c, [&](auto ncc, auto nvc) {
-            constexpr int NC = decltype(ncc)::value, NV = decltype(nvc)::value;
-            hipLaunchKernelGGL((conv_u_kernel<R, NC, NV>), dim3(kb.x, vg), dim3(256), 0, s, c.nk, norb, nv, Vt, Xb, N,
-                               U.p);
-            hipLaunchKernelGGL((conv_z_kernel<R, NC>), dim3(kb.x, (norb + conv_orb_group<R>() - 1) / conv_orb_group<R>(), nv),
-                               dim3(256), 0, s, c.nk, norb, nv, lay, cs.d_gk.p, Ct, U.p, G.p);
-        });
+        const int na = c.lat.natoms;
+        const int ncv = c.nc * c.nv;
+        const int nblk = static_cast<int>((N + kScanRows - 1) / kScanRows);
+        const int nseries = na * 2 * nv;
+        cs.part.reserve(static_cast<size_t>(nblk) * nseries);
+        cs.total.reserve(static_cast<size_t>(nseries));
+        hipLaunchKernelGGL(xscan_partial_kernel, dim3(nblk, nv), dim3(kScanRows), 0, s, na, ncv, c.d_e1.p, c.d_e2.p, Xb,
+                           N, nv, cs.part.p);
+        hipLaunchKernelGGL(xscan_offsets_kernel, dim3((nseries + 255) / 256), dim3(256), 0, s, nblk, nseries, cs.part.p,
+                           cs.total.p);
+        hipLaunchKernelGGL(xscan_apply_kernel, dim3(nblk, nv), dim3(kScanRows), 0, s, na, ncv, c.d_e1.p, c.d_e2.p, Xb, N,
+                           nv, cs.part.p, cs.total.p, Yb);
         XATU_HIP(hipGetLastError());
-        int fa = 0, fb = 0;
-        four_step_factors(c.lat.mesh_n, fa, fb);
-        const size_t plane_lds = conv_plane_lds<R>(c.lat.mesh_n);
-        if (inter && fa > 0 && plane_lds <= conv_lds_limit(cs)) {
-            // whole planes in LDS: G read and written once
-            hipLaunchKernelGGL((conv_plane_kernel<R, plane_threads<R>()>), dim3(batch), dim3(plane_threads<R>()),
-                               plane_lds, s, c.lat,
-                               c.lat.mesh_n, fa, fb, batch, nv, M, P, G.p);
-        } else {
-            ConvState::Plan& p = get_plan<R>(c, cs, batch, inter);
-            void* buf[1] = {G.p};
-            XATU_FFT(rocfft_execute(p.fwd, buf, nullptr, p.info));
-            if (inter && fa > 0) {
-                const int64_t count = static_cast<int64_t>(batch) * c.lat.mesh_n;
-                hipLaunchKernelGGL((conv_columns4_kernel<R>),
-                                   dim3(static_cast<unsigned>((count + kFourStepCols - 1) / kFourStepCols)), dim3(512), 0,
-                                   s, c.lat, c.lat.mesh_n, fa, fb, count, nv, M, P, G.p);
-            } else {
-                if (p.fwd2) XATU_FFT(rocfft_execute(p.fwd2, buf, nullptr, p.info));
-                hipLaunchKernelGGL((conv_multiply_kernel<R>), dim3((M + 255) / 256, batch), dim3(256), 0, s, c.lat, nv,
-                                   M, lay, P, G.p);
-                if (p.bwd2) XATU_FFT(rocfft_execute(p.bwd2, buf, nullptr, p.info));
-            }
-            XATU_HIP(hipGetLastError());
-            XATU_FFT(rocfft_execute(p.bwd, buf, nullptr, p.info));
-        }
-        XATU_HIP(hipGetLastError());
-        with_bands<R>(c, [&](auto ncc, auto nvc) {
-            constexpr int NC = decltype(ncc)::value, NV = decltype(nvc)::value;
-            const int yg = (nv + conv_y_group<R>() - 1) / conv_y_group<R>();
-            hipLaunchKernelGGL((conv_y_kernel<R, NC, NV>), dim3(kb.x, yg), dim3(256), 0, s, c.nk, norb, nv, lay,
-                               cs.d_gk.p, Ct, Vt, c.d_eval_k.p, c.d_eval_kq.p, c.scissor, G.p, Xb, N, Yb);
-        });
-        XATU_HIP(hipGetLastError());
-        if (c.inter.exchange) {
-            const int na = c.lat.natoms;
-            const int ncv = c.nc * c.nv;
-            const int nblk = static_cast<int>((N + kScanRows - 1) / kScanRows);
-            const int nseries = na * 2 * nv;
-            cs.part.alloc(std::max<size_t>(cs.part.n, static_cast<size_t>(nblk) * nseries));
-            cs.total.alloc(std::max<size_t>(cs.total.n, static_cast<size_t>(nseries)));
-            hipLaunchKernelGGL(xscan_partial_kernel, dim3(nblk, nv), dim3(kScanRows), 0, s, na, ncv, c.d_e1.p,
-                               c.d_e2.p, Xb, N, nv, cs.part.p);
-            hipLaunchKernelGGL(xscan_offsets_kernel, dim3((nseries + 255) / 256), dim3(256), 0, s, nblk, nseries,
-                               cs.part.p, cs.total.p);
-            hipLaunchKernelGGL(xscan_apply_kernel, dim3(nblk, nv), dim3(kScanRows), 0, s, na, ncv, c.d_e1.p, c.d_e2.p,
-                               Xb, N, nv, cs.part.p, cs.total.p, Yb);
-            XATU_HIP(hipGetLastError());
-        }
     }
 }
 
 }  // namespace
+
+// Whether the operator's convolution runs on the row and column transforms.
+bool conv_rows_available(Context& c) {
+    ensure_conv(c);
+    return c.conv->rows;
+}
+
+// Adjoint of the lattice sums for the Hellmann-Feynman gradients, on the cells directly:
+//   Shat_p(R) = sum_q [S_ab(q) e^{iqR} + S_ba(q) e^{-iqR}] (a < b),  sum_q S_aa(q) e^{-iqR} (a = b)
+// with S_ab(q) the pair densities of conv_pair_density. Their transform is the power spectrum of
+// z, so Shat_p(R) = sum_{al in a, be in b} |Z_{al be}(-R)|^2 + sum_{al in b, be in a} |Z_{al be}(R)|^2
+// (a = b: one sum, at R), Z the forward transform of z on the window that holds every cell.
+// shat[(s npairs + p) nR + R] for the ns <= 32 states of psi (N x ns).
+void conv_cell_density(Context& c, const double2* psi, int ns, double* shat) {
+    ensure_conv(c);
+    ConvState& cs = *c.conv;
+    ConvBuffers<double> b(cs);
+    hipStream_t s = c.stream;
+    const int npairs = c.lat.natoms * (c.lat.natoms + 1) / 2;
+    conv_bands_in<double>(c, b, psi, ns, s);
+    conv_rows_forward<double>(c, cs, b, ns, false, s);
+    hipLaunchKernelGGL(cell_power_kernel, dim3((c.nR + 255) / 256, npairs, ns), dim3(256), 0, s, c.lat, cs.W, cs.w0,
+                       c.d_cells.p, c.nR, npairs, ns, b.G.p, shat);
+    XATU_HIP(hipGetLastError());
+}
 
 // Pair-density adjoint of the direct term for the Hellmann-Feynman gradients:
 //   S_ab(q) = sum_k G_ab(k, k+q),  G_ab(k,k') = sum_{al in a, be in b} conj(z_ab(k)) z_ab(k'),
@@ -1135,7 +1003,7 @@ void conv_pair_density(Context& c, const double2* psi, int ns, double2* S) {
     const int batch = norb * norb * ns;
     cs.G64.alloc(std::max<size_t>(cs.G64.n, static_cast<size_t>(batch) * M));
     cs.U64.alloc(std::max<size_t>(cs.U64.n, static_cast<size_t>(ns) * c.nc * norb * c.nk));
-    if (static_cast<int64_t>(c.nk) != M) XATU_HIP(hipMemsetAsync(cs.G64.p, 0, static_cast<size_t>(batch) * M * sizeof(double2), s));
+    if (!cs.full) XATU_HIP(hipMemsetAsync(cs.G64.p, 0, static_cast<size_t>(batch) * M * sizeof(double2), s));
     const dim3 kb((c.nk + 255) / 256);
     with_bands<double>(c, [&](auto ncc, auto nvc) {
         constexpr int NC = decltype(ncc)::value, NV = decltype(nvc)::value;
@@ -1164,12 +1032,12 @@ void conv_pair_density(Context& c, const double2* psi, int ns, double2* S) {
 
 void launch_conv64(Context& c, const double2* X, double2* Y, int nvec, hipStream_t s) {
     ensure_conv(c);
-    conv_product<double>(c, X, Y, nvec, s, c.conv->G64, c.conv->U64, c.conv->P64.p, c.conv->Ct64.p, c.conv->Vt64.p);
+    conv_product<double>(c, X, Y, nvec, s);
 }
 
 void launch_conv32(Context& c, const double2* X, double2* Y, int nvec, hipStream_t s) {
     ensure_conv(c);
-    conv_product<float>(c, X, Y, nvec, s, c.conv->G32, c.conv->U32, c.conv->P32.p, c.conv->Ct32.p, c.conv->Vt32.p);
+    conv_product<float>(c, X, Y, nvec, s);
 }
 
 }  // namespace xatu_dev

@@ -34,6 +34,7 @@ namespace {
 
 constexpr int kHfThreads = 256;
 constexpr int kHfStates = 4;  // states per pass of the pair-density adjoint
+constexpr int kHfRowStates = 8;  // ... when it runs on the row and column transforms
 
 // dV/dtheta for pair p and cell R. which: 0 r0, 1 eps (m or s: identical).
 __global__ void dpotential_table_kernel(LatticeDesc lat, PotDesc pot, const int* __restrict__ cells, int nR, int npairs,
@@ -248,8 +249,16 @@ void hf_gradients(Context& c, int nstates, const double2* d_vec, int nparams, co
     S.alloc(static_cast<size_t>(kHfStates) * c.lat.nmesh * na * na);
     DevBuf<double> shat;
     shat.alloc(static_cast<size_t>(nstates) * npairs * nR);
-    for (int s0 = 0; s0 < nstates; s0 += kHfStates) {
-        const int ns = std::min(kHfStates, nstates - s0);
+    const bool direct = c.lat.ndim == 2 && conv_rows_available(c);
+    const int step = direct ? kHfRowStates : kHfStates;
+    for (int s0 = 0; s0 < nstates; s0 += step) {
+        const int ns = std::min(step, nstates - s0);
+        if (direct) {
+            // the cells' adjoint is the power spectrum of the transforms: no sums over q
+            conv_cell_density(c, d_vec + static_cast<int64_t>(s0) * c.N, ns,
+                              shat.p + static_cast<size_t>(s0) * npairs * nR);
+            continue;
+        }
         if (c.lat.ndim <= 2) {
             // autocorrelation on the mesh with FFTs: O(norb^2 M log M) instead of O(nk^2) pairs
             conv_pair_density(c, d_vec + static_cast<int64_t>(s0) * c.N, ns, S.p);

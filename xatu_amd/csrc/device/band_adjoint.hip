@@ -27,11 +27,13 @@
 //   g_B(c',al)  += -1/2 [ sum_c  conj Y_t(c,c') A_c,al - sum_v' conj T_t(v',c') P_v',al ]
 //   g_Q(v,al)   += -1/2 [ sum_v' conj S_t(v',v) P_v',al - sum_c conj U_t(c,v) A_c,al ]
 // (A and P enter F conjugated, so their derivative is -1/2 p dF/d conj; B and Q enter
-// holomorphically, so theirs is -1/2 conj(p dF/dB)). Every canonical pair is handled by
-// one thread, which adds its contributions to the four coefficient vectors with
-// hardware FP64 atomics. Conduction vectors belong to the k+Q stack, valence vectors
+// holomorphically, so theirs is -1/2 conj(p dF/dB)). Where the operator is a convolution on a
+// 2-D mesh with row and column transforms the same sums come from those (conv_band_adjoint);
+// otherwise (1-D and 3-D meshes, the reciprocal-space table, other mesh sides) every
+// canonical pair is handled by one thread, which adds its contributions to the four
+// coefficient vectors with hardware FP64 atomics. Conduction vectors belong to the k+Q stack, valence vectors
 // to the k stack, as in the assembly.
-#include <vector>
+#include <algorithm>
 
 #include "context.hpp"
 #include "cplx.hpp"
@@ -41,13 +43,15 @@ namespace xatu_dev {
 
 namespace {
 
+constexpr int kBandStates = 8;  // states per pass of the transforms
+
 __device__ inline void atomic_add_cx(double2* p, double2 v) {
     unsafeAtomicAdd(&p->x, v.x);
     unsafeAtomicAdd(&p->y, v.y);
 }
 
 template <int NA, int NC, int NV, int TK>
-__global__ __launch_bounds__(TK* TK) void band_adjoint_kernel(LatticeDesc lat, int nk, const double2* __restrict__ evk,
+__global__ __launch_bounds__(TK* TK) void band_adjoint_pairs_kernel(LatticeDesc lat, int nk, const double2* __restrict__ evk,
                                                               const double2* __restrict__ evkq,
                                                               const int* __restrict__ kcoord,
                                                               const double2* __restrict__ ft,
@@ -301,22 +305,24 @@ __global__ __launch_bounds__(TK* TK) void band_adjoint_kernel(LatticeDesc lat, i
 }
 
 template <int NA, int NC, int NV>
-bool launch_shape(const Context& c, const double2* psi, double2* gK, double2* gKQ, hipStream_t s) {
-    if (c.lat.natoms != NA || c.nc != NC || c.nv != NV) return false;
+void launch_shape(const Context& c, const double2* psi, double2* gK, double2* gKQ, hipStream_t s) {
     constexpr int TK = 8;
     const size_t lds = static_cast<size_t>(2 * TK) * c.lat.norb * (NC + NV) * sizeof(double2);
-    if (lds > 160 * 1024) throw Error(XATU_ERR_INVALID_ARGUMENT, "too many orbitals for the band adjoint kernel");
     const int nT = (c.nk + TK - 1) / TK;
-    hipLaunchKernelGGL((band_adjoint_kernel<NA, NC, NV, TK>), dim3(nT, nT), dim3(TK * TK), lds, s, c.lat, c.nk,
+    hipLaunchKernelGGL((band_adjoint_pairs_kernel<NA, NC, NV, TK>), dim3(nT, nT), dim3(TK * TK), lds, s, c.lat, c.nk,
                        c.d_evec_k.p, c.d_evec_kq.p, c.d_kcoord.p, c.d_ft.p, c.d_ftq.p, c.d_e1.p, c.d_e2.p,
                        c.inter.exchange, psi, gK, gKQ);
     XATU_HIP(hipGetLastError());
-    return true;
 }
 
-bool launch_band_adjoint(const Context& c, const double2* psi, double2* gK, double2* gKQ, hipStream_t s) {
+using PairsLauncher = void (*)(const Context&, const double2*, double2*, double2*, hipStream_t);
+
+// The pair kernel of the context's shape; refuses the shapes that have none (the gradients are
+// offered for the same shapes whichever way they are computed).
+PairsLauncher pairs_launcher(const Context& c) {
+    PairsLauncher f = nullptr;
 #define XATU_BA_SHAPE(NA, NC, NV) \
-    if (launch_shape<NA, NC, NV>(c, psi, gK, gKQ, s)) return true;
+    if (c.lat.natoms == NA && c.nc == NC && c.nv == NV) f = launch_shape<NA, NC, NV>;
     XATU_BA_SHAPE(1, 1, 1)
     XATU_BA_SHAPE(1, 2, 2)
     XATU_BA_SHAPE(2, 1, 1)
@@ -327,44 +333,70 @@ bool launch_band_adjoint(const Context& c, const double2* psi, double2* gK, doub
     XATU_BA_SHAPE(4, 2, 2)
     XATU_BA_SHAPE(4, 3, 3)
 #undef XATU_BA_SHAPE
-    return false;
+    if (!f) {
+        throw Error(XATU_ERR_INVALID_ARGUMENT,
+                    "band gradients support natoms <= 4 and nv == nc <= 2 (nv == nc == 3 with 4 atoms)");
+    }
+    if (static_cast<size_t>(16) * c.lat.norb * c.nb * sizeof(double2) > 160 * 1024) {
+        throw Error(XATU_ERR_INVALID_ARGUMENT, "too many orbitals for the band adjoint kernel");
+    }
+    return f;
+}
+
+// w[((n 2 + stack) nk + k) nb + b]: dE/dE_c(k+Q) = sum_v |psi|^2, dE/dE_v(k) = -sum_c |psi|^2, zero for
+// the other columns of each stack. grid (ceil(nk / 256), states)
+__global__ void band_energy_kernel(int nk, int nv, int nc, const double2* __restrict__ psi, int64_t N,
+                                   double* __restrict__ w) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= nk) return;
+    const int n = blockIdx.y, nb = nv + nc;
+    const double2* p = psi + static_cast<int64_t>(n) * N + static_cast<int64_t>(k) * nc * nv;
+    double* wk = w + (static_cast<size_t>(n) * 2 * nk + k) * nb;
+    double* wq = wk + static_cast<size_t>(nk) * nb;
+    for (int v = 0; v < nv; ++v) {
+        double s = 0.0;
+        for (int c = 0; c < nc; ++c) s -= p[c * nv + v].x * p[c * nv + v].x + p[c * nv + v].y * p[c * nv + v].y;
+        wk[v] = s;
+        wq[v] = 0.0;
+    }
+    for (int c = 0; c < nc; ++c) {
+        double s = 0.0;
+        for (int v = 0; v < nv; ++v) s += p[c * nv + v].x * p[c * nv + v].x + p[c * nv + v].y * p[c * nv + v].y;
+        wq[nv + c] = s;
+        wk[nv + c] = 0.0;
+    }
 }
 
 }  // namespace
 
 void band_gradients(Context& c, int nstates, const double2* d_vec, double* w_out, double* g_out) {
     if (!c.prepared) throw Error(XATU_ERR_LOGIC, "operator not prepared (call xatu_build_bse)");
+    const PairsLauncher pairs = pairs_launcher(c);
     const size_t stack = static_cast<size_t>(c.lat.norb) * c.nb * c.nk;  // complex entries per stack
     const int64_t N = c.N;
     hipStream_t s = c.stream;
+    DevBuf<double> w;
+    w.alloc(static_cast<size_t>(nstates) * 2 * c.nb * c.nk);
+    hipLaunchKernelGGL(band_energy_kernel, dim3((c.nk + 255) / 256, nstates), dim3(256), 0, s, c.nk, c.nv, c.nc, d_vec, N,
+                       w.p);
+    XATU_HIP(hipGetLastError());
+    const bool direct = c.lat.ndim == 2 && !c.lat.recip && conv_rows_available(c);
+    const int step = direct ? std::min(nstates, kBandStates) : 1;
     DevBuf<double2> g;
-    g.alloc(2 * stack);
-    std::vector<double2> psi(static_cast<size_t>(N) * nstates);
-    XATU_HIP(hipMemcpyAsync(psi.data(), d_vec, psi.size() * sizeof(double2), hipMemcpyDeviceToHost, s));
-    for (int st = 0; st < nstates; ++st) {
-        XATU_HIP(hipMemsetAsync(g.p, 0, g.bytes(), s));
-        if (!launch_band_adjoint(c, d_vec + static_cast<int64_t>(st) * N, g.p, g.p + stack, s)) {
-            throw Error(XATU_ERR_INVALID_ARGUMENT,
-                        "band gradients support natoms <= 4 and nv == nc <= 2 (nv == nc == 3 with 4 atoms)");
+    g.alloc(2 * stack * step);
+    for (int st = 0; st < nstates; st += step) {
+        const int ns = std::min(step, nstates - st);
+        const double2* psi = d_vec + static_cast<int64_t>(st) * N;
+        if (direct) {
+            conv_band_adjoint(c, psi, ns, g.p);
+        } else {
+            XATU_HIP(hipMemsetAsync(g.p, 0, g.bytes(), s));
+            pairs(c, psi, g.p, g.p + stack, s);
         }
-        XATU_HIP(hipMemcpyAsync(g_out + 2 * (2 * stack) * st, g.p, g.bytes(), hipMemcpyDeviceToHost, s));
+        XATU_HIP(hipMemcpyAsync(g_out + 4 * stack * st, g.p, 2 * stack * ns * sizeof(double2), hipMemcpyDeviceToHost, s));
     }
+    XATU_HIP(hipMemcpyAsync(w_out, w.p, w.bytes(), hipMemcpyDeviceToHost, s));
     XATU_HIP(hipStreamSynchronize(s));
-    // energy sensitivities: dE/dE_c(k+Q) = sum_v |psi|^2, dE/dE_v(k) = -sum_c |psi|^2
-    const int nb = c.nb, nv = c.nv, nc = c.nc, ncv = nc * nv;
-    for (int st = 0; st < nstates; ++st) {
-        double* wk = w_out + static_cast<size_t>(st) * 2 * nb * c.nk;
-        double* wkq = wk + static_cast<size_t>(nb) * c.nk;
-        for (size_t i = 0; i < static_cast<size_t>(2) * nb * c.nk; ++i) wk[i] = 0.0;
-        for (int k = 0; k < c.nk; ++k)
-            for (int ic = 0; ic < nc; ++ic)
-                for (int iv = 0; iv < nv; ++iv) {
-                    const double2 z = psi[static_cast<size_t>(st) * N + static_cast<size_t>(k) * ncv + ic * nv + iv];
-                    const double a2 = z.x * z.x + z.y * z.y;
-                    wkq[static_cast<size_t>(k) * nb + nv + ic] += a2;
-                    wk[static_cast<size_t>(k) * nb + iv] -= a2;
-                }
-    }
 }
 
 }  // namespace xatu_dev

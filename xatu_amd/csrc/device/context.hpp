@@ -352,6 +352,8 @@ void conv_pair_density(Context& c, const double2* psi, int ns, double2* S);
 // on the cells, shat[(s npairs + p) nR + R], for ns <= 32 states.
 bool conv_rows_available(Context& c);
 void conv_cell_density(Context& c, const double2* psi, int ns, double* shat);
+// ... and the derivatives by the band vectors (2 stacks of norb x nb x nk per state).
+void conv_band_adjoint(Context& c, const double2* psi, int ns, double2* g);
 // Matrix-free products Y = H X (complex FP64 vectors) with tiles of H recomputed in
 // FP64 / FP32 arithmetic inside the product (FP32: FP32 tiles, FP32 accumulation).
 void launch_matfree64(Context& c, const double2* X, double2* Y, int nvec, hipStream_t s);

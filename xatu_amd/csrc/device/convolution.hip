@@ -529,6 +529,118 @@ __global__ void power_sum_kernel(LatticeDesc lat, int ns, int64_t M, const doubl
     Pw[(static_cast<int64_t>(n) * lat.natoms * lat.natoms + ab) * M + xi] = mk(sum, 0.0);
 }
 
+// Scans of the exchange adjoint, from the block sums of xscan_partial_kernel with x = psi:
+//   S_a(i) = 2 sum_{j>i} A_a(j) + A_a(i),  F_a(i) = conj(2 sum_{j<i} B_a(j) + B_a(i)),
+// A_a = E2_a psi, B_a = conj(E1_a) psi; S[(n NA + a) N + i] and F likewise. grid (blocks, nvec).
+__global__ __launch_bounds__(kScanRows) void xscan_adjoint_kernel(int na, int ncv, const double2* __restrict__ e1,
+                                                                  const double2* __restrict__ e2,
+                                                                  const double2* __restrict__ X, int64_t N, int nvec,
+                                                                  const double2* __restrict__ part,
+                                                                  const double2* __restrict__ total,
+                                                                  double2* __restrict__ S, double2* __restrict__ F) {
+    __shared__ double2 s[kScanRows];
+    const int n = blockIdx.y;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kScanRows + threadIdx.x;
+    const bool ok = i < N;
+    const double2 x = ok ? X[i + n * N] : mk(0.0, 0.0);
+    const int64_t k = ok ? i / ncv : 0;
+    const int cv = ok ? static_cast<int>(i % ncv) : 0;
+    const int nseries = na * 2 * nvec;
+    for (int a = 0; a < na; ++a) {
+        const size_t off = (static_cast<size_t>(k) * na + a) * ncv + cv;
+        for (int sidx = 0; sidx < 2; ++sidx) {
+            const double2 e = ok ? (sidx == 0 ? e2[off] : cconj(e1[off])) : mk(0.0, 0.0);
+            const double2 v = cmul(e, x);
+            s[threadIdx.x] = v;
+            __syncthreads();
+            for (int st = 1; st < kScanRows; st <<= 1) {
+                const double2 add = threadIdx.x >= st ? s[threadIdx.x - st] : mk(0.0, 0.0);
+                __syncthreads();
+                s[threadIdx.x] = cadd(s[threadIdx.x], add);
+                __syncthreads();
+            }
+            const size_t ser = (static_cast<size_t>(a) * 2 + sidx) * nvec + n;
+            const double2 incl = cadd(part[static_cast<size_t>(blockIdx.x) * nseries + ser], s[threadIdx.x]);
+            if (ok) {
+                const size_t out = (static_cast<size_t>(n) * na + a) * N + i;
+                if (sidx == 0) {
+                    const double2 after = csub(total[ser], incl);
+                    S[out] = mk(2.0 * after.x + v.x, 2.0 * after.y + v.y);
+                } else {
+                    const double2 before = csub(incl, v);
+                    F[out] = mk(2.0 * before.x + v.x, -(2.0 * before.y + v.y));
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// Band-vector derivatives of one state per blockIdx.y (see conv_band_adjoint): thread per
+// (k, orbital), the orbital fastest. g[((n 2 + stack) nk + k) nb + b) norb + orbital].
+__global__ __launch_bounds__(256) void band_adjoint_kernel(LatticeDesc lat, int nk, int nv, int nc, int nvec, int parts1,
+                                                           int parts2, const double2* __restrict__ Ct,
+                                                           const double2* __restrict__ Vt,
+                                                           const double2* __restrict__ psi, int64_t N,
+                                                           const double2* __restrict__ T1,
+                                                           const double2* __restrict__ T2, int exchange,
+                                                           const double2* __restrict__ ftq,
+                                                           const double2* __restrict__ S,
+                                                           const double2* __restrict__ F, double2* __restrict__ g) {
+    const int norb = lat.norb, na = lat.natoms, nb = nv + nc, ncv = nc * nv;
+    const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (idx >= static_cast<int64_t>(nk) * norb) return;
+    const int al = static_cast<int>(idx % norb), k = static_cast<int>(idx / norb);
+    const int n = blockIdx.y;
+    const int a = atom_of(lat, al);
+    const double2* p = psi + static_cast<int64_t>(n) * N + static_cast<int64_t>(k) * ncv;
+    const size_t stack = static_cast<size_t>(nk) * nb * norb;
+    double2* gk = g + static_cast<size_t>(n) * 2 * stack + static_cast<size_t>(k) * nb * norb + al;
+    double2* gq = gk + stack;
+    auto term = [&](const double2* T, int parts, int nch, int ch) {
+        double2 t = mk(0.0, 0.0);
+        for (int q = 0; q < parts; ++q)
+            t = cadd(t, T[(((static_cast<size_t>(q) * nvec + n) * nch + ch) * norb + al) * nk + k]);
+        return t;
+    };
+    // H_a = S_a + conj(sum_b F_b MQ_ba) of a row
+    auto row_h = [&](int cv) {
+        const size_t i = static_cast<size_t>(k) * ncv + cv;
+        double2 f = mk(0.0, 0.0);
+        for (int b = 0; b < na; ++b) cfma(f, F[(static_cast<size_t>(n) * na + b) * N + i], ftq[b + na * a]);
+        return cadd(S[(static_cast<size_t>(n) * na + a) * N + i], cconj(f));
+    };
+    for (int c = 0; c < nc; ++c) {
+        double2 s = mk(0.0, 0.0);
+        for (int v = 0; v < nv; ++v) {
+            const double2 q = cconj(p[c * nv + v]);
+            double2 t = term(T2, parts2, nv, v);
+            t = mk(-t.x, -t.y);
+            if (exchange) {
+                const double2 h = cmul(row_h(c * nv + v), Vt[(static_cast<size_t>(v) * norb + al) * nk + k]);
+                t = mk(t.x + 0.5 * h.x, t.y + 0.5 * h.y);
+            }
+            cfma(s, q, t);
+        }
+        gq[(nv + c) * norb] = s;
+        gk[(nv + c) * norb] = mk(0.0, 0.0);
+    }
+    for (int v = 0; v < nv; ++v) {
+        double2 s = mk(0.0, 0.0);
+        for (int c = 0; c < nc; ++c) {
+            double2 t = cconj(term(T1, parts1, nc, c));
+            t = mk(-t.x, -t.y);
+            if (exchange) {
+                const double2 h = cmul(cconj(row_h(c * nv + v)), Ct[(static_cast<size_t>(c) * norb + al) * nk + k]);
+                t = mk(t.x + 0.5 * h.x, t.y + 0.5 * h.y);
+            }
+            cfma(s, p[c * nv + v], t);
+        }
+        gk[v * norb] = s;
+        gq[v * norb] = mk(0.0, 0.0);
+    }
+}
+
 // shat[(s npairs + p) nR + R] from the forward transforms G[(xi_1 batch + (al norb + be) ns + s) W + j]
 // (see conv_cell_density); grid (ceil(nR / 256), npairs, ns)
 __global__ void cell_power_kernel(LatticeDesc lat, int W, int w0, const int* __restrict__ cells, int nR, int npairs,
@@ -600,6 +712,7 @@ struct ConvState {
     DevBuf<double2> G64, U64, Ct64, Vt64;
     DevBuf<float2> G32, U32, Ct32, Vt32;
     DevBuf<double2> part, total;
+    DevBuf<double2> S, F, T64b;  // exchange scans and second contraction of the band adjoint
     DevBuf<double2> Mt;  // interaction table on the mesh (set-up scratch, kept between set-ups)
     // row and column transforms (2-D meshes with a supported side): window of the first axis, real
     // spectra on it, cell lists of the spectrum, k-point of each mesh point (-1: none)
@@ -924,6 +1037,21 @@ int rows_vectors(const Context& c, const ConvState& cs, int nvec) {
     return (nvec + passes - 1) / passes;
 }
 
+// Block sums of the exchange scans of nv vectors, as offsets (cs.part) and totals; returns the
+// number of blocks.
+int exchange_scans(Context& c, ConvState& cs, const double2* X, int nv, hipStream_t s) {
+    const int nblk = static_cast<int>((c.N + kScanRows - 1) / kScanRows);
+    const int nseries = c.lat.natoms * 2 * nv;
+    cs.part.reserve(static_cast<size_t>(nblk) * nseries);
+    cs.total.reserve(static_cast<size_t>(nseries));
+    hipLaunchKernelGGL(xscan_partial_kernel, dim3(nblk, nv), dim3(kScanRows), 0, s, c.lat.natoms, c.nc * c.nv, c.d_e1.p,
+                       c.d_e2.p, X, c.N, nv, cs.part.p);
+    hipLaunchKernelGGL(xscan_offsets_kernel, dim3((nseries + 255) / 256), dim3(256), 0, s, nblk, nseries, cs.part.p,
+                       cs.total.p);
+    XATU_HIP(hipGetLastError());
+    return nblk;
+}
+
 template <typename R>
 void conv_product(Context& c, const double2* X, double2* Y, int nvec, hipStream_t s) {
     ConvState& cs = *c.conv;
@@ -944,14 +1072,7 @@ void conv_product(Context& c, const double2* X, double2* Y, int nvec, hipStream_
         double2* Yb = Y + static_cast<int64_t>(v0) * N;
         const int na = c.lat.natoms;
         const int ncv = c.nc * c.nv;
-        const int nblk = static_cast<int>((N + kScanRows - 1) / kScanRows);
-        const int nseries = na * 2 * nv;
-        cs.part.reserve(static_cast<size_t>(nblk) * nseries);
-        cs.total.reserve(static_cast<size_t>(nseries));
-        hipLaunchKernelGGL(xscan_partial_kernel, dim3(nblk, nv), dim3(kScanRows), 0, s, na, ncv, c.d_e1.p, c.d_e2.p, Xb,
-                           N, nv, cs.part.p);
-        hipLaunchKernelGGL(xscan_offsets_kernel, dim3((nseries + 255) / 256), dim3(256), 0, s, nblk, nseries, cs.part.p,
-                           cs.total.p);
+        const int nblk = exchange_scans(c, cs, Xb, nv, s);
         hipLaunchKernelGGL(xscan_apply_kernel, dim3(nblk, nv), dim3(kScanRows), 0, s, na, ncv, c.d_e1.p, c.d_e2.p, Xb, N,
                            nv, cs.part.p, cs.total.p, Yb);
         XATU_HIP(hipGetLastError());
@@ -983,6 +1104,55 @@ void conv_cell_density(Context& c, const double2* psi, int ns, double* shat) {
     hipLaunchKernelGGL(cell_power_kernel, dim3((c.nR + 255) / 256, npairs, ns), dim3(256), 0, s, c.lat, cs.W, cs.w0,
                        c.d_cells.p, c.nR, npairs, ns, b.G.p, shat);
     XATU_HIP(hipGetLastError());
+}
+
+// Adjoint of the assembly with respect to the band vectors by the same transforms: with
+// z_{al be} = sum_cv C_al conj(V_be) psi_cv and w = M (*) z the direct term's energy is
+// -sum_k conj(z) w, so that (Wirtinger derivatives by the conjugated coefficients, M Hermitian)
+//   g_C(c, al) = -sum_v conj(psi_cv) sum_be V_be,v w_{al be},
+//   g_V(v, be) = -sum_c psi_cv conj(sum_al conj(C_al,c) w_{al be}):
+// the contraction of the product and the same with the orbitals exchanged. The exchange term
+// along the upper triangle, Re sum_a [2 sum_{i<j} f_a(i) A_a(j) + sum_i f_a(i) A_a(i)] with
+// f_a = conj(psi) E1_a and A_a = E2_a psi, adds with its scans S and F (xscan_adjoint_kernel) and
+// H_a = S_a + conj(sum_b F_b MQ_ba)
+//   g_C(c, al) += 1/2 sum_v conj(psi_cv) V_al,v H_a,  g_V(v, al) += 1/2 sum_c psi_cv C_al,c conj(H_a).
+// Cost per state: the transforms of one product, against nk^2 / 2 pairs of k-points with atomic
+// adds (36 x 36, 18 orbitals, 8 states: 0.2 ms for 104 ms). g: ns states of 2 stacks.
+void conv_band_adjoint(Context& c, const double2* psi, int ns, double2* g) {
+    ensure_conv(c);
+    ConvState& cs = *c.conv;
+    ConvBuffers<double> b(cs);
+    hipStream_t s = c.stream;
+    const int norb = c.lat.norb, na = c.lat.natoms;
+    const size_t stack = static_cast<size_t>(norb) * c.nb * c.nk;
+    const int step = rows_vectors<double>(c, cs, std::min(ns, kBlockVectors));
+    for (int v0 = 0; v0 < ns; v0 += step) {
+        const int nv = std::min(step, ns - v0);
+        const double2* X = psi + static_cast<int64_t>(v0) * c.N;
+        conv_bands_in<double>(c, b, X, nv, s);
+        conv_rows_forward<double>(c, cs, b, nv, true, s);
+        const RowsArgs a1 = rows_args(c, cs, nv);
+        RowsArgs a2 = a1;  // fixed al, looped be
+        a2.conj = 0;
+        a2.sl = nv;
+        a2.sf = static_cast<int64_t>(norb) * nv;
+        const int parts = rows_out_chunks(a1);
+        b.T.reserve(static_cast<size_t>(parts) * nv * c.nc * norb * c.nk);
+        cs.T64b.reserve(static_cast<size_t>(parts) * nv * c.nv * norb * c.nk);
+        launch_rows_out<double>(a1, c.nc, parts, cs.d_kmap.p, c.d_twiddle.p, b.Ct, b.G.p, b.T.p, s);
+        launch_rows_out<double>(a2, c.nv, parts, cs.d_kmap.p, c.d_twiddle.p, b.Vt, b.G.p, cs.T64b.p, s);
+        if (c.inter.exchange) {
+            const int nblk = exchange_scans(c, cs, X, nv, s);
+            cs.S.reserve(static_cast<size_t>(nv) * na * c.N);
+            cs.F.reserve(static_cast<size_t>(nv) * na * c.N);
+            hipLaunchKernelGGL(xscan_adjoint_kernel, dim3(nblk, nv), dim3(kScanRows), 0, s, na, c.nc * c.nv, c.d_e1.p,
+                               c.d_e2.p, X, c.N, nv, cs.part.p, cs.total.p, cs.S.p, cs.F.p);
+        }
+        hipLaunchKernelGGL(band_adjoint_kernel, dim3((static_cast<size_t>(c.nk) * norb + 255) / 256, nv), dim3(256), 0, s,
+                           c.lat, c.nk, c.nv, c.nc, nv, parts, parts, b.Ct, b.Vt, X, c.N, b.T.p, cs.T64b.p,
+                           c.inter.exchange, c.d_ftq.p, cs.S.p, cs.F.p, g + 2 * stack * v0);
+        XATU_HIP(hipGetLastError());
+    }
 }
 
 // Pair-density adjoint of the direct term for the Hellmann-Feynman gradients:

@@ -78,13 +78,9 @@ std::vector<int> truncate_supercell(const double* vecs, int ndim, int ncell, dou
     const int shift = ncell / 2;
     long long total = 1;
     for (int j = 0; j < ndim; ++j) total *= ncell;
+    int m[3] = {0, 0, 0};
+    for (int j = 0; j < ndim; ++j) m[j] = -shift;
     for (long long i = 0; i < total; ++i) {
-        int m[3] = {0, 0, 0};
-        long long rem = i;
-        for (int j = 0; j < ndim; ++j) {
-            m[j] = static_cast<int>(rem % ncell) - shift;
-            rem /= ncell;
-        }
         double v[3] = {0.0, 0.0, 0.0};
         for (int j = 0; j < ndim; ++j) {
             v[0] += m[j] * vecs[3 * j + 0];
@@ -95,6 +91,7 @@ std::vector<int> truncate_supercell(const double* vecs, int ndim, int ncell, dou
         if (d < radius + 1E-5) {
             for (int j = 0; j < ndim; ++j) out.push_back(m[j]);
         }
+        for (int j = 0; j < ndim && ++m[j] == ncell - shift; ++j) m[j] = -shift;
     }
     return out;
 }
@@ -440,6 +437,18 @@ int xatu_fourier_sums(xatu_ctx* ctx, const xatu_interaction* inter) {
         c.d_cells.alloc(padded.size());
         XATU_HIP(hipMemcpyAsync(c.d_cells.p, padded.data(), padded.size() * sizeof(int), hipMemcpyHostToDevice,
                                 c.stream));
+        std::vector<int4> rows;
+        if (c.lat.ndim == 2) {
+            // consecutive cells of one second coefficient, the first one counting up
+            for (int r = 0; r < c.nR; ++r) {
+                const int m1 = c.h_cells[2 * static_cast<size_t>(r)], m2 = c.h_cells[2 * static_cast<size_t>(r) + 1];
+                if (!rows.empty() && rows.back().x == m2 && rows.back().y + rows.back().w == m1) ++rows.back().w;
+                else rows.push_back(make_int4(m2, m1, r, 1));
+            }
+            c.d_rows.reserve(rows.size());
+            XATU_HIP(hipMemcpyAsync(c.d_rows.p, rows.data(), rows.size() * sizeof(int4), hipMemcpyHostToDevice, c.stream));
+        }
+        c.n_rows = static_cast<int>(rows.size());
         const int npairs = c.lat.natoms * (c.lat.natoms + 1) / 2;
         const int na2 = c.lat.natoms * c.lat.natoms;
         c.d_vtab.alloc(static_cast<size_t>(npairs) * c.nR);

@@ -179,6 +179,9 @@ struct Context {
     int nR = 0;
     std::vector<int> h_cells;   // nR x ndim integer coefficients
     DevBuf<int> d_cells;        // nR x 3 (padded)
+    int n_rows = 0;
+    DevBuf<int4> d_rows;        // 2-D: the cells as rows {m_2, first m_1, first cell, count}
+    DevBuf<double2> d_rowsum;   // sums along the rows and their remainders
     DevBuf<double> d_vtab;      // npairs x nR direct potential table
     DevBuf<double> d_vtabx;     // npairs x nR exchange potential table
     DevBuf<double2> d_twiddle;  // 2*mesh_n roots of unity
@@ -295,7 +298,7 @@ struct EventTimer {
 // Kernel launchers implemented in the .hip translation units.
 void launch_potential_table(const Context& c, const PotDesc& pot, double* out, hipStream_t s);
 void launch_twiddles(int mesh_n, double2* out, hipStream_t s);
-void launch_fourier_mesh(const Context& c, hipStream_t s);
+void launch_fourier_mesh(Context& c, hipStream_t s);
 void launch_fourier_q(const Context& c, hipStream_t s);
 // Reciprocal-mode tables: M_ab(q) over the raw mesh differences into d_ft and, with
 // exchange, M_ab(Q) into d_ftq; d_gvec holds ng reciprocal lattice vectors (x, y, z).

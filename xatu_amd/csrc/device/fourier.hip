@@ -14,7 +14,7 @@
 // the rows then (fourier_mesh2_kernel): rows (cells of a row + n) n terms per pair instead of cells n^2.
 // Both steps carry sum and remainder (error-free products and sums), so that splitting the
 // phase in two rounded roots costs what the rounded products of the direct sum cost (measured
-against extended precision, 16 to 128 points a side: rms 0.6 to 0.9 of the direct sum's). Bound by
+// against extended precision, 16 to 128 points a side: rms 0.6 to 0.9 of the direct sum's). Bound by
 // FP64 latency, a few microseconds of arithmetic: 120 x 120, 2263 cells, 10 pairs: 652 -> 38 us.
 // 1-D and 3-D meshes: one workgroup owns one mesh point; its threads stream R (coalesced
 // table reads), accumulate with Neumaier compensation, and reduce pairwise through LDS.

@@ -351,9 +351,13 @@ __global__ __launch_bounds__(256) void conv_y_kernel(int nk, int norb, int nvec,
 }
 
 // Y[k NCV + c NV + v, n] = e(kcv) x - sum_be V_k[be, v] t[n][c][be][k] with t the sum of the
-// parts that conv_rows_out_kernel left (T[((part nvec + n) NC + c) norb + be][k]); thread per k,
-// blockIdx.y = vector n
-template <typename R, int NC, int NV>
+// parts that conv_rows_out_kernel left (T[((part nvec + n) NC + c) norb + be][k]). grid (k, vector);
+// S threads of a workgroup share a k-point, each with the orbitals be = its number modulo S, and their sums
+// meet in LDS. Reads T once, so bound by HBM when there are many k-points and vectors (S = 1) and
+// by the latency of the loads of one thread when there are few (S = kBandsShare; 25 x 25, 4 vectors,
+// 18 orbitals, FP64: 76 -> 14 us; 48 x 48, 8 vectors, 8 orbitals: 20 -> 10 us).
+constexpr int kBandsShare = 8;
+template <typename R, int NC, int NV, int S>
 __global__ __launch_bounds__(256) void conv_bands_y_kernel(int nk, int norb, int nvec, int parts,
                                                            const cx_t<R>* __restrict__ Vt,
                                                            const double* __restrict__ eval_k,
@@ -361,9 +365,13 @@ __global__ __launch_bounds__(256) void conv_bands_y_kernel(int nk, int norb, int
                                                            const cx_t<R>* __restrict__ T,
                                                            const double2* __restrict__ X, int64_t N,
                                                            double2* __restrict__ Y) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    constexpr int KB = 256 / S;
+    __shared__ cx_t<R> sums[S > 1 ? S : 1][NV][S > 1 ? KB : 1];
+    const int share = threadIdx.x / KB;
+    const int k = blockIdx.x * KB + threadIdx.x % KB;
     const int n = blockIdx.y;
-    if (k >= nk) return;
+    const bool ok = k < nk;
+    if (S == 1 && !ok) return;
     constexpr int nb = NV + NC, ncv = NC * NV;
     cx_t<R> acc[NC][NV];
 #pragma unroll
@@ -372,28 +380,45 @@ __global__ __launch_bounds__(256) void conv_bands_y_kernel(int nk, int norb, int
         for (int v = 0; v < NV; ++v) acc[c][v] = mk(R(0), R(0));
     const size_t part_stride = static_cast<size_t>(nvec) * NC * norb * nk;
     const cx_t<R>* tn = T + static_cast<size_t>(n) * NC * norb * nk + k;
-    for (int be = 0; be < norb; ++be) {
-        cx_t<R> vb[NV];
+    for (int be = share; ok && be < norb; be += S) {
+        cx_t<R> vb[NV], t[NC];
 #pragma unroll
         for (int v = 0; v < NV; ++v) vb[v] = Vt[(static_cast<size_t>(v) * norb + be) * nk + k];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const cx_t<R>* tc = tn + (static_cast<size_t>(c) * norb + be) * nk;
-            cx_t<R> t = tc[0];
-            for (int q = 1; q < parts; ++q) t = cadd(t, tc[q * part_stride]);
+        for (int c = 0; c < NC; ++c) t[c] = tn[(static_cast<size_t>(c) * norb + be) * nk];
+#pragma unroll 4
+        for (int q = 1; q < parts; ++q)
 #pragma unroll
-            for (int v = 0; v < NV; ++v) cfma(acc[c][v], vb[v], t);
+            for (int c = 0; c < NC; ++c) t[c] = cadd(t[c], tn[q * part_stride + (static_cast<size_t>(c) * norb + be) * nk]);
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) cfma(acc[c][v], vb[v], t[c]);
+    }
+    auto store = [&](int c, int v, cx_t<R> sum) {
+        const int64_t row = static_cast<int64_t>(k) * ncv + c * NV + v;
+        const double e = (scissor + eval_kq[static_cast<size_t>(k) * nb + NV + c]) - eval_k[static_cast<size_t>(k) * nb + v];
+        const double2 x = X[row + n * N];
+        Y[row + n * N] = mk(e * x.x - static_cast<double>(sum.x), e * x.y - static_cast<double>(sum.y));
+    };
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if (S == 1) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) store(c, v, acc[c][v]);
+        } else {
+            if (c > 0) __syncthreads();
+#pragma unroll
+            for (int v = 0; v < NV; ++v) sums[share][v][threadIdx.x % KB] = acc[c][v];
+            __syncthreads();
+            if (ok && share < NV) {
+                cx_t<R> sum = sums[0][share][threadIdx.x % KB];
+#pragma unroll
+                for (int q = 1; q < S; ++q) sum = cadd(sum, sums[q][share][threadIdx.x % KB]);
+                store(c, share, sum);
+            }
         }
     }
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const int64_t row = static_cast<int64_t>(k) * ncv + c * NV + v;
-            const double e = (scissor + eval_kq[static_cast<size_t>(k) * nb + NV + c]) - eval_k[static_cast<size_t>(k) * nb + v];
-            const double2 x = X[row + n * N];
-            Y[row + n * N] = mk(e * x.x - static_cast<double>(acc[c][v].x), e * x.y - static_cast<double>(acc[c][v].y));
-        }
 }
 
 // Launch the contraction kernels for the context's band counts (nc, nv in 1..4).
@@ -982,8 +1007,14 @@ void conv_rows_product(Context& c, ConvState& cs, ConvBuffers<R>& b, const doubl
     launch_rows_out<R>(a, c.nc, parts, cs.d_kmap.p, c.d_twiddle.p, b.Ct, b.G.p, b.T.p, s);
     with_bands<R>(c, [&](auto ncc, auto nvc) {
         constexpr int NC = decltype(ncc)::value, NV = decltype(nvc)::value;
-        hipLaunchKernelGGL((conv_bands_y_kernel<R, NC, NV>), dim3((c.nk + 255) / 256, nv), dim3(256), 0, s, c.nk,
-                           c.lat.norb, nv, parts, b.Vt, c.d_eval_k.p, c.d_eval_kq.p, c.scissor, b.T.p, X, c.N, Y);
+        // shared k-points while they leave CUs without a workgroup otherwise
+        if (static_cast<int64_t>(c.nk) * nv <= 65536)
+            hipLaunchKernelGGL((conv_bands_y_kernel<R, NC, NV, kBandsShare>), dim3((c.nk * kBandsShare + 255) / 256, nv),
+                               dim3(256), 0, s, c.nk, c.lat.norb, nv, parts, b.Vt, c.d_eval_k.p, c.d_eval_kq.p,
+                               c.scissor, b.T.p, X, c.N, Y);
+        else
+            hipLaunchKernelGGL((conv_bands_y_kernel<R, NC, NV, 1>), dim3((c.nk + 255) / 256, nv), dim3(256), 0, s, c.nk,
+                               c.lat.norb, nv, parts, b.Vt, c.d_eval_k.p, c.d_eval_kq.p, c.scissor, b.T.p, X, c.N, Y);
     });
     XATU_HIP(hipGetLastError());
 }

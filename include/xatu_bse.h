@@ -114,9 +114,9 @@ typedef struct xatu_solve_report {
     int converged;           /* 1 if every wanted residual met tol */
     double max_residual;     /* FP64 residual ||H x - e x|| max over the wanted states */
     double ms_total;         /* wall time of the solve (ms) */
-    double ms_products;      /* time in the matrix-vector products (ms, HIP events) */
-    double ms_rayleigh_ritz; /* time in the host Rayleigh-Ritz eigenproblems (ms) */
-    double ms_projections;   /* time in the basis projections and Ritz-vector products (ms, HIP events) */
+    double ms_products;      /* time in the matrix-vector products (ms, device clock or HIP events) */
+    double ms_rayleigh_ritz; /* time in the Rayleigh-Ritz eigenproblems (ms) */
+    double ms_projections;   /* time in the basis projections and Ritz-vector products (ms, device clock or HIP events) */
 } xatu_solve_report;
 
 typedef struct xatu_timings {

@@ -35,6 +35,7 @@ DEVICE_SOURCES = [
     "device/assemble.hip",
     "device/matvec.hip",
     "device/vec_kernels.hip",
+    "device/solver_step.hip",
     "device/hf.hip",
     "device/band_adjoint.hip",
     "device/convolution.hip",

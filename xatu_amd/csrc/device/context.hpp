@@ -107,11 +107,16 @@ struct HostBuf {
 // block X, AX, residuals R, scratch block Tb (N x b), projections P, Ritz coefficients Y
 // (mmax x b), Ritz values theta (b), residual partial sums, the projected matrix Tm (mmax x
 // mmax) and its reflectors (device Rayleigh-Ritz). Held by the context between solves.
+struct StepReport;  // solver_step.hpp
 struct SolverWorkspace {
     DevBuf<double2> V, W, X, AX, R, Tb;
     DevBuf<double2> P, Y;
     DevBuf<double> theta, partial;
     DevBuf<double2> Tm, refl;
+    DevBuf<double2> S;                    // whitening of a correction block
+    DevBuf<double> norm2;
+    DevBuf<int> flag;
+    DevBuf<unsigned long long> stamps;    // device clock of the iteration's phases
 };
 
 // Geometry and lattice-sum description shared with the kernels (by value).
@@ -234,7 +239,8 @@ struct Context {
     // Ritz coefficients and values, residual partial sums, block whitening coefficients
     HostBuf<double2> h_proj, h_coef, h_whiten;
     HostBuf<double> h_theta, h_part;
-    HostBuf<double> h_gather;  // mapped: the per-iteration results of the device solver
+    HostBuf<StepReport> h_step;  // mapped: the per-iteration results of the device solver
+    unsigned long long step_sequence = 0;  // of the last report asked for
     // solver workspaces, kept (grow only) between solves: [0] the FP64 solve or refinement,
     // [1] the FP32 phase of the mixed form, which both exist during a mixed solve
     SolverWorkspace solver_ws[2];

@@ -8,7 +8,7 @@
 // products H V use the FP64 or the FP32 matrix (or the matrix-free product);
 // the projected matrix V^H W is formed incrementally (Gram kernel, FP64) and
 // diagonalised on the device (Rayleigh-Ritz, projected_eigen.hip; on the host for
-// bases above 128 or blocks above 64); corrections use the diagonal
+// bases above 128 or blocks above 32); corrections use the diagonal
 // preconditioner r / (theta - diag H), are orthogonalised twice against V
 // (classical Gram-Schmidt, FP64) and orthonormalised by an eigen-decomposition
 // of their Gram matrix, dropping dependent directions; the block products with the
@@ -18,10 +18,10 @@
 // entries (the reference uses the first 2*nstates unit vectors, :19), no dense
 // (M - theta I) is ever formed (:37), and convergence is on residual norms
 // rather than on the change of the eigenvalues (:43).
-// With the device Rayleigh-Ritz an iteration synchronises with the host once: the
-// residual norms, the Ritz values and the correction block's Gram matrix arrive together
-// (the corrections are formed before the convergence test; the block is whitened on the
-// host, a 32 x 32 eigenproblem).
+// With the device Rayleigh-Ritz an iteration waits for the host once: the corrections are
+// formed, orthogonalised and whitened on the device (solver_step.hip; by a Cholesky
+// factorisation, an ill-conditioned block by the host) before the convergence test, and
+// the residual norms and the Ritz values arrive meanwhile.
 // The FP32 form runs this loop with FP32 products to a loose tolerance and then
 // refines in FP64: it restarts from the FP32 Ritz block and iterates with FP64
 // products until the FP64 residuals meet the tolerance.
@@ -32,10 +32,12 @@
 #include <memory>
 #include <cmath>
 #include <complex>
+#include <cstring>
 #include <numeric>
 
 #include "../common/heev.hpp"
 #include "context.hpp"
+#include "solver_step.hpp"
 
 namespace xatu_dev {
 
@@ -45,15 +47,11 @@ void launch_precondition(const double2* R, const double* theta, const double* di
                          hipStream_t s);
 void launch_unit_vectors(const int* idx, int64_t N, int nvec, double2* V, hipStream_t s);
 void launch_copy_vectors(const double2* src, int64_t n, double2* dst, hipStream_t s);
-void launch_gather3(const double* a, int na, const double* b, int nb, const double* c, int nc, double* dst,
-                    hipStream_t s);
 int projected_eigen_max_dim();
 int projected_eigen_max_want();
 // fp32_reduction: the Householder reduction in FP32 (the FP32 phase of the mixed form)
 void launch_projected_eigen(const double2* T, int ldt, int m, int nwant, double2* refl, double* theta, double2* Y,
-                            int ldy, bool fp32_reduction, hipStream_t s);
-void launch_extend_projected(const double2* P, int m0, int nb, double2* T, int ldt, hipStream_t s);
-void launch_restart_projected(double2* T, int ld, const double* theta, int nb, hipStream_t s);
+                            int ldy, bool fp32_reduction, unsigned long long* stamp, hipStream_t s);
 
 namespace {
 
@@ -82,25 +80,34 @@ public:
         ws_.W.reserve(static_cast<size_t>(N_) * mmax_);
         ws_.X.reserve(static_cast<size_t>(N_) * b_);
         ws_.AX.reserve(static_cast<size_t>(N_) * b_);
-        ws_.R.reserve(static_cast<size_t>(N_) * b_);
-        ws_.Tb.reserve(static_cast<size_t>(N_) * b_);
         ws_.P.reserve(static_cast<size_t>(mmax_) * b_);
         ws_.Y.reserve(static_cast<size_t>(mmax_) * b_);
         ws_.theta.reserve(b_);
-        ws_.partial.reserve(static_cast<size_t>(b_) * ((N_ + 255) / 256));
         T_.assign(static_cast<size_t>(mmax_) * mmax_, cd(0.0, 0.0));
         c_.h_proj.reserve(static_cast<size_t>(mmax_) * b_);
         c_.h_coef.reserve(static_cast<size_t>(mmax_) * b_);
         c_.h_whiten.reserve_mapped(static_cast<size_t>(b_) * b_);
         c_.h_theta.reserve(b_);
-        c_.h_part.reserve(static_cast<size_t>(b_) * ((N_ + 255) / 256));
-        c_.h_gather.reserve_mapped(2 * static_cast<size_t>(mmax_) * b_ + static_cast<size_t>(b_) * ((N_ + 255) / 256) + b_);
         dev_rr_ = mmax_ <= projected_eigen_max_dim() && b_ <= projected_eigen_max_want();
         if (dev_rr_) {
             const int md = projected_eigen_max_dim();
             ws_.Tm.reserve(static_cast<size_t>(mmax_) * mmax_);
             ws_.refl.reserve(static_cast<size_t>(md) * md);
-            XATU_HIP(hipMemsetAsync(ws_.Tm.p, 0, ws_.Tm.bytes(), c_.stream));
+            ws_.partial.reserve(static_cast<size_t>(b_) * ritz_block_partials(N_));
+            ws_.S.reserve(static_cast<size_t>(b_) * b_);
+            ws_.norm2.reserve(b_);
+            ws_.flag.reserve(1);
+            ws_.stamps.reserve(kStamps);
+            c_.h_step.reserve_mapped(1);
+            // fresh memory may hold the report of a context that is gone; sequence numbers only grow
+            std::fill_n(c_.h_step.p->entry, kReportEntries, make_ulonglong2(0, 0));
+            int khz = 0;
+            XATU_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c_.device));
+            tick_ms_ = 1.0 / khz;
+        } else {
+            ws_.R.reserve(static_cast<size_t>(N_) * b_);
+            ws_.partial.reserve(static_cast<size_t>(b_) * ((N_ + 255) / 256));
+            c_.h_part.reserve(static_cast<size_t>(b_) * ((N_ + 255) / 256));
         }
     }
 
@@ -119,6 +126,7 @@ public:
         XATU_HIP(hipMemsetAsync(ws_.V.p, 0, static_cast<size_t>(N_) * b_ * sizeof(double2), c_.stream));
         launch_unit_vectors(d_idx.p, N_, b_, ws_.V.p, c_.stream);
         m_ = 0;
+        if (dev_rr_) launch_stamp(ws_.stamps.p + kStampProduct, c_.stream);
         append_block(b_);
         XATU_HIP(hipStreamSynchronize(c_.stream));
     }
@@ -131,6 +139,7 @@ public:
         m_ = 0;
         const int kept = orthonormalise_slot(b_);
         if (kept < b_) throw Error(XATU_ERR_NOT_CONVERGED, "Davidson: the refinement's starting block is rank deficient");
+        if (dev_rr_) launch_stamp(ws_.stamps.p + kStampProduct, c_.stream);
         append_block(b_);
     }
 
@@ -164,102 +173,133 @@ public:
     double projections_ms() const { return proj_ms_; }
 
 private:
-    // Event pairs read after the next synchronisation (reading them adds no wait).
-    struct Pending {
-        std::unique_ptr<EventTimer> ev;
-        int kind;  // 0 product (nvec), 1 projection, 2 Rayleigh-Ritz
-        int nvec;
-    };
-    EventTimer* timer(int kind, int nvec = 0) {
-        pending_.push_back({std::make_unique<EventTimer>(c_.stream), kind, nvec});
-        return pending_.back().ev.get();
-    }
-    // Reads the event pairs; with completed_only, only those already complete (the others
-    // stay pending), so that it can run while the device works.
-    void drain_timers(bool completed_only = false) {
-        std::vector<Pending> later;
-        for (Pending& p : pending_) {
-            if (completed_only && hipEventQuery(p.ev->b) != hipSuccess) {
-                later.push_back(std::move(p));
-                continue;
-            }
-            const double ms = p.ev->ms();
-            if (p.kind == 0) {
-                prod_ms_ += ms;
-                record_product(c_, mf_, ms, p.nvec);
-            } else if (p.kind == 1) {
-                proj_ms_ += ms;
-            } else {
-                rr_ms_ += ms;
-            }
-        }
-        pending_ = std::move(later);
-    }
-
-    // One iteration per synchronisation: Rayleigh-Ritz on the device, Ritz block and
-    // residuals, restart when the basis is full, preconditioned corrections and their
-    // Gram matrix against the basis; then residual norms, Ritz values and the Gram matrix
-    // to the host together.
+    // One wait per iteration: Rayleigh-Ritz on the device, Ritz block, residuals,
+    // preconditioned corrections (restart when the basis is full), their orthogonalisation and
+    // whitening; the residual norms, the Ritz values and the times of the phases arrive from the
+    // whitening kernel while the whitening is applied.
     bool run_device(double tol, int maxit) {
         const int n = static_cast<int>(N_);
         for (int it = 0; it < maxit; ++it) {
-            EventTimer* er = timer(2);
-            er->start();
             launch_projected_eigen(ws_.Tm.p, mmax_, m_, b_, ws_.refl.p, ws_.theta.p, ws_.Y.p, m_, prec_ == XATU_FP32,
-                                   c_.stream);
-            er->stop();
-            EventTimer* ep = timer(1);
-            ep->start();
-            launch_block_gemm(ws_.V.p, n, ws_.Y.p, m_, N_, m_, b_, 1.0, 0.0, ws_.X.p, n, c_.stream);
-            launch_block_gemm(ws_.W.p, n, ws_.Y.p, m_, N_, m_, b_, 1.0, 0.0, ws_.AX.p, n, c_.stream);
-            ep->stop();
-            int nblk = 0;
-            launch_residual(ws_.X.p, ws_.AX.p, ws_.theta.p, N_, b_, ws_.R.p, ws_.partial.p, &nblk, c_.stream);
+                                   ws_.stamps.p + kStampEigen, c_.stream);
             rep_->iterations++;
-            if (m_ + b_ > mmax_) {
-                launch_copy_vectors(ws_.X.p, static_cast<int64_t>(N_) * b_, ws_.V.p, c_.stream);
-                launch_copy_vectors(ws_.AX.p, static_cast<int64_t>(N_) * b_, ws_.W.p, c_.stream);
-                launch_restart_projected(ws_.Tm.p, mmax_, ws_.theta.p, b_, c_.stream);
+            RitzBlockArgs a{};
+            a.V = ws_.V.p;
+            a.W = ws_.W.p;
+            a.Y = ws_.Y.p;
+            a.theta = ws_.theta.p;
+            a.diag = c_.d_diag.p;
+            a.N = N_;
+            a.m = m_;
+            a.b = b_;
+            a.restart = m_ + b_ > mmax_;
+            if (a.restart) {
                 m_ = b_;
                 rep_->restarts++;
             }
-            const int nb = std::min(b_, mmax_ - m_);
-            const int np = nb > 0 ? 2 * (m_ + nb) * nb : 0;  // doubles of the block's Gram rows
+            const int nb = std::min(b_, mmax_ - m_), mn = m_ + nb;
+            double2* T = ws_.V.p + static_cast<size_t>(m_) * N_;
+            a.nb = nb;
+            a.X = ws_.X.p;
+            a.AX = ws_.AX.p;
+            a.T = T;
+            a.partial = ws_.partial.p;
+            a.Tm = ws_.Tm.p;
+            a.ldt = mmax_;
+            a.stamps = ws_.stamps.p;
+            launch_ritz_block(a, c_.stream);
             if (nb > 0) {
-                launch_precondition(ws_.R.p, ws_.theta.p, c_.d_diag.p, N_, nb, ws_.V.p + static_cast<size_t>(m_) * N_,
-                                    c_.stream);
-                ortho_gram(nb);
+                launch_gram(c_, ws_.V.p, n, T, n, mn, nb, ws_.P.p, mn, c_.stream);
+                launch_block_gemm(ws_.V.p, n, ws_.P.p, mn, N_, m_, nb, -1.0, 1.0, T, n, c_.stream);
             }
-            // Gram rows, residual partial sums and Ritz values stored into mapped host memory by
-            // one kernel (three device-to-host copies each waited tens of microseconds here)
-            launch_gather3(reinterpret_cast<const double*>(ws_.P.p), np, ws_.partial.p, nblk * b_, ws_.theta.p, b_,
-                           c_.h_gather.dev, c_.stream);
-            XATU_HIP(hipStreamSynchronize(c_.stream));
-            const double* got = c_.h_gather.p;
-            theta_.assign(got + np + nblk * b_, got + np + nblk * b_ + b_);
-            residual_norms(nblk, got + np);
+            launch_gram_norms(c_, ws_.V.p, n, T, n, mn, nb, ws_.P.p, mn, ws_.partial.p, ritz_block_partials(N_), b_,
+                              ws_.norm2.p, c_.stream);
+            if (nb > 0) launch_block_gemm(ws_.V.p, n, ws_.P.p, mn, N_, m_, nb, -1.0, 1.0, T, n, c_.stream);
+            WhitenArgs w{};
+            w.P = ws_.P.p + m_;
+            w.ldp = mn;
+            w.nb = nb;
+            w.b = b_;
+            w.T = T;
+            w.N = N_;
+            w.S = ws_.S.p;
+            w.flag = ws_.flag.p;
+            w.theta = ws_.theta.p;
+            w.norm2 = ws_.norm2.p;
+            w.stamps = ws_.stamps.p;
+            w.product_stamp = ws_.stamps.p + kStampProduct;
+            w.host = c_.h_step.dev;
+            w.sequence = ++c_.step_sequence;
+            launch_whiten(w, c_.stream);
+            unsigned long long got[kReportEntries];
+            wait_report(got);
+            theta_.resize(b_);
+            res_.resize(b_);
+            std::memcpy(theta_.data(), got, b_ * sizeof(double));
+            std::memcpy(res_.data(), got + kStepMaxBlock, b_ * sizeof(double));
+            for (double& r : res_) r = std::sqrt(r);
+            add_times(got + 2 * kStepMaxBlock, true);
             double worst = 0.0;
             for (int i = 0; i < nev_; ++i) worst = std::max(worst, res_[i]);
             last_worst_ = worst;
-            if (worst < tol || nb <= 0) {
-                drain_timers();
-                return worst < tol;
-            }
-            const int kept = ortho_whiten(nb, 0, reinterpret_cast<const cd*>(got));
-            if (kept == 0) {
-                drain_timers();
-                return false;
+            if (worst < tol) return true;
+            if (nb <= 0) return false;
+            int kept = nb;
+            if (!got[2 * kStepMaxBlock + kStamps]) {
+                XATU_HIP(hipMemcpyAsync(c_.h_proj.p, ws_.P.p, static_cast<size_t>(mn) * nb * sizeof(cd),
+                                        hipMemcpyDeviceToHost, c_.stream));
+                XATU_HIP(hipStreamSynchronize(c_.stream));
+                kept = ortho_whiten(nb, 0);
+                if (kept == 0) return false;
+                launch_stamp(ws_.stamps.p + kStampProduct, c_.stream);
             }
             append_block(kept);
-            drain_timers(true);  // the timings of this iteration, while the next one runs
         }
-        drain_timers();
+        unsigned long long last[kStamps];
+        XATU_HIP(hipMemcpyAsync(last, ws_.stamps.p, sizeof(last), hipMemcpyDeviceToHost, c_.stream));
+        XATU_HIP(hipStreamSynchronize(c_.stream));
+        add_times(last, false);
         return false;
     }
 
-    // part: the residual kernel's per-block partial sums on the host (nblk x b_)
-    void residual_norms(int nblk, const double* part = nullptr) {
-        if (!part) part = c_.h_part.p;
+    // Waits for the report of this iteration: its values in mapped memory, seen some microseconds
+    // before the stream's end would be; after a while for the stream itself.
+    void wait_report(unsigned long long* got) {
+        const ulonglong2* e = c_.h_step.p->entry;
+        auto arrived = [&](int i) {
+            got[i] = __atomic_load_n(&e[i].x, __ATOMIC_ACQUIRE);
+            return (__atomic_load_n(&e[i].y, __ATOMIC_ACQUIRE) ^ c_.step_sequence) == got[i];
+        };
+        int n = 0;
+        for (int spin = 0; spin < 100000 && n < kReportEntries; ++spin) {
+            while (n < kReportEntries && arrived(n)) ++n;
+            __builtin_ia32_pause();
+        }
+        if (n == kReportEntries) return;
+        XATU_HIP(hipStreamSynchronize(c_.stream));
+        for (n = 0; n < kReportEntries; ++n)
+            if (!arrived(n)) throw Error(XATU_ERR_DEVICE, "Davidson: the iteration's report did not arrive");
+    }
+
+    // Times of an iteration from the device's clock: the product and the projections after
+    // the previous one, and (whole) this one's Rayleigh-Ritz and block work.
+    void add_times(const unsigned long long* t, bool whole) {
+        auto ms = [&](int from, int to) { return t[to] > t[from] ? (t[to] - t[from]) * tick_ms_ : 0.0; };
+        if (last_nb_ > 0) {
+            const double p = ms(kStampProduct, kStampExtend);
+            prod_ms_ += p;
+            record_product(c_, mf_, p, last_nb_);
+            last_nb_ = 0;
+        }
+        if (whole) {
+            proj_ms_ += ms(kStampExtend, kStampEigen) + ms(kStampRitz, kStampWhiten);
+            rr_ms_ += ms(kStampEigen, kStampRitz);
+        }
+    }
+
+    // from the residual kernel's per-block partial sums on the host (nblk x b_)
+    void residual_norms(int nblk) {
+        const double* part = c_.h_part.p;
         res_.assign(b_, 0.0);
         for (int j = 0; j < b_; ++j) {
             double s = 0.0;
@@ -273,18 +313,11 @@ private:
         double2* Vn = ws_.V.p + static_cast<size_t>(m_) * N_;
         double2* Wn = ws_.W.p + static_cast<size_t>(m_) * N_;
         if (dev_rr_) {
-            EventTimer* ev = timer(0, nb);
-            ev->start();
             launch_operator(c_, prec_, mf_, Vn, Wn, nb);
-            ev->stop();
             rep_->products += nb;
-            const int mn = m_ + nb;
-            EventTimer* eg = timer(1);
-            eg->start();
-            launch_gram(c_, ws_.V.p, static_cast<int>(N_), Wn, static_cast<int>(N_), mn, nb, ws_.P.p, mn, c_.stream);
-            eg->stop();
-            launch_extend_projected(ws_.P.p, m_, nb, ws_.Tm.p, mmax_, c_.stream);
-            m_ = mn;
+            launch_gram_extend(c_, ws_.V.p, Wn, N_, m_, nb, ws_.Tm.p, mmax_, ws_.stamps.p, c_.stream);
+            last_nb_ = nb;
+            m_ += nb;
             return;
         }
         // event pairs are read after the synchronisation below, so that timing adds no waits
@@ -375,37 +408,32 @@ private:
     // dropping dependent directions. An ill-conditioned block (kept eigenvalues spanning
     // more than 1e8) repeats the whole procedure once on the whitened vectors.
     int orthonormalise_slot(int nb, int round = 0) {
-        ortho_gram(nb);
-        XATU_HIP(hipMemcpyAsync(c_.h_proj.p, ws_.P.p, static_cast<size_t>(m_ + nb) * nb * sizeof(cd),
-                                hipMemcpyDeviceToHost, c_.stream));
-        XATU_HIP(hipStreamSynchronize(c_.stream));
-        drain_timers();
-        return ortho_whiten(nb, round);
-    }
-
-    // The device part: two classical Gram-Schmidt passes; P = [V, T]^H T of the second.
-    void ortho_gram(int nb) {
         const int n = static_cast<int>(N_);
         const int mn = m_ + nb;
         double2* T = ws_.V.p + static_cast<size_t>(m_) * N_;
-        EventTimer* ev = timer(1);
-        ev->start();
+        EventTimer ev(c_.stream);
+        ev.start();
         for (int pass = 0; pass < 2; ++pass) {
             launch_gram(c_, ws_.V.p, n, T, n, mn, nb, ws_.P.p, mn, c_.stream);
             if (m_ > 0) {
                 launch_block_gemm(ws_.V.p, n, ws_.P.p, mn, N_, m_, nb, -1.0, 1.0, T, n, c_.stream);
             }
         }
-        ev->stop();
+        ev.stop();
+        XATU_HIP(hipMemcpyAsync(c_.h_proj.p, ws_.P.p, static_cast<size_t>(mn) * nb * sizeof(cd), hipMemcpyDeviceToHost,
+                                c_.stream));
+        XATU_HIP(hipStreamSynchronize(c_.stream));
+        proj_ms_ += ev.ms();
+        return ortho_whiten(nb, round);
     }
 
-    // The host part, with P on the host (Ph, else the pinned copy): whiten the block (its Gram
-    // matrix rows m..m+nb).
-    int ortho_whiten(int nb, int round, const cd* Ph = nullptr) {
+    // The host part, with P on the host: whiten the block (its Gram matrix rows m..m+nb).
+    int ortho_whiten(int nb, int round) {
         const int n = static_cast<int>(N_);
         const int mn = m_ + nb;
         double2* T = ws_.V.p + static_cast<size_t>(m_) * N_;
-        const cd* P = Ph ? Ph : reinterpret_cast<const cd*>(c_.h_proj.p);
+        const cd* P = reinterpret_cast<const cd*>(c_.h_proj.p);
+        ws_.Tb.reserve(static_cast<size_t>(N_) * nb);
         // column-normalised Gram matrix of the block
         std::vector<cd> G(static_cast<size_t>(nb) * nb);
         std::vector<double> dsc(nb);
@@ -496,10 +524,11 @@ private:
     int prec_, mf_, nev_, b_, mmax_;
     Workspace& ws_;  // the context's: kept between solves
     bool dev_rr_ = false;
-    std::vector<Pending> pending_;
     xatu_solve_report* rep_;
     int64_t N_ = 0;
     int m_ = 0;
+    int last_nb_ = 0;       // columns of the last product whose time has not been read
+    double tick_ms_ = 0.0;  // of the device clock
     std::vector<cd> T_;
     std::vector<double> theta_, res_;
     double prod_ms_ = 0.0, rr_ms_ = 0.0, proj_ms_ = 0.0, last_worst_ = 0.0;

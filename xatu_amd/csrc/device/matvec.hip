@@ -18,6 +18,7 @@
 #include "context.hpp"
 #include "cplx.hpp"
 #include "mfma.hpp"
+#include "solver_step.hpp"
 
 namespace xatu_dev {
 
@@ -290,7 +291,9 @@ constexpr int kGM = 64, kGN = 32, kGR = 16;
 
 __global__ __launch_bounds__(256) void gram_partial_kernel(const double2* __restrict__ A, int lda,
                                                            const double2* __restrict__ B, int ldb, int64_t N, int m,
-                                                           int n, int64_t rows_per_chunk, double2* __restrict__ P) {
+                                                           int n, int64_t rows_per_chunk, double2* __restrict__ P,
+                                                           unsigned long long* __restrict__ stamp) {
+    if (stamp && blockIdx.x + blockIdx.y + blockIdx.z == 0 && threadIdx.x == 0) *stamp = wall_clock64();
     __shared__ double2 sA[kGR][kGM + 1];
     __shared__ double2 sB[kGR][kGN + 1];
     const int tm = threadIdx.x % 16, tn = threadIdx.x / 16;
@@ -357,36 +360,100 @@ __global__ __launch_bounds__(256) void gram_partial_kernel(const double2* __rest
         }
 }
 
-// C[i + j ldc] = sum over chunks of P[chunk][i + j m]. One workgroup of 1024 threads
-// per 64 outputs: 16 slices each sum every 16th chunk, then the slices are added in
-// a fixed order, so the result does not depend on scheduling.
+// Sums over the chunks of P[chunk][i + j m], one workgroup of 1024 threads per 64 outputs: 16
+// slices each sum every 16th chunk, then the slices are added in a fixed order, so the
+// result does not depend on scheduling. What becomes of the sums (both fused kinds save a
+// launch of the solver's iteration):
+//   kGramPlain   C[i + j ldc]
+//   kGramNorms   the same, and the workgroups after the outputs each sum a column of residual partials
+//   kGramExtend  rows and columns m0 .. m0 + n of the Hermitian matrix C = V^H W (m = m0 + n); its
+//                diagonal block is symmetrised, so its threads sum the mirrored entry too
 constexpr int kRedOut = 64, kRedSlices = 16;
+enum { kGramPlain, kGramNorms, kGramExtend };
+template <int KIND>
 __global__ __launch_bounds__(kRedOut* kRedSlices) void gram_reduce_kernel(const double2* __restrict__ P, int m, int n,
-                                                                          int chunks, double2* __restrict__ C,
-                                                                          int ldc) {
+                                                                          int chunks, double2* __restrict__ C, int ldc,
+                                                                          const double* __restrict__ partial,
+                                                                          int npartial, double* __restrict__ norm2) {
     __shared__ double2 part[kRedSlices][kRedOut];
     const int o = threadIdx.x % kRedOut, sl = threadIdx.x / kRedOut;
-    const int idx = blockIdx.x * kRedOut + o;
     const int64_t mn = static_cast<int64_t>(m) * n;
-    double sr = 0.0, si = 0.0;
-    if (idx < mn) {
+    if (KIND == kGramNorms) {
+        const int outs = static_cast<int>((mn + kRedOut - 1) / kRedOut);
+        if (static_cast<int>(blockIdx.x) >= outs) {
+            double* red = &part[0][0].x;
+            const int j = blockIdx.x - outs;
+            double v = 0.0;
+            for (int i = threadIdx.x; i < npartial; i += kRedOut * kRedSlices) v += partial[static_cast<int64_t>(j) * npartial + i];
+            red[threadIdx.x] = v;
+            __syncthreads();
+            for (int st = kRedOut * kRedSlices / 2; st > 0; st >>= 1) {
+                if (static_cast<int>(threadIdx.x) < st) red[threadIdx.x] += red[threadIdx.x + st];
+                __syncthreads();
+            }
+            if (threadIdx.x == 0) norm2[j] = red[0];
+            return;
+        }
+    }
+    auto chunk_sum = [&](int64_t idx) {
+        double sr = 0.0, si = 0.0;
 #pragma unroll 4
         for (int c = sl; c < chunks; c += kRedSlices) {
             const double2 v = P[static_cast<int64_t>(c) * mn + idx];
             sr += v.x;
             si += v.y;
         }
-    }
-    part[sl][o] = mk(sr, si);
+        return mk(sr, si);
+    };
+    auto slice_sum = [&]() {
+        double2 v = part[0][o];
+        for (int k = 1; k < kRedSlices; ++k) v = cadd(v, part[k][o]);
+        return v;
+    };
+    const int64_t idx = static_cast<int64_t>(blockIdx.x) * kRedOut + o;
+    const int i = static_cast<int>(idx % m), j = static_cast<int>(idx / m);
+    part[sl][o] = idx < mn ? chunk_sum(idx) : mk(0.0, 0.0);
     __syncthreads();
-    if (sl == 0 && idx < mn) {
-        for (int k = 1; k < kRedSlices; ++k) {
-            sr += part[k][o].x;
-            si += part[k][o].y;
-        }
-        const int i = idx % m, j = idx / m;
-        C[i + static_cast<int64_t>(j) * ldc] = mk(sr, si);
+    if (KIND != kGramExtend) {
+        if (sl == 0 && idx < mn) C[i + static_cast<int64_t>(j) * ldc] = slice_sum();
+        return;
     }
+    const int m0 = m - n;
+    const double2 v = slice_sum();
+    __syncthreads();
+    const bool mirrored = idx < mn && i >= m0;
+    part[sl][o] = mirrored ? chunk_sum((m0 + j) + static_cast<int64_t>(i - m0) * m) : mk(0.0, 0.0);
+    __syncthreads();
+    if (sl != 0 || idx >= mn) return;
+    if (mirrored) {
+        const double2 w = slice_sum();
+        C[i + static_cast<int64_t>(m0 + j) * ldc] = mk(0.5 * (v.x + w.x), i - m0 == j ? 0.0 : 0.5 * (v.y - w.y));
+    } else {
+        C[i + static_cast<int64_t>(m0 + j) * ldc] = v;
+        C[(m0 + j) + static_cast<int64_t>(i) * ldc] = cconj(v);
+    }
+}
+
+// Partial products of A^H B to c.s_gram; the number of row chunks.
+int gram_partials(Context& c, const double2* A, int lda, const double2* B, int ldb, int m, int n,
+                  unsigned long long* stamp, hipStream_t s) {
+    const int64_t N = c.N;
+    const int tiles = ((m + kGM - 1) / kGM) * ((n + kGN - 1) / kGN);
+    int chunks = std::max(1, std::min<int>(static_cast<int>((N + kGR - 1) / kGR), 512 / tiles));
+    int64_t rows = ((N + chunks - 1) / chunks + kGR - 1) / kGR * kGR;
+    chunks = static_cast<int>((N + rows - 1) / rows);
+    c.s_gram.alloc(std::max<size_t>(c.s_gram.n, static_cast<size_t>(chunks) * m * n));
+    hipLaunchKernelGGL(gram_partial_kernel, dim3((m + kGM - 1) / kGM, (n + kGN - 1) / kGN, chunks), dim3(256), 0, s, A,
+                       lda, B, ldb, N, m, n, rows, c.s_gram.p, stamp);
+    return chunks;
+}
+
+template <int KIND>
+void gram_reduce(const Context& c, int m, int n, int chunks, double2* C, int ldc, const double* partial, int npartial,
+                 int ncols, double* norm2, hipStream_t s) {
+    hipLaunchKernelGGL((gram_reduce_kernel<KIND>), dim3((m * n + kRedOut - 1) / kRedOut + ncols), dim3(kRedOut * kRedSlices),
+                       0, s, c.s_gram.p, m, n, chunks, C, ldc, partial, npartial, norm2);
+    XATU_HIP(hipGetLastError());
 }
 
 // Vectors per tile row of a product launch: one 16-vector matrix tile for up to 16 vectors.
@@ -532,17 +599,22 @@ void launch_block_gemm(const double2* A, int lda, const double2* B, int ldb, int
 
 void launch_gram(Context& c, const double2* A, int lda, const double2* B, int ldb, int m, int n, double2* C, int ldc,
                  hipStream_t s) {
-    const int64_t N = c.N;
-    const int tiles = ((m + kGM - 1) / kGM) * ((n + kGN - 1) / kGN);
-    int chunks = std::max(1, std::min<int>(static_cast<int>((N + kGR - 1) / kGR), 512 / tiles));
-    int64_t rows = ((N + chunks - 1) / chunks + kGR - 1) / kGR * kGR;
-    chunks = static_cast<int>((N + rows - 1) / rows);
-    c.s_gram.alloc(std::max<size_t>(c.s_gram.n, static_cast<size_t>(chunks) * m * n));
-    hipLaunchKernelGGL(gram_partial_kernel, dim3((m + kGM - 1) / kGM, (n + kGN - 1) / kGN, chunks), dim3(256), 0, s, A,
-                       lda, B, ldb, N, m, n, rows, c.s_gram.p);
-    hipLaunchKernelGGL(gram_reduce_kernel, dim3((m * n + kRedOut - 1) / kRedOut), dim3(kRedOut * kRedSlices), 0, s,
-                       c.s_gram.p, m, n, chunks, C, ldc);
-    XATU_HIP(hipGetLastError());
+    const int chunks = gram_partials(c, A, lda, B, ldb, m, n, nullptr, s);
+    gram_reduce<kGramPlain>(c, m, n, chunks, C, ldc, nullptr, 0, 0, nullptr, s);
+}
+
+void launch_gram_norms(Context& c, const double2* A, int lda, const double2* B, int ldb, int m, int n, double2* P, int ldp,
+                       const double* partial, int npartial, int ncols, double* norm2, hipStream_t s) {
+    const int chunks = n > 0 ? gram_partials(c, A, lda, B, ldb, m, n, nullptr, s) : 0;
+    gram_reduce<kGramNorms>(c, m, n, chunks, P, ldp, partial, npartial, ncols, norm2, s);
+}
+
+void launch_gram_extend(Context& c, const double2* V, const double2* W, int64_t N, int m0, int nb, double2* Tm, int ldt,
+                        unsigned long long* stamps, hipStream_t s) {
+    const int mn = m0 + nb;
+    if (nb <= 0 || mn > ldt) throw Error(XATU_ERR_INVALID_ARGUMENT, "projected matrix: block exceeds its size");
+    const int chunks = gram_partials(c, V, static_cast<int>(N), W, static_cast<int>(N), mn, nb, stamps + kStampExtend, s);
+    gram_reduce<kGramExtend>(c, mn, nb, chunks, Tm, ldt, nullptr, 0, 0, nullptr, s);
 }
 
 }  // namespace xatu_dev

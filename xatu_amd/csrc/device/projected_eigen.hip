@@ -459,7 +459,9 @@ template <typename TR>
 __global__ __launch_bounds__(kEThreads) void projected_eigen_kernel(const double2* __restrict__ A, int lda, int m,
                                                                     int nwant, cx_t<TR>* __restrict__ refl,
                                                                     double* __restrict__ theta,
-                                                                    double2* __restrict__ Y, int ldy) {
+                                                                    double2* __restrict__ Y, int ldy,
+                                                                    unsigned long long* __restrict__ stamp) {
+    if (threadIdx.x == 0) *stamp = wall_clock64();
     using CT = cx_t<TR>;
     // working accuracy of the tridiagonal: the eigenvalues are resolved to it (multisection
     // tolerance, shift separation, inverse-iteration growth test), not beyond
@@ -739,69 +741,22 @@ __global__ __launch_bounds__(kEThreads) void projected_eigen_kernel(const double
     else back_transform<TR, 8>(s, m, nwant, refl, theta, Y, ldy);
 }
 
-// T[i][j] for the new block columns j in [m0, m0 + nb) (and the mirrored rows) from
-// P = V[:, 0:m0+nb]^H W[:, m0:m0+nb] (ld mn = m0 + nb); the new diagonal block is
-// symmetrised, (P[m0+i, j] + conj(P[m0+j, i])) / 2, with a real diagonal.
-__global__ void extend_projected_kernel(const double2* __restrict__ P, int m0, int nb, double2* __restrict__ T,
-                                        int ldt) {
-    const int mn = m0 + nb;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    if (i >= mn) return;
-    if (i < m0) {
-        const double2 v = P[i + static_cast<size_t>(j) * mn];
-        T[i + static_cast<size_t>(m0 + j) * ldt] = v;
-        T[(m0 + j) + static_cast<size_t>(i) * ldt] = cconj(v);
-        return;
-    }
-    const int ii = i - m0;
-    if (ii > j) return;
-    const double2 pij = P[(m0 + ii) + static_cast<size_t>(j) * mn];
-    const double2 pji = P[(m0 + j) + static_cast<size_t>(ii) * mn];
-    double2 avg = make_double2(0.5 * (pij.x + pji.x), 0.5 * (pij.y - pji.y));
-    if (ii == j) avg.y = 0.0;
-    T[(m0 + ii) + static_cast<size_t>(m0 + j) * ldt] = avg;
-    T[(m0 + j) + static_cast<size_t>(m0 + ii) * ldt] = cconj(avg);
-}
-
-// T (ld x ld) = diag(theta[0..nb)), zero elsewhere.
-__global__ void restart_projected_kernel(double2* __restrict__ T, int ld, const double* __restrict__ theta, int nb) {
-    const int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (e >= static_cast<int64_t>(ld) * ld) return;
-    const int i = static_cast<int>(e % ld), j = static_cast<int>(e / ld);
-    T[e] = (i == j && i < nb) ? make_double2(theta[i], 0.0) : make_double2(0.0, 0.0);
-}
-
 }  // namespace
 
 int projected_eigen_max_dim() { return kEM; }
 int projected_eigen_max_want() { return kEWant; }
 
 void launch_projected_eigen(const double2* T, int ldt, int m, int nwant, double2* refl, double* theta, double2* Y,
-                            int ldy, bool fp32_reduction, hipStream_t s) {
+                            int ldy, bool fp32_reduction, unsigned long long* stamp, hipStream_t s) {
     if (m < 1 || m > kEM || nwant < 1 || nwant > kEWant || nwant > m || ldt < m || ldy < m)
         throw Error(XATU_ERR_INVALID_ARGUMENT, "projected eigensolver: unsupported dimensions");
     if (fp32_reduction) {
         hipLaunchKernelGGL(projected_eigen_kernel<float>, dim3(1), dim3(kEThreads), 0, s, T, ldt, m, nwant,
-                           reinterpret_cast<float2*>(refl), theta, Y, ldy);
+                           reinterpret_cast<float2*>(refl), theta, Y, ldy, stamp);
     } else {
         hipLaunchKernelGGL(projected_eigen_kernel<double>, dim3(1), dim3(kEThreads), 0, s, T, ldt, m, nwant, refl,
-                           theta, Y, ldy);
+                           theta, Y, ldy, stamp);
     }
-    XATU_HIP(hipGetLastError());
-}
-
-void launch_extend_projected(const double2* P, int m0, int nb, double2* T, int ldt, hipStream_t s) {
-    const int mn = m0 + nb;
-    if (nb <= 0 || mn > ldt) throw Error(XATU_ERR_INVALID_ARGUMENT, "projected matrix: block exceeds its size");
-    hipLaunchKernelGGL(extend_projected_kernel, dim3((mn + 127) / 128, nb), dim3(128), 0, s, P, m0, nb, T, ldt);
-    XATU_HIP(hipGetLastError());
-}
-
-void launch_restart_projected(double2* T, int ld, const double* theta, int nb, hipStream_t s) {
-    const int64_t n = static_cast<int64_t>(ld) * ld;
-    hipLaunchKernelGGL(restart_projected_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, T, ld,
-                       theta, nb);
     XATU_HIP(hipGetLastError());
 }
 

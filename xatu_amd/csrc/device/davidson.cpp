@@ -607,12 +607,19 @@ void solve_davidson(Context& c, const xatu_solve_options& opt, double* eigval_ou
         // with 2).
         d32->run(std::max(0.5 * tol, opt.matrix_free ? 2e-5 : 6e-4), maxit);
         const int it32 = rep->iterations;
-        // ... then FP64 refinement from the lowest nev Ritz vectors, with FP64 products
+        // ... then FP64 refinement from the lowest Ritz vectors, with FP64 products
         // (matrix-free when no FP64 matrix is resident), until the FP64 residuals meet tol.
-        // Block nev, basis 6 nev up to the device Rayleigh-Ritz limit (N = 36864, nev = 16:
-        // basis 96 took 7 refinement iterations against 8 with 64, 53.5 against 55.0 ms per
-        // step; 128 also 7, at 54.0 ms; blocks of 24 or 32 cost more per product than they save)
-        const int bref = nev;
+        // Block: nev and some guard vectors, because the highest state wanted converges with its
+        // distance from the first state outside the block, which may be next to nothing (a block
+        // of nev took 64 iterations, 99 ms, where four guard vectors took 14, 49 ms: N = 36864, nev
+        // = 16). Over N = 1875, 9216 and 36864, three spectra each, nev = 3, 4, 8, 16, guard max(4, nev / 4)
+        // against none: 0.49 to 1.08 of the time, 0.88 in the mean; the whole block, twice nev, costs more per
+        // product than it saves (53, 22 and 18 ms where a quarter took 49, 18 and 14). A resident FP64 matrix
+        // is multiplied by whole tiles of 16 vectors: the guard fills the last one. Basis 6 blocks up to the device
+        // Rayleigh-Ritz limit (4 blocks: up to 1.2 of the time).
+        const bool resident = !opt.matrix_free && c.built64;
+        const int guard = std::max(4, nev / 4);
+        const int bref = std::min({b, nev + guard, resident ? (nev + 15) / 16 * 16 : b});
         const int mref = static_cast<int>(std::min<int64_t>(
             N, std::max({4 * bref, std::min(6 * bref, projected_eigen_max_dim()), bref + 1})));
         dav = std::make_unique<Davidson>(c, c.solver_ws[0], XATU_FP64, opt.matrix_free ? opt.matrix_free : (c.built64 ? 0 : 1), nev, bref, mref, rep);

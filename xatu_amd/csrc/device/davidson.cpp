@@ -611,14 +611,15 @@ void solve_davidson(Context& c, const xatu_solve_options& opt, double* eigval_ou
         // (matrix-free when no FP64 matrix is resident), until the FP64 residuals meet tol.
         // Block: nev and some guard vectors, because the highest state wanted converges with its
         // distance from the first state outside the block, which may be next to nothing (a block
-        // of nev took 64 iterations, 99 ms, where four guard vectors took 14, 49 ms: N = 36864, nev
-        // = 16). Over N = 1875, 9216 and 36864, three spectra each, nev = 3, 4, 8, 16, guard max(4, nev / 4)
-        // against none: 0.49 to 1.08 of the time, 0.88 in the mean; the whole block, twice nev, costs more per
-        // product than it saves (53, 22 and 18 ms where a quarter took 49, 18 and 14). A resident FP64 matrix
-        // is multiplied by whole tiles of 16 vectors: the guard fills the last one. Basis 6 blocks up to the device
+        // of nev took 64 iterations, 99 ms, where two guard vectors took 14, 47 ms: N = 36864, nev
+        // = 16; the whole FP32 block, twice nev, 53 ms). max(2, nev / 4) against none, N = 1875 to 36864, nev = 2 to
+        // 16, several spectra each: 0.38 to 1.05 of the time. None where the product takes the slower
+        // transforms over the whole mesh (sides without a factor pair), which cost up to 1.4 with them
+        // when the spectrum has its gap (142 x 142, nev = 5: 44 -> 63 ms). A resident FP64 matrix is multiplied by whole tiles of
+        // 16 vectors: the guard fills the last one. Basis 6 blocks up to the device
         // Rayleigh-Ritz limit (4 blocks: up to 1.2 of the time).
         const bool resident = !opt.matrix_free && c.built64;
-        const int guard = std::max(4, nev / 4);
+        const int guard = resident || conv_rows_available(c) ? std::max(2, nev / 4) : 0;
         const int bref = std::min({b, nev + guard, resident ? (nev + 15) / 16 * 16 : b});
         const int mref = static_cast<int>(std::min<int64_t>(
             N, std::max({4 * bref, std::min(6 * bref, projected_eigen_max_dim()), bref + 1})));

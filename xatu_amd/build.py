@@ -36,6 +36,7 @@ DEVICE_SOURCES = [
     "device/matvec.hip",
     "device/vec_kernels.hip",
     "device/solver_step.hip",
+    "device/tridiagonal.hip",
     "device/hf.hip",
     "device/band_adjoint.hip",
     "device/convolution.hip",

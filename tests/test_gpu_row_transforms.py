@@ -1,5 +1,5 @@
 """The convolution product on its row and column transforms: every kind of side they support (the
-smallest and largest, square and uneven factor pairs, one factor equal to 1), windows narrower than
+smallest and largest, square and uneven factor pairs, one factor equal to 1, long prime factors), windows narrower than
 the mesh and as wide as it, reduced meshes (mesh points without a k-point), unequal band numbers,
 and offsets that place two k-points on one mesh point (which stays on the general path). Reference:
 the oracle's matrix; FP64 within 1e-12 and FP32 within 1e-5 of the largest entry of H X, as the other
@@ -35,6 +35,36 @@ def test_large_sides(n):
     # against the recomputed-tiles operator, which shares no code with the transforms
     print(f"[rows] hBN {n}x{n}", flush=True)
     ex = oracle_case(MODELS / "hBN.model", n, 1, 0, (1, 1, 10), cutoff=8, exchange=True)
+    ctx = gpu_context(ex)
+    ctx.build(2)
+    rng = np.random.default_rng(n)
+    x = rng.normal(size=(ex.N, 2)) + 1j * rng.normal(size=(ex.N, 2))
+    ref = ctx.matvec(x, precision=0, matrix_free=2)
+    assert rel_err(ctx.matvec(x, precision=0, matrix_free=1), ref) < 1e-12
+    assert rel_err(ctx.matvec(x, precision=1, matrix_free=1), ref) < 1e-5
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [7, 11, 13, 14, 17, 19, 21, 22, 23, 26, 28, 29, 31, 33, 34, 35])
+def test_sides_with_prime_factors(n):
+    print(f"[rows] hBN {n}x{n}", flush=True)
+    check(oracle_case(MODELS / "hBN.model", n, 1, 0, (1, 1, 10), cutoff=n / 3, exchange=True, Q=(0.03, 0, 0)), 3, n)
+
+
+@pytest.mark.parametrize("n", [38, 46, 49, 57, 58, 62, 69, 77, 87, 91, 92, 93, 98, 102, 110, 112, 115, 119, 121, 124, 126, 37, 41,
+                               43, 47, 53, 59, 61, 74, 106, 111, 122, 123, 67])
+def test_large_sides_with_prime_factors(n):
+    # against the recomputed-tiles operator, which shares no code with the transforms; from 43 on the
+    # primes and their multiples stay on the transforms over whole meshes
+    test_large_sides(n)
+
+
+@pytest.mark.parametrize("n", [7, 13, 23])
+@pytest.mark.parametrize("bands", [(1, 3), (3, 1), (4, 4)])
+def test_bands_with_prime_factors(n, bands, synthetic18):
+    nv, nc = bands
+    print(f"[rows] {n}x{n} bands {bands}", flush=True)
+    ex = oracle_case(synthetic18, n, 4, 0, (1, 1, 40), cutoff=2.0, exchange=True, bands=list(range(1 - nv, nc + 1)))
     ctx = gpu_context(ex)
     ctx.build(2)
     rng = np.random.default_rng(n)

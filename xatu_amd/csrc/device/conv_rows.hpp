@@ -22,6 +22,7 @@
 // SIMD: their vector instructions alone take about half the time.
 #pragma once
 #include <cstdint>
+#include <type_traits>
 
 #include "context.hpp"
 #include "cplx.hpp"
@@ -30,7 +31,10 @@
 namespace xatu_dev {
 
 constexpr int kRowWaves = 4;   // waves per workgroup of the row kernels
-constexpr int kColGroup = 32;  // adjacent columns per workgroup of the column kernel
+// Adjacent columns per workgroup of the column kernel: fewer for the long prime factors, whose
+// workgroups would have too many waves for the registers of their DFT (62 x 62, FP64, 16 columns: 1.70 ms
+// a product, 8: 1.23; 124 x 124: 4.8 and 5.5).
+constexpr int col_group(int A, int B) { return B <= 16 ? 32 : A <= 2 && B > 23 ? 8 : 16; }
 
 // Waves per SIMD of the row kernels (three made the FP32 ones spill: 1.72 -> 1.84 ms).
 constexpr int kRowOccupancy = 2;
@@ -105,6 +109,121 @@ __device__ inline void rows_exchange(void* buf, bool wr, const cx_t<R> (&v)[NW],
     }
 }
 
+// The step of a long prime length B with a short A, spread over the B lanes of a group: each lane
+// forms one frequency of every of the A transforms from the entries of all lanes, which it reads from
+// LDS (the same address for the whole group), with its own B - 1 cosines and sines in registers. In the
+// other form A lanes hold a whole transform each and the others wait: 2 (B - 1)^2 against 4 A (B - 1)
+// multiply-adds (62 = 2 x 31: 1800 on two lanes against 240 on all).
+template <int A, int B>
+constexpr bool rows_spread() {
+    return B >= 11 && B != 12 && B != 14 && B != 15 && B != 16 && 4 * A <= B;
+}
+// Steps of the sum whose LDS reads may be in flight together (more of them spilled: the compiler
+// moved all reads to the front).
+constexpr int kSpreadLoads = 4;
+template <typename R, int B>
+struct SpreadRoots {
+    static constexpr int H = (B - 1) / 2;
+    R c[H], s[H];  // of e^{-2 pi i j k / B}, j = 1 .. H, k the lane's
+    __device__ void load(const cx_t<R>* tw, int A, int k) {
+#pragma unroll
+        for (int j = 1; j <= H; ++j) {
+            const cx_t<R> t = tw[(j * k % B) * A];
+            c[j - 1] = t.x;
+            s[j - 1] = t.y;
+        }
+    }
+};
+// p + i q (SG -1) or p - i q (SG 1): the sums of the entries with the roots or their conjugates.
+template <typename R, int SG>
+__device__ inline cx_t<R> spread_value(cx_t<R> p, cx_t<R> q) {
+    return SG < 0 ? mk(p.x - q.y, p.y + q.x) : mk(p.x + q.y, p.y - q.x);
+}
+// z[k1] of the lanes k2 = 0 .. B - 1 of a group -> out[k1] = sum_k2 z_k2[k1] e^{SG 2 pi i k2 s / B}
+template <typename R, int A, int B, int SG>
+__device__ inline void rows_spread_dft(void* buf, bool on, int s, const cx_t<R> (&z)[A], const SpreadRoots<R, B>& w,
+                                       cx_t<R> (&out)[A]) {
+    constexpr int H = (B - 1) / 2, AP = A | 1;
+    cx_t<R> p[A], q[A];
+    if constexpr (sizeof(R) == 8) {
+        double* e = static_cast<double*>(buf);
+#pragma unroll
+        for (int part = 0; part < 2; ++part) {
+            if (on) {
+#pragma unroll
+                for (int k = 0; k < A; ++k) e[s * AP + k] = part ? z[k].y : z[k].x;
+            }
+            rows_wave_sync();
+            if (on) {
+                double a[A], d[A];
+#pragma unroll
+                for (int k = 0; k < A; ++k) {
+                    a[k] = e[k];
+                    d[k] = 0.0;
+                }
+#pragma unroll
+                for (int j = 1; j <= H; ++j) {
+                    if (j % kSpreadLoads == 0) asm volatile("" ::: "memory");
+#pragma unroll
+                    for (int k = 0; k < A; ++k) {
+                        const double x = e[j * AP + k], y = e[(B - j) * AP + k];
+                        a[k] += w.c[j - 1] * (x + y);
+                        d[k] += w.s[j - 1] * (x - y);
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < A; ++k) {
+                    if (part) {
+                        p[k].y = a[k];
+                        q[k].y = d[k];
+                    } else {
+                        p[k].x = a[k];
+                        q[k].x = d[k];
+                    }
+                }
+            }
+            rows_wave_sync();
+        }
+    } else {
+        float2* e = static_cast<float2*>(buf);
+        if (on) {
+#pragma unroll
+            for (int k = 0; k < A; ++k) e[s * AP + k] = z[k];
+        }
+        rows_wave_sync();
+        if (on) {
+#pragma unroll
+            for (int k = 0; k < A; ++k) {
+                p[k] = e[k];
+                q[k] = mk(0.0f, 0.0f);
+            }
+#pragma unroll
+            for (int j = 1; j <= H; ++j) {
+                if (j % kSpreadLoads == 0) asm volatile("" ::: "memory");
+#pragma unroll
+                for (int k = 0; k < A; ++k) {
+                    const float2 x = e[j * AP + k], y = e[(B - j) * AP + k];
+                    p[k] = mk(p[k].x + w.c[j - 1] * (x.x + y.x), p[k].y + w.c[j - 1] * (x.y + y.y));
+                    q[k] = mk(q[k].x + w.s[j - 1] * (x.x - y.x), q[k].y + w.s[j - 1] * (x.y - y.y));
+                }
+            }
+        }
+        rows_wave_sync();
+    }
+#pragma unroll
+    for (int k = 0; k < A; ++k) out[k] = on ? spread_value<R, SG>(p[k], q[k]) : mk(R(0), R(0));
+}
+// Offsets of the frequencies k1 + A s of a lane of the spread form.
+template <int A, int B>
+__device__ inline void spread_offsets(const RowsArgs& a, int s, int at, bool on, int (&off)[A]) {
+#pragma unroll
+    for (int k1 = 0; k1 < A; ++k1) {
+        int j = k1 + A * s - a.w0;
+        if (j < 0) j += A * B;
+        off[k1] = (on && j < a.W) ? at + j : -1;
+    }
+}
+
 // Coefficients Coef[(c nloop + l) nk + k] of the looped orbitals l0 .. l0 + count - 1 on mesh row
 // o1 to sc[(l NCH + c) n + o0] (zero where the mesh point has no k-point).
 template <typename R, int NCH>
@@ -172,8 +291,16 @@ __global__ __launch_bounds__(64 * kRowWaves, kRowOccupancy) void conv_rows_in_ke
     const int l0 = blockIdx.z * a.lchunk, l1 = min(a.nloop, l0 + a.lchunk);
     // uniform base of the mesh row, 32-bit offsets of the lane's window entries (-1: outside)
     C* grow = G + static_cast<int64_t>(o1) * a.batch * a.W;
-    int off[B];
-    row_offsets<A, B>(a, s, static_cast<int>(f * a.sf + v) * a.W, live && s < A, off);
+    constexpr bool kSpread = rows_spread<A, B>();
+    int off[kSpread ? A : B];
+    SpreadRoots<R, kSpread ? B : 1> roots;
+    if constexpr (kSpread) {
+        spread_offsets<A, B>(a, s, static_cast<int>(f * a.sf + v) * a.W, live, off);
+        __syncthreads();  // the twiddles
+        roots.load(tw, A, s);
+    } else {
+        row_offsets<A, B>(a, s, static_cast<int>(f * a.sf + v) * a.W, live && s < A, off);
+    }
     for (int ls = l0; ls < l1; ls += a.stage) {
         const int count = min(a.stage, l1 - ls);
         __syncthreads();
@@ -190,15 +317,25 @@ __global__ __launch_bounds__(64 * kRowWaves, kRowOccupancy) void conv_rows_in_ke
             dft_len<R, A, -1>(z);
 #pragma unroll
             for (int k1 = 1; k1 < A; ++k1) z[k1] = cmul(z[k1], tw[s * k1]);
-            C x[B];
-            rows_exchange<R, A, B>(
-                xb, gi < GW, z, [&](int i) { return s * AP + i; }, gi < GW && s < A, x, [&](int i) { return i * AP + s; });
-            if (live && s < A) {
-                dft_len<R, B, -1>(x);
+            if constexpr (kSpread) {
+                C x[A];
+                rows_spread_dft<R, A, B, -1>(xb, gi < GW, s, z, roots, x);
                 C* out = grow + static_cast<int64_t>(ls + l) * a.sl * a.W;
 #pragma unroll
-                for (int k2 = 0; k2 < B; ++k2)
-                    if (off[k2] >= 0) out[static_cast<unsigned>(off[k2])] = x[k2];
+                for (int k1 = 0; k1 < A; ++k1)
+                    if (off[k1] >= 0) out[static_cast<unsigned>(off[k1])] = x[k1];
+            } else {
+                C x[B];
+                rows_exchange<R, A, B>(
+                    xb, gi < GW, z, [&](int i) { return s * AP + i; }, gi < GW && s < A, x,
+                    [&](int i) { return i * AP + s; });
+                if (live && s < A) {
+                    dft_len<R, B, -1>(x);
+                    C* out = grow + static_cast<int64_t>(ls + l) * a.sl * a.W;
+#pragma unroll
+                    for (int k2 = 0; k2 < B; ++k2)
+                        if (off[k2] >= 0) out[static_cast<unsigned>(off[k2])] = x[k2];
+                }
             }
         }
     }
@@ -234,15 +371,25 @@ __global__ __launch_bounds__(64 * kRowWaves, kRowOccupancy) void conv_rows_out_k
     const int l0 = blockIdx.z * a.lchunk, l1 = min(a.nloop, l0 + a.lchunk);
     const C* grow = G + static_cast<int64_t>(o1) * a.batch * a.W;
     const R cs = a.conj ? R(-1) : R(1);
-    int off[B];
-    row_offsets<A, B>(a, s, static_cast<int>(f * a.sf + v) * a.W, live && s < A, off);
+    constexpr bool kSpread = rows_spread<A, B>();
+    constexpr int NX = kSpread ? A : B;  // window entries of a lane
+    int off[NX];
+    SpreadRoots<R, kSpread ? B : 1> roots;
+    if constexpr (kSpread) {
+        spread_offsets<A, B>(a, s, static_cast<int>(f * a.sf + v) * a.W, live, off);
+        __syncthreads();  // the twiddles
+        roots.load(tw, A, s);
+    } else {
+        row_offsets<A, B>(a, s, static_cast<int>(f * a.sf + v) * a.W, live && s < A, off);
+    }
     // the next row's window is loaded one row ahead where the registers allow it
-    constexpr bool kAhead = sizeof(R) * (A * NCH + 3 * B) <= 8 * 56;
-    C x[B];
+    // (a long prime's DFT holds its entries twice)
+    constexpr bool kAhead = kSpread || sizeof(R) * (A * NCH + (B > 16 ? 5 : 3) * B) <= 8 * 56;
+    C x[NX];
     auto load = [&](int l) {
         const C* in = grow + static_cast<int64_t>(l) * a.sl * a.W;
 #pragma unroll
-        for (int k2 = 0; k2 < B; ++k2) x[k2] = off[k2] >= 0 ? in[static_cast<unsigned>(off[k2])] : mk(R(0), R(0));
+        for (int k2 = 0; k2 < NX; ++k2) x[k2] = off[k2] >= 0 ? in[static_cast<unsigned>(off[k2])] : mk(R(0), R(0));
     };
     if (kAhead && l0 < l1) load(l0);
     for (int ls = l0; ls < l1; ls += a.stage) {
@@ -252,18 +399,24 @@ __global__ __launch_bounds__(64 * kRowWaves, kRowOccupancy) void conv_rows_out_k
         __syncthreads();
         for (int l = 0; l < count; ++l) {
             if (!kAhead) load(ls + l);
-            C y[B];
+            C y[NX], w[A];
 #pragma unroll
-            for (int i = 0; i < B; ++i) y[i] = x[i];
+            for (int i = 0; i < NX; ++i) y[i] = x[i];
             if (kAhead && ls + l + 1 < l1) load(ls + l + 1);
-            dft_len<R, B, 1>(y);
-            if (s < A) {
+            if constexpr (kSpread) {
+                rows_spread_dft<R, A, B, 1>(xb, gi < GW, s, y, roots, w);
 #pragma unroll
-                for (int i = 1; i < B; ++i) y[i] = cmul(y[i], cconj(tw[i * s]));
+                for (int k1 = 1; k1 < A; ++k1) w[k1] = cmul(w[k1], cconj(tw[s * k1]));
+            } else {
+                dft_len<R, B, 1>(y);
+                if (s < A) {
+#pragma unroll
+                    for (int i = 1; i < B; ++i) y[i] = cmul(y[i], cconj(tw[i * s]));
+                }
+                rows_exchange<R, B, A>(
+                    xb, gi < GW && s < A, y, [&](int i) { return i * AP + s; }, gi < GW, w,
+                    [&](int i) { return s * AP + i; });
             }
-            C w[A];
-            rows_exchange<R, B, A>(
-                xb, gi < GW && s < A, y, [&](int i) { return i * AP + s; }, gi < GW, w, [&](int i) { return s * AP + i; });
             dft_len<R, A, 1>(w);
 #pragma unroll
             for (int j = 0; j < A; ++j)
@@ -287,17 +440,30 @@ __global__ __launch_bounds__(64 * kRowWaves, kRowOccupancy) void conv_rows_out_k
     }
 }
 
+// The spectrum of column u = b W + j: entry xi_1 at [xi_1 W].
+template <typename R>
+__device__ inline const R* spectrum_of(const LatticeDesc& lat, int W, int nvec, int64_t u, int n, const R* P) {
+    const int64_t b = u / W;
+    const int j = static_cast<int>(u - b * W);
+    const int ab = static_cast<int>(b / nvec);
+    const int al = ab / lat.norb, be = ab - al * lat.norb;
+    int pa = 0, pb = 0;
+    while (al >= lat.orb_begin[pa + 1]) ++pa;
+    while (be >= lat.orb_begin[pb + 1]) ++pb;
+    return P + static_cast<int64_t>(pa + lat.natoms * pb) * n * W + j;
+}
+
 // Columns u = b W + j of G (length n, stride count = batch W): transform along o1, times the real
 // spectrum P[(pa n + xi_1) W + j] of the atom pair of b, inverse; in place. SPECTRUM false:
 // forward transform only, frequency xi_1 left at row xi_1. Lane (s, column) holds rows B j2 + s,
-// then frequency k1 = s of the first step. grid ceil(count / 32), block 32 B, dynamic LDS
-// (n + 32 n) entries.
+// then frequency k1 = s of the first step. T = col_group(A, B): grid ceil(count / T), block T B, dynamic LDS
+// (n + T n) entries.
 template <typename R, int A, int B, bool SPECTRUM>
-__global__ __launch_bounds__(kColGroup* B) void conv_columns_kernel(LatticeDesc lat, int W, int64_t count, int nvec,
+__global__ __launch_bounds__(col_group(A, B) * B) void conv_columns_kernel(LatticeDesc lat, int W, int64_t count, int nvec,
                                                                     const double2* __restrict__ root,
                                                                     const R* __restrict__ P, cx_t<R>* __restrict__ G) {
     using C = cx_t<R>;
-    constexpr int n = A * B, T = kColGroup;
+    constexpr int n = A * B, T = col_group(A, B);
     extern __shared__ unsigned char rows_raw[];
     C* tw = reinterpret_cast<C*>(rows_raw);
     C* ex = tw + n;
@@ -316,21 +482,61 @@ __global__ __launch_bounds__(kColGroup* B) void conv_columns_kernel(LatticeDesc 
         for (int k = 0; k < A; ++k) ex[(s * A + k) * T + c] = k ? cmul(v[k], tw[s * k]) : v[k];
     }
     __syncthreads();
+    if constexpr (rows_spread<A, B>() && A <= 2) {
+        // the long prime's step spread over the lanes of a column (as in the row kernels; from A = 3 on
+        // the whole transforms per lane are the faster ones here: 87 x 87 and 124 x 124 products
+        // 3.0 against 3.6 ms and 6.2 against 7.8)
+        SpreadRoots<R, B> roots;
+        roots.load(tw, A, s);
+        C v[A];
+        auto spread = [&](auto sign) {
+            constexpr int SG = decltype(sign)::value;
+#pragma unroll
+            for (int k1 = 0; k1 < A; ++k1) {
+                C p = ex[k1 * T + c], q = mk(R(0), R(0));
+#pragma unroll
+                for (int j = 1; j <= (B - 1) / 2; ++j) {
+                    const C x = ex[(j * A + k1) * T + c], y = ex[((B - j) * A + k1) * T + c];
+                    p = mk(p.x + roots.c[j - 1] * (x.x + y.x), p.y + roots.c[j - 1] * (x.y + y.y));
+                    q = mk(q.x + roots.s[j - 1] * (x.x - y.x), q.y + roots.s[j - 1] * (x.y - y.y));
+                }
+                v[k1] = spread_value<R, SG>(p, q);
+            }
+        };
+        spread(std::integral_constant<int, -1>{});
+        if constexpr (SPECTRUM) {
+            const R* p = spectrum_of(lat, W, nvec, live ? u : count - 1, n, P);
+#pragma unroll
+            for (int k1 = 0; k1 < A; ++k1) {
+                const R f = p[static_cast<int64_t>(k1 + A * s) * W];
+                v[k1].x *= f;
+                v[k1].y *= f;
+            }
+            __syncthreads();  // every lane has read the entries
+#pragma unroll
+            for (int k1 = 0; k1 < A; ++k1) ex[(s * A + k1) * T + c] = v[k1];
+            __syncthreads();
+            spread(std::integral_constant<int, 1>{});
+#pragma unroll
+            for (int k1 = 1; k1 < A; ++k1) v[k1] = cmul(v[k1], cconj(tw[s * k1]));
+            dft_len<R, A, 1>(v);
+            if (live) {
+#pragma unroll
+                for (int j = 0; j < A; ++j) g[static_cast<int64_t>(B * j + s) * count] = v[j];
+            }
+        } else if (live) {
+#pragma unroll
+            for (int k1 = 0; k1 < A; ++k1) g[static_cast<int64_t>(k1 + A * s) * count] = v[k1];
+        }
+        return;
+    } else {
     C v[B];
     if (s < A) {
 #pragma unroll
         for (int i = 0; i < B; ++i) v[i] = ex[(i * A + s) * T + c];
         dft_len<R, B, -1>(v);
         if constexpr (SPECTRUM) {
-            const int64_t uu = live ? u : count - 1;
-            const int64_t b = uu / W;
-            const int j = static_cast<int>(uu - b * W);
-            const int ab = static_cast<int>(b / nvec);
-            const int al = ab / lat.norb, be = ab - al * lat.norb;
-            int pa = 0, pb = 0;
-            while (al >= lat.orb_begin[pa + 1]) ++pa;
-            while (be >= lat.orb_begin[pb + 1]) ++pb;
-            const R* p = P + static_cast<int64_t>(pa + lat.natoms * pb) * n * W + j;
+            const R* p = spectrum_of(lat, W, nvec, live ? u : count - 1, n, P);
 #pragma unroll
             for (int k = 0; k < B; ++k) {
                 const R q = p[static_cast<int64_t>(s + A * k) * W];
@@ -360,6 +566,7 @@ __global__ __launch_bounds__(kColGroup* B) void conv_columns_kernel(LatticeDesc 
 #pragma unroll
             for (int j = 0; j < A; ++j) g[static_cast<int64_t>(B * j + s) * count] = w[j];
         }
+    }
     }
 }
 

@@ -1,4 +1,4 @@
-"""Full diagonalisation on the own reduction to tridiagonal form: dimensions around a wave's 64 rows,
+"""Full diagonalisation on the own reduction to tridiagonal form and back-transformation (to 1024): dimensions around a wave's 64 rows,
 the row counts its kernels are compiled for (256, 512, 1024, 2048), the smallest it takes (4 here) and one
 past it, which stays with the library; real matrices without an exchange term among them, degenerate pairs
 and off-diagonals that vanish. Errors of a backward stable reduction grow at most like n 2^-53 of the norm:

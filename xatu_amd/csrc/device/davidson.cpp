@@ -2,8 +2,8 @@
 //
 // Dense path ("diag", reference src/ExcitonTB.cpp:940-943 -> LAPACK zheevd):
 // all eigenpairs ascending, from a device copy of the FP64 matrix: up to n = 2048 the own
-// reduction to tridiagonal form (tridiagonal.hip) between rocSOLVER's tridiagonal eigensolver and
-// back-transformation, rocSOLVER zheevd beyond.
+// reduction to tridiagonal form and (to 1024) back-transformation (tridiagonal.hip) around rocSOLVER's
+// tridiagonal eigensolver, rocSOLVER zheevd beyond.
 //
 // Block Davidson ("davidson", reference src/davidson.cpp:5-61, redesigned):
 // the basis V, its image W = H V, Ritz vectors and residuals live in HBM in FP64;
@@ -50,6 +50,8 @@ void launch_precondition(const double2* R, const double* theta, const double* di
 void launch_unit_vectors(const int* idx, int64_t N, int nvec, double2* V, hipStream_t s);
 void launch_copy_vectors(const double2* src, int64_t n, double2* dst, hipStream_t s);
 int tridiagonal_max_dim();
+int reflectors_max_dim();
+void launch_apply_reflectors(const double2* R, const double2* tau, int n, double2* C, hipStream_t s);
 void launch_tridiagonal(double2* A, int n, double2* p, double2* R, double2* tau, double* D, double* E, hipStream_t s);
 int projected_eigen_max_dim();
 int projected_eigen_max_want();
@@ -557,8 +559,9 @@ void solve_dense_diag(Context& c, int nstates, double* eigval_out, double* eigve
     XATU_HIP(hipMemcpyAsync(A.p, c.d_H64.p, nn * sizeof(double2), hipMemcpyDeviceToDevice, c.stream));
     const double2* vec = A.p;
     if (own) {
-        // own reduction to tridiagonal form, one kernel per column, where it is the faster one (it
-        // ends at 2048; the library: n = 100 2.2 ms against 1.6, 2025 68 against 48)
+        // own reduction to tridiagonal form, one kernel per column, and to 1024 own back-transformation,
+        // where they are the faster ones (the library: n = 100 2.2 ms against 1.2, 1024 28.6 against
+        // 12.7, 2025 68 against 45)
         DevBuf<double2>&R = c.solver_ws[0].W, &C = c.solver_ws[0].X, &small = c.solver_ws[0].AX;
         R.reserve(nn);
         C.reserve(nn);
@@ -567,8 +570,11 @@ void solve_dense_diag(Context& c, int nstates, double* eigval_out, double* eigve
         XATU_HIP(hipMemsetAsync(R.p, 0, nn * sizeof(double2), c.stream));  // what no reflector stores stays finite
         launch_tridiagonal(A.p, n, small.p, R.p, tau, D, E, c.stream);
         XATU_BLAS(rocsolver_zstedc(c.blas, rocblas_evect_tridiagonal, n, D, E, bz(C.p), n, info.p));
-        XATU_BLAS(rocsolver_zunmtr(c.blas, rocblas_side_left, rocblas_fill_lower, rocblas_operation_none, n, n, bz(R.p), n,
-                                   bz(tau), bz(C.p), n));
+        if (n <= reflectors_max_dim())
+            launch_apply_reflectors(R.p, tau, n, C.p, c.stream);
+        else
+            XATU_BLAS(rocsolver_zunmtr(c.blas, rocblas_side_left, rocblas_fill_lower, rocblas_operation_none, n, n,
+                                       bz(R.p), n, bz(tau), bz(C.p), n));
         vec = C.p;
     } else {
         XATU_BLAS(rocsolver_zheevd(c.blas, rocblas_evect_original, rocblas_fill_lower, n, bz(A.p), n, D, E, info.p));

@@ -14,6 +14,7 @@
 #include "context.hpp"
 #include "cplx.hpp"
 #include "solver_step.hpp"
+#include "wave_sums.hpp"
 
 #include <algorithm>
 
@@ -101,8 +102,7 @@ __global__ __launch_bounds__(64 * kStepMaxBlock / kCols) __attribute__((amdgpu_w
             const double th = theta[j];
             const double2 r = mk(w[j].x - th * x[j].x, w[j].y - th * x[j].y);
             double s = ok ? r.x * r.x + r.y * r.y : 0.0;
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+            s = wave_sum(s);
             if (lane == 0) a.partial[static_cast<int64_t>(jj) * gridDim.x + blockIdx.x] = s;
             if (ok) {
                 const int64_t at = i + static_cast<int64_t>(jj) * a.N;

@@ -10,21 +10,17 @@
 // column, its reflector) and then, for its own columns, applies the update and multiplies by
 // the new reflector in one pass over the column. The loads of the columns are issued before
 // the small part. A column always belongs to the same workgroup number, hence to the same XCD's L2.
-// n = 400: 5.5 us a step, the reduction about 8 -> 2.2 ms, all eigenpairs 10.8 -> 5.6 ms; n = 1024: 28.6 ->
-// 16.1 ms; n = 2025: 68 -> 48 ms. A lane keeps its rows of a column in registers, which ends at
+// n = 400: 5.0 us a step (5.5 with the sums over a wave by shuffles instead of DPP), the reduction about
+// 8 -> 2.0 ms; all eigenpairs with apply_reflectors_kernel 10.8 -> 4.1 ms, n = 1024 28.6 -> 12.7, n = 2025 68
+// -> 45 ms. A lane keeps its rows of a column in registers, which ends at
 // 32 (n = 2048; a step then moves 64 MB through the last-level cache and costs as much as the library's).
 #include "context.hpp"
 #include "cplx.hpp"
+#include "wave_sums.hpp"
 
 namespace xatu_dev {
 
 namespace {
-
-__device__ inline double wave_total(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
 
 // Step j. v (column j - 1 of R with its unit entry) and p = A v of step j - 1 give w = tau p -
 // (tau / 2) (tau p)^H v v; A <- A - v w^H - w v^H on rows and columns j and above; column j then gives D[j],
@@ -73,8 +69,8 @@ __global__ __launch_bounds__(64 * WAVES) void tridiagonal_step_kernel(double2* _
         si += w[k].x * v[k].y - w[k].y * v[k].x;
     }
     if (j > 0) {
-        sr = wave_total(sr);
-        si = wave_total(si);
+        sr = wave_sum(sr);
+        si = wave_sum(si);
         if (lane == 0) {
             s_red[0][wave][0] = sr;
             s_red[0][wave][1] = si;
@@ -114,7 +110,7 @@ __global__ __launch_bounds__(64 * WAVES) void tridiagonal_step_kernel(double2* _
         if (r == j + 1 && r < n) s_alpha = a[k];
         if (r == j && last) D[j] = a[k].x;
     }
-    norm = wave_total(norm);
+    norm = wave_sum(norm);
     if (lane == 0) s_red[1][wave][0] = norm;
     __syncthreads();
     if (j + 1 >= n) return;
@@ -163,9 +159,72 @@ __global__ __launch_bounds__(64 * WAVES) void tridiagonal_step_kernel(double2* _
             pi += x.x * y.y - x.y * y.x;
         }
     }
-    pr = wave_total(pr);
-    pi = wave_total(pi);
+    pr = wave_sum(pr);
+    pi = wave_sum(pi);
     if (lane == 0) next[c] = mk(pr, pi);
+}
+
+// C <- Q C: a wave holds one column of C in registers and applies the reflectors to it from the last
+// one on, each as a dot product over the wave and an update; the next few reflectors are on their way
+// meanwhile. Bound by that chain, 0.5 us a reflector, while the reflectors, which every wave
+// reads, come from the caches: n = 400 1.3 ms by the library's blocked products -> 0.21 (0.38 with
+// one reflector ahead and branches around the finished rows). To n = 1024, where all of them are 16 MB.
+template <int Q>
+__global__ __launch_bounds__(256) void apply_reflectors_kernel(const double2* __restrict__ R,
+                                                               const double2* __restrict__ tau, int n,
+                                                               double2* __restrict__ C) {
+    const int lane = threadIdx.x & 63;
+    const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (c >= n) return;
+    double2* col = C + static_cast<int64_t>(c) * n;
+    constexpr int D = 4;  // reflectors in flight
+    double2 x[Q], v[D][Q], t[D];
+    // without branches, so that the loads of several reflectors can be counted: R is zero where no
+    // reflector is stored
+    auto load = [&](double2 (&dst)[Q], double2& tj, int j) {
+        const int64_t jj = j < 0 ? 0 : j;
+        tj = tau[jj];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) dst[q] = R[min(lane + 64 * q, n - 1) + jj * n];
+    };
+    auto apply = [&](double2 (&u)[Q], double2 tj, int j) {
+        double sr = 0.0, si = 0.0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int r = lane + 64 * q;
+            const bool in = r < n;
+            u[q].x = r == j + 1 ? 1.0 : in ? u[q].x : 0.0;
+            u[q].y = in ? u[q].y : 0.0;  // zero at j + 1
+            sr += u[q].x * x[q].x + u[q].y * x[q].y;  // conj(v) x
+            si += u[q].x * x[q].y - u[q].y * x[q].x;
+        }
+        const double2 f = cmul(tj, mk(wave_sum(sr), wave_sum(si)));
+#pragma unroll
+        for (int q = 0; q < Q; ++q) x[q] = csub(x[q], cmul(f, u[q]));
+    };
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int r = lane + 64 * q;
+        x[q] = r < n ? col[r] : mk(0.0, 0.0);
+    }
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d) load(v[d], t[d], n - 2 - d);
+    int j = n - 2;
+    for (; j >= D - 1; j -= D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            load(v[(d + D - 1) % D], t[(d + D - 1) % D], j - d - (D - 1));
+            apply(v[d], t[d], j - d);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d)
+        if (j - d >= 0) apply(v[d], t[d], j - d);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int r = lane + 64 * q;
+        if (r < n) col[r] = x[q];
+    }
 }
 
 template <int Q, int WAVES>
@@ -179,6 +238,16 @@ void run_steps(double2* A, int n, double2* p, double2* R, double2* tau, double* 
 }  // namespace
 
 int tridiagonal_max_dim() { return 2048; }
+int reflectors_max_dim() { return 1024; }
+
+void launch_apply_reflectors(const double2* R, const double2* tau, int n, double2* C, hipStream_t s) {
+    if (n < 2 || n > reflectors_max_dim()) throw Error(XATU_ERR_INVALID_ARGUMENT, "reflectors: unsupported dimension");
+    const dim3 grid((n + 3) / 4), block(256);
+    if (n <= 256) hipLaunchKernelGGL((apply_reflectors_kernel<4>), grid, block, 0, s, R, tau, n, C);
+    else if (n <= 512) hipLaunchKernelGGL((apply_reflectors_kernel<8>), grid, block, 0, s, R, tau, n, C);
+    else hipLaunchKernelGGL((apply_reflectors_kernel<16>), grid, block, 0, s, R, tau, n, C);
+    XATU_HIP(hipGetLastError());
+}
 
 void launch_tridiagonal(double2* A, int n, double2* p, double2* R, double2* tau, double* D, double* E, hipStream_t s) {
     if (n < 1 || n > tridiagonal_max_dim()) throw Error(XATU_ERR_INVALID_ARGUMENT, "tridiagonal reduction: unsupported dimension");

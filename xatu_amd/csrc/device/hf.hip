@@ -19,13 +19,13 @@
 // the reference's construction H = A + A^H from the upper triangle:
 //   psi^H dX psi = Re sum_ab dMQ_ab (2 P_ab + G_ab),
 //   P_ab = sum_j (sum_{i<j} f_a(i)) g_b(j),  G_ab = sum_i f_a(i) g_b(i),
-// with f_a(i) = conj(psi_i) rho1_a(i), g_b(j) = rho2_b(j) psi_j (rows on the GPU,
-// the prefix sums on the host).
+// with f_a(i) = conj(psi_i) rho1_a(i), g_b(j) = rho2_b(j) psi_j (prefixes by runs of rows).
 #include <cmath>
 #include <vector>
 
 #include "context.hpp"
 #include "cplx.hpp"
+#include "wave_sums.hpp"
 #include "potential_dev.hpp"
 
 namespace xatu_dev {
@@ -217,6 +217,92 @@ __global__ void exchange_rows_kernel(LatticeDesc lat, int nk, int nv, int nc, co
     }
 }
 
+// Sum over the workgroup's 256 threads, the same in every thread.
+__device__ inline double group_sum(double x, double* red) {
+    x = wave_sum(x);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+    __syncthreads();
+    return (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// W[s][a + na b] = 2 P_ab + G_ab, P_ab = sum_{j < i} f_a(j) g_b(i), G_ab = sum_i f_a(i) g_b(i): the
+// exchange sums along the upper triangle. A thread has a run of rows; the runs' sums of f are
+// scanned in LDS, which gives each its prefix. grid (states, na), block 256. Bound by the latency of a thread's
+// loads: N = 5184, 3 atoms, 8 states: 20 us (on the host these sums, the contractions below and their
+// read-backs took 2.4 of the 2.8 ms of a call).
+__global__ __launch_bounds__(256) void exchange_sums_kernel(int na, int64_t N, const double2* __restrict__ fg,
+                                                            double2* __restrict__ W) {
+    __shared__ double2 s_run[256];
+    __shared__ double red[4];
+    const int st = blockIdx.x, a = blockIdx.y, t = threadIdx.x;
+    const int64_t run = (N + 255) / 256, i0 = min(N, t * run), i1 = min(N, i0 + run);
+    const double2* row = fg + static_cast<size_t>(st) * N * 2 * na;
+    double2 total = mk(0.0, 0.0);
+#pragma unroll 4
+    for (int64_t i = i0; i < i1; ++i) total = cadd(total, row[i * 2 * na + a]);
+    s_run[t] = total;
+    __syncthreads();
+    for (int d = 1; d < 256; d <<= 1) {
+        const double2 v = t >= d ? s_run[t - d] : mk(0.0, 0.0);
+        __syncthreads();
+        s_run[t] = cadd(s_run[t], v);
+        __syncthreads();
+    }
+    const double2 before = t > 0 ? s_run[t - 1] : mk(0.0, 0.0);
+    for (int b = 0; b < na; ++b) {
+        double2 F = before, P = mk(0.0, 0.0), G = mk(0.0, 0.0);
+#pragma unroll 4
+        for (int64_t i = i0; i < i1; ++i) {
+            const double2 f = row[i * 2 * na + a], g = row[i * 2 * na + na + b];
+            cfma(P, F, g);
+            cfma(G, f, g);
+            F = cadd(F, f);
+        }
+        const double re = group_sum(2.0 * P.x + G.x, red), im = group_sum(2.0 * P.y + G.y, red);
+        if (t == 0) W[static_cast<size_t>(st) * na * na + a + na * b] = mk(re, im);
+    }
+}
+
+// Contractions of the derivative tables: out[s] = sum_e dv[e] Shat[s][e] (workgroup per state), and after them
+// per pair sum_R dvx_p(R) e^{iQ R} as two values. block 256
+__global__ __launch_bounds__(256) void gradient_sums_kernel(LatticeDesc lat, int nstates, int npairs, int nR,
+                                                            const double* __restrict__ dv,
+                                                            const double* __restrict__ dvx,
+                                                            const double* __restrict__ shat,
+                                                            const int* __restrict__ cells, double qx, double qy,
+                                                            double qz, double* __restrict__ out) {
+    __shared__ double red[4];
+    if (static_cast<int>(blockIdx.x) < nstates) {
+        const int64_t n = static_cast<int64_t>(npairs) * nR;
+        const double* sh = shat + blockIdx.x * n;
+        double sum = 0.0;
+#pragma unroll 4
+        for (int64_t e = threadIdx.x; e < n; e += 256) sum += dv[e] * sh[e];
+        sum = group_sum(sum, red);
+        if (threadIdx.x == 0) out[blockIdx.x] = sum;
+        return;
+    }
+    const int p = blockIdx.x - nstates;
+    double mr = 0.0, mi = 0.0;
+    for (int R = threadIdx.x; R < nR; R += 256) {
+        double v[3] = {0.0, 0.0, 0.0};
+        for (int j = 0; j < lat.ndim; ++j)
+            for (int x = 0; x < 3; ++x) v[x] += static_cast<double>(cells[3 * R + j]) * lat.bravais[3 * j + x];
+        double si, co;
+        sincos(qx * v[0] + qy * v[1] + qz * v[2], &si, &co);
+        const double d = dvx[static_cast<int64_t>(p) * nR + R];
+        mr += d * co;
+        mi += d * si;
+    }
+    mr = group_sum(mr, red);
+    mi = group_sum(mi, red);
+    if (threadIdx.x == 0) {
+        out[nstates + 2 * p] = mr;
+        out[nstates + 2 * p + 1] = mi;
+    }
+}
+
 }  // namespace
 
 void hf_gradients(Context& c, int nstates, const double2* d_vec, int nparams, const int* params, double* grad_out) {
@@ -227,29 +313,32 @@ void hf_gradients(Context& c, int nstates, const double2* d_vec, int nparams, co
     const double T = static_cast<double>(c.inter.total_cells);
     hipStream_t s = c.stream;
 
-    // k -> mesh-offset map
-    const int n = c.lat.mesh_n;
-    std::vector<int> kmap(c.lat.nmesh, -1);
-    for (int k = 0; k < c.nk; ++k) {
-        int lin = 0, mul = 1;
-        for (int j = 0; j < c.lat.ndim; ++j) {
-            int o = c.h_koff[k * c.lat.ndim + j] % n;
-            if (o < 0) o += n;
-            lin += o * mul;
-            mul *= n;
-        }
-        kmap[lin] = k;
-    }
+    const bool direct = c.lat.ndim == 2 && conv_rows_available(c);
     DevBuf<int> d_kmap;
-    d_kmap.alloc(kmap.size());
-    XATU_HIP(hipMemcpyAsync(d_kmap.p, kmap.data(), kmap.size() * sizeof(int), hipMemcpyHostToDevice, s));
-
-    // pair-density adjoint S and its lattice adjoint Shat, kHfStates states at a time
     DevBuf<double2> S;
-    S.alloc(static_cast<size_t>(kHfStates) * c.lat.nmesh * na * na);
+    if (!direct) {
+        // pair-density adjoint of kHfStates states at a time; k -> mesh-offset map
+        const int n = c.lat.mesh_n;
+        std::vector<int> kmap(c.lat.nmesh, -1);
+        for (int k = 0; k < c.nk; ++k) {
+            int lin = 0, mul = 1;
+            for (int j = 0; j < c.lat.ndim; ++j) {
+                int o = c.h_koff[k * c.lat.ndim + j] % n;
+                if (o < 0) o += n;
+                lin += o * mul;
+                mul *= n;
+            }
+            kmap[lin] = k;
+        }
+        d_kmap.alloc(kmap.size());
+        XATU_HIP(hipMemcpyAsync(d_kmap.p, kmap.data(), kmap.size() * sizeof(int), hipMemcpyHostToDevice, s));
+        S.alloc(static_cast<size_t>(kHfStates) * c.lat.nmesh * na * na);
+        XATU_HIP(hipStreamSynchronize(s));  // the map goes
+    }
+
+    // the lattice adjoint Shat of every state
     DevBuf<double> shat;
     shat.alloc(static_cast<size_t>(nstates) * npairs * nR);
-    const bool direct = c.lat.ndim == 2 && conv_rows_available(c);
     const int step = direct ? kHfRowStates : kHfStates;
     for (int s0 = 0; s0 < nstates; s0 += step) {
         const int ns = std::min(step, nstates - s0);
@@ -271,114 +360,69 @@ void hf_gradients(Context& c, int nstates, const double2* d_vec, int nparams, co
                            shat.p + static_cast<size_t>(s0) * npairs * nR);
         XATU_HIP(hipGetLastError());
     }
-    std::vector<double> h_shat(shat.n);
-    XATU_HIP(hipMemcpyAsync(h_shat.data(), shat.p, shat.bytes(), hipMemcpyDeviceToHost, s));
-
-    // exchange rows f, g (host prefix sums below)
-    std::vector<double2> h_fg;
-    if (c.inter.exchange) {
-        DevBuf<double2> fg;
+    const bool exchange = c.inter.exchange;
+    DevBuf<double2> fg, Wx;
+    if (exchange) {
         fg.alloc(static_cast<size_t>(nstates) * c.N * 2 * na);
+        Wx.alloc(static_cast<size_t>(nstates) * na * na);
         hipLaunchKernelGGL(exchange_rows_kernel, dim3((c.N + 255) / 256, nstates), dim3(256), 0, s, c.lat, c.nk, c.nv,
                            c.nc, c.d_evec_k.p, c.d_evec_kq.p, c.d_e1.p, d_vec, c.N, fg.p);
+        hipLaunchKernelGGL(exchange_sums_kernel, dim3(nstates, na), dim3(256), 0, s, na, c.N, fg.p, Wx.p);
         XATU_HIP(hipGetLastError());
-        h_fg.resize(fg.n);
-        XATU_HIP(hipMemcpyAsync(h_fg.data(), fg.p, fg.bytes(), hipMemcpyDeviceToHost, s));
-        XATU_HIP(hipStreamSynchronize(s));
     }
-    XATU_HIP(hipStreamSynchronize(s));
-    std::vector<double> cellsR(static_cast<size_t>(nR) * 3, 0.0);
-    for (int r = 0; r < nR; ++r)
-        for (int j = 0; j < c.lat.ndim; ++j)
-            for (int x = 0; x < 3; ++x) cellsR[3 * r + x] += c.h_cells[r * c.lat.ndim + j] * c.lat.bravais[3 * j + x];
-
-    // W_ab = 2 P_ab + G_ab per state (triangular exchange sums, FP64 on the host)
-    std::vector<double2> Wx(static_cast<size_t>(nstates) * na * na, mk(0.0, 0.0));
-    if (c.inter.exchange) {
-        for (int st = 0; st < nstates; ++st) {
-            std::vector<double> Fr(na, 0.0), Fi(na, 0.0);
-            std::vector<double> Pr(na * na, 0.0), Pi(na * na, 0.0), Gr(na * na, 0.0), Gi(na * na, 0.0);
-            for (int64_t i = 0; i < c.N; ++i) {
-                const double2* row = h_fg.data() + (static_cast<size_t>(st) * c.N + i) * 2 * na;
-                for (int a = 0; a < na; ++a)
-                    for (int b = 0; b < na; ++b) {
-                        const double2 g = row[na + b];
-                        Pr[a + na * b] += Fr[a] * g.x - Fi[a] * g.y;
-                        Pi[a + na * b] += Fr[a] * g.y + Fi[a] * g.x;
-                        const double2 f = row[a];
-                        Gr[a + na * b] += f.x * g.x - f.y * g.y;
-                        Gi[a + na * b] += f.x * g.y + f.y * g.x;
-                    }
-                for (int a = 0; a < na; ++a) {
-                    Fr[a] += row[a].x;
-                    Fi[a] += row[a].y;
-                }
-            }
-            for (int e = 0; e < na * na; ++e)
-                Wx[static_cast<size_t>(st) * na * na + e] = mk(2.0 * Pr[e] + Gr[e], 2.0 * Pi[e] + Gi[e]);
-        }
-    }
-    DevBuf<double> dv;
-    dv.alloc(static_cast<size_t>(npairs) * nR);
-    std::vector<double> h_dv(dv.n), h_dvx(dv.n);
     // quadrature rule of the dV/dr0 evaluation
     static const std::vector<double> h_gl = [] {
         std::vector<double> r(2 * kGlNodes);
         gauss_legendre_rule(r.data());
         return r;
     }();
-    DevBuf<double> gl;
-    gl.alloc(h_gl.size());
-    XATU_HIP(hipMemcpyAsync(gl.p, h_gl.data(), gl.bytes(), hipMemcpyHostToDevice, s));
+    // derivative tables of one parameter (direct, exchange), their contractions for all parameters
+    const size_t ntab = static_cast<size_t>(npairs) * nR, nout = static_cast<size_t>(nstates) + 2 * npairs;
+    DevBuf<double> work;
+    work.alloc(h_gl.size() + 2 * ntab + nout * nparams);
+    double *gl = work.p, *dv = gl + h_gl.size(), *dvx = dv + ntab, *out = dvx + ntab;
+    XATU_HIP(hipMemcpyAsync(gl, h_gl.data(), h_gl.size() * sizeof(double), hipMemcpyHostToDevice, s));
     for (int ip = 0; ip < nparams; ++ip) {
         const int which = (params[ip] == XATU_PARAM_R0) ? 0 : 1;
         hipLaunchKernelGGL(dpotential_table_kernel, dim3((nR + 255) / 256, npairs), dim3(256), 0, s, c.lat, c.pot_d,
-                           c.d_cells.p, nR, npairs, which, gl.p, dv.p);
-        XATU_HIP(hipGetLastError());
-        XATU_HIP(hipMemcpyAsync(h_dv.data(), dv.p, dv.bytes(), hipMemcpyDeviceToHost, s));
-        if (c.inter.exchange) {
-            XATU_HIP(hipStreamSynchronize(s));
+                           c.d_cells.p, nR, npairs, which, gl, dv);
+        if (exchange)
             hipLaunchKernelGGL(dpotential_table_kernel, dim3((nR + 255) / 256, npairs), dim3(256), 0, s, c.lat,
-                               c.pot_x, c.d_cells.p, nR, npairs, which, gl.p, dv.p);
-            XATU_HIP(hipGetLastError());
-            XATU_HIP(hipMemcpyAsync(h_dvx.data(), dv.p, dv.bytes(), hipMemcpyDeviceToHost, s));
-        }
-        XATU_HIP(hipStreamSynchronize(s));
+                               c.pot_x, c.d_cells.p, nR, npairs, which, gl, dvx);
+        hipLaunchKernelGGL(gradient_sums_kernel, dim3(nstates + (exchange ? npairs : 0)), dim3(256), 0, s, c.lat, nstates,
+                           npairs, nR, dv, dvx, shat.p, c.d_cells.p, c.inter.Q[0], c.inter.Q[1], c.inter.Q[2],
+                           out + nout * ip);
+        XATU_HIP(hipGetLastError());
+    }
+    std::vector<double> h_out(nout * nparams);
+    std::vector<double2> h_W(static_cast<size_t>(nstates) * na * na);
+    XATU_HIP(hipMemcpyAsync(h_out.data(), out, h_out.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+    if (exchange) XATU_HIP(hipMemcpyAsync(h_W.data(), Wx.p, Wx.bytes(), hipMemcpyDeviceToHost, s));
+    XATU_HIP(hipStreamSynchronize(s));
+    for (int ip = 0; ip < nparams; ++ip)
         for (int st = 0; st < nstates; ++st) {
             // direct: psi^H dD psi = (1/T) sum_p sum_R dV_p(R) Shat_p(R)
-            double dd = 0.0;
-            const double* sh = h_shat.data() + static_cast<size_t>(st) * npairs * nR;
-            for (size_t e = 0; e < static_cast<size_t>(npairs) * nR; ++e) dd += h_dv[e] * sh[e];
-            dd /= T;
+            const double dd = h_out[nout * ip + st] / T;
             // exchange: Re sum_ab dMQ_ab W_ab, with dMQ_ab = (1/T) sum_R dV_p(R) e^{iQR} (a < b),
             // dMQ_ba and dMQ_aa with e^{-iQR} (lower triangle and diagonal by conjugation)
             double dx = 0.0;
-            if (c.inter.exchange) {
-                const double2* W = Wx.data() + static_cast<size_t>(st) * na * na;
-                int p = 0;
+            if (exchange) {
+                const double2* W = h_W.data() + static_cast<size_t>(st) * na * na;
+                const double* m = h_out.data() + nout * ip + nstates;
                 for (int a = 0; a < na; ++a)
-                    for (int b = a; b < na; ++b, ++p) {
-                        double mr = 0.0, mi = 0.0;  // sum_R dV e^{iQR}
-                        for (int r = 0; r < nR; ++r) {
-                            const double* R = cellsR.data() + 3 * r;
-                            const double ph = c.inter.Q[0] * R[0] + c.inter.Q[1] * R[1] + c.inter.Q[2] * R[2];
-                            const double d = h_dvx[static_cast<size_t>(p) * nR + r];
-                            mr += d * std::cos(ph);
-                            mi += d * std::sin(ph);
-                        }
+                    for (int b = a; b < na; ++b, m += 2) {
                         if (a < b) {
                             const double2 wab = W[a + na * b], wba = W[b + na * a];
-                            dx += (mr * wab.x - mi * wab.y) + (mr * wba.x + mi * wba.y);
+                            dx += (m[0] * wab.x - m[1] * wab.y) + (m[0] * wba.x + m[1] * wba.y);
                         } else {
                             const double2 waa = W[a + na * a];
-                            dx += mr * waa.x + mi * waa.y;
+                            dx += m[0] * waa.x + m[1] * waa.y;
                         }
                     }
                 dx /= T;
             }
             grad_out[static_cast<size_t>(ip) * nstates + st] = -(dd - dx);
         }
-    }
 }
 
 }  // namespace xatu_dev

@@ -44,6 +44,7 @@
 #include "conv_rows.hpp"
 #include "cplx.hpp"
 #include "mfma.hpp"
+#include "wave_sums.hpp"
 
 #define XATU_FFT(call)                                                                                    \
     do {                                                                                                  \
@@ -58,7 +59,8 @@ namespace xatu_dev {
 
 namespace {
 
-constexpr int kScanRows = 256;
+constexpr int kScanRows = 64;   // rows of one block of the exchange scans: a wave
+constexpr int kScanWaves = 4;   // waves per workgroup of the scans
 
 // Layout of the correlation buffer G (batch entries b of M mesh points g = o0 + mesh_n o1).
 // Entry-major: G[b M + g]. Row-interleaved (2-D meshes): G[(o1 batch + b) mesh_n + o0],
@@ -438,97 +440,97 @@ void with_bands(const Context& c, Fn&& fn) {
 }
 
 // ---- exchange term along the upper triangle (FP64) ----
-// Block sums of A_a(i) = E2_a(i) x_i and B_a(i) = conj(E1_a(i)) x_i over kScanRows rows:
-// part[((blk NA + a) 2 + s) nvec + n]
-__global__ __launch_bounds__(kScanRows) void xscan_partial_kernel(int na, int ncv, const double2* __restrict__ e1,
-                                                                  const double2* __restrict__ e2,
-                                                                  const double2* __restrict__ X, int64_t N, int nvec,
-                                                                  double2* __restrict__ part) {
-    __shared__ double2 s[kScanRows];
-    const int n = blockIdx.y;
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kScanRows + threadIdx.x;
+// A block is the 64 rows of one wave, so that its sums and scans stay in registers (DPP) and need no
+// barrier; the price, four times as many blocks as with 256 rows, falls on the scan over the
+// blocks, which 64 threads share per series. N = 129600, 32 vectors, 4 atoms: sums, offsets and application
+// 109 + 127 + 169 -> 86 + 17 + 107 us (the vector units busy with the sums); N = 1875, 8 vectors: 7.5 + 5 + 10.6
+// -> 4.3 + 4.2 + 4.4 us.
+// Block sums of A_a(i) = E2_a(i) x_i and B_a(i) = conj(E1_a(i)) x_i:
+// part[((n nblk + blk) NA + a) 2 + s], a wave's values in one store; grid (workgroups, vectors)
+__global__ __launch_bounds__(64 * kScanWaves) void xscan_partial_kernel(int na, int ncv, const double2* __restrict__ e1,
+                                                                        const double2* __restrict__ e2,
+                                                                        const double2* __restrict__ X, int64_t N,
+                                                                        int nblk, double2* __restrict__ part) {
+    const int n = blockIdx.y, lane = threadIdx.x & 63;
+    const int64_t blk = static_cast<int64_t>(blockIdx.x) * kScanWaves + (threadIdx.x >> 6);
+    const int64_t i = blk * kScanRows + lane;
+    if (blk * kScanRows >= N) return;
     const bool ok = i < N;
     const double2 x = ok ? X[i + n * N] : mk(0.0, 0.0);
     const int64_t k = ok ? i / ncv : 0;
     const int cv = ok ? static_cast<int>(i % ncv) : 0;
+    double mr = 0.0, mi = 0.0;  // of the series that this lane stores
     for (int a = 0; a < na; ++a) {
-        for (int sidx = 0; sidx < 2; ++sidx) {
-            double2 v = mk(0.0, 0.0);
-            if (ok) {
-                const size_t off = (static_cast<size_t>(k) * na + a) * ncv + cv;
-                v = sidx == 0 ? cmul(e2[off], x) : cmul(cconj(e1[off]), x);
-            }
-            s[threadIdx.x] = v;
-            __syncthreads();
-            for (int st = kScanRows / 2; st > 0; st >>= 1) {
-                if (threadIdx.x < st) s[threadIdx.x] = cadd(s[threadIdx.x], s[threadIdx.x + st]);
-                __syncthreads();
-            }
-            if (threadIdx.x == 0) part[((static_cast<size_t>(blockIdx.x) * na + a) * 2 + sidx) * nvec + n] = s[0];
-            __syncthreads();
-        }
+        const size_t off = (static_cast<size_t>(k) * na + a) * ncv + cv;
+        const double2 va = cmul(e2[off], x), vb = cmul(cconj(e1[off]), x);
+        const double ar = wave_sum(va.x), ai = wave_sum(va.y), br = wave_sum(vb.x), bi = wave_sum(vb.y);
+        mr = lane == 2 * a ? ar : lane == 2 * a + 1 ? br : mr;
+        mi = lane == 2 * a ? ai : lane == 2 * a + 1 ? bi : mi;
     }
+    if (lane < 2 * na) part[(static_cast<size_t>(n) * nblk + blk) * 2 * na + lane] = mk(mr, mi);
 }
 
-// Exclusive prefix over blocks, in place, one thread per series (a, s, n); also the totals.
-__global__ void xscan_offsets_kernel(int nblk, int nseries, double2* __restrict__ part, double2* __restrict__ total) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nseries) return;
-    double2 run = mk(0.0, 0.0);
-    for (int b = 0; b < nblk; ++b) {
-        const size_t i = static_cast<size_t>(b) * nseries + t;
-        const double2 v = part[i];
-        part[i] = run;
-        run = cadd(run, v);
+// Exclusive prefix over the blocks, in place, and the totals. Series t = (n, a, s), ns of them per vector: a workgroup has 16 of them,
+// each shared by 64 threads with a run of blocks, whose sums are scanned in LDS. block 1024
+constexpr int kOffSeries = 16, kOffRuns = 64;
+__global__ __launch_bounds__(kOffSeries* kOffRuns) void xscan_offsets_kernel(int nblk, int nseries, int ns,
+                                                                             double2* __restrict__ part,
+                                                                             double2* __restrict__ total) {
+    __shared__ double2 s_run[kOffRuns][kOffSeries];
+    const int c = threadIdx.x % kOffSeries, q = threadIdx.x / kOffSeries;
+    const int t = blockIdx.x * kOffSeries + c;
+    const int run = (nblk + kOffRuns - 1) / kOffRuns, b0 = min(nblk, q * run), b1 = t < nseries ? min(nblk, b0 + run) : b0;
+    double2* p = part + (static_cast<size_t>(t / ns) * nblk) * ns + t % ns;
+    double2 sum = mk(0.0, 0.0);
+#pragma unroll 8
+    for (int b = b0; b < b1; ++b) sum = cadd(sum, p[static_cast<size_t>(b) * ns]);
+    s_run[q][c] = sum;
+    __syncthreads();
+    for (int d = 1; d < kOffRuns; d <<= 1) {
+        const double2 v = q >= d ? s_run[q - d][c] : mk(0.0, 0.0);
+        __syncthreads();
+        s_run[q][c] = cadd(s_run[q][c], v);
+        __syncthreads();
     }
-    total[t] = run;
+    double2 at = q > 0 ? s_run[q - 1][c] : mk(0.0, 0.0);
+    if (q == kOffRuns - 1 && t < nseries) total[t] = s_run[q][c];
+#pragma unroll 8
+    for (int b = b0; b < b1; ++b) {
+        const size_t i = static_cast<size_t>(b) * ns;
+        const double2 v = p[i];
+        p[i] = at;
+        at = cadd(at, v);
+    }
 }
 
 // y_i += sum_a [E1_a(i) (A_tot - sum_{j<=i} A_a(j)) + conj(E2_a(i)) sum_{j<i} B_a(j)] + Re(sum_a E1_a E2_a) x_i
-__global__ __launch_bounds__(kScanRows) void xscan_apply_kernel(int na, int ncv, const double2* __restrict__ e1,
-                                                                const double2* __restrict__ e2,
-                                                                const double2* __restrict__ X, int64_t N, int nvec,
-                                                                const double2* __restrict__ part,
-                                                                const double2* __restrict__ total,
-                                                                double2* __restrict__ Y) {
-    __shared__ double2 s[kScanRows];
-    const int n = blockIdx.y;
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kScanRows + threadIdx.x;
+__global__ __launch_bounds__(64 * kScanWaves) void xscan_apply_kernel(int na, int ncv, const double2* __restrict__ e1,
+                                                                      const double2* __restrict__ e2,
+                                                                      const double2* __restrict__ X, int64_t N, int nblk,
+                                                                      const double2* __restrict__ part,
+                                                                      const double2* __restrict__ total,
+                                                                      double2* __restrict__ Y) {
+    const int n = blockIdx.y, lane = threadIdx.x & 63;
+    const int64_t blk = static_cast<int64_t>(blockIdx.x) * kScanWaves + (threadIdx.x >> 6);
+    const int64_t i = blk * kScanRows + lane;
+    if (blk * kScanRows >= N) return;
     const bool ok = i < N;
     const double2 x = ok ? X[i + n * N] : mk(0.0, 0.0);
     const int64_t k = ok ? i / ncv : 0;
     const int cv = ok ? static_cast<int>(i % ncv) : 0;
-    const int nseries = na * 2 * nvec;
+    const double2* before = part + (static_cast<size_t>(n) * nblk + blk) * 2 * na;  // sums over earlier blocks
+    const double2* tot = total + static_cast<size_t>(n) * 2 * na;
     double2 y = mk(0.0, 0.0);
     double diag = 0.0;
     for (int a = 0; a < na; ++a) {
         const size_t off = (static_cast<size_t>(k) * na + a) * ncv + cv;
-        const double2 E1 = ok ? e1[off] : mk(0.0, 0.0);
-        const double2 E2 = ok ? e2[off] : mk(0.0, 0.0);
-        diag += E1.x * E2.x - E1.y * E2.y;
-        for (int sidx = 0; sidx < 2; ++sidx) {
-            const double2 v = sidx == 0 ? cmul(E2, x) : cmul(cconj(E1), x);
-            // inclusive scan within the block (Hillis-Steele, fixed order)
-            s[threadIdx.x] = v;
-            __syncthreads();
-            for (int st = 1; st < kScanRows; st <<= 1) {
-                const double2 add = threadIdx.x >= st ? s[threadIdx.x - st] : mk(0.0, 0.0);
-                __syncthreads();
-                s[threadIdx.x] = cadd(s[threadIdx.x], add);
-                __syncthreads();
-            }
-            const size_t ser = (static_cast<size_t>(a) * 2 + sidx) * nvec + n;
-            const double2 before = part[static_cast<size_t>(blockIdx.x) * nseries + ser];  // sum over earlier blocks
-            const double2 incl = cadd(before, s[threadIdx.x]);
-            if (sidx == 0) {
-                const double2 after = csub(total[ser], incl);  // sum_{j>i} A_a(j)
-                cfma(y, E1, after);
-            } else {
-                const double2 excl = csub(incl, v);            // sum_{j<i} B_a(j)
-                cfma(y, cconj(E2), excl);
-            }
-            __syncthreads();
-        }
+        const double2 E1 = e1[off], E2 = e2[off];
+        if (ok) diag += E1.x * E2.x - E1.y * E2.y;
+        const double2 va = cmul(E2, x), vb = cmul(cconj(E1), x);
+        const double2 A = cadd(before[2 * a], mk(wave_scan(va.x), wave_scan(va.y)));
+        const double2 B = cadd(before[2 * a + 1], mk(wave_scan(vb.x), wave_scan(vb.y)));
+        cfma(y, E1, csub(tot[2 * a], A));        // sum_{j>i} A_a(j)
+        cfma(y, cconj(E2), csub(B, vb));             // sum_{j<i} B_a(j)
     }
     if (ok) {
         double2 o = Y[i + n * N];
@@ -557,46 +559,32 @@ __global__ void power_sum_kernel(LatticeDesc lat, int ns, int64_t M, const doubl
 // Scans of the exchange adjoint, from the block sums of xscan_partial_kernel with x = psi:
 //   S_a(i) = 2 sum_{j>i} A_a(j) + A_a(i),  F_a(i) = conj(2 sum_{j<i} B_a(j) + B_a(i)),
 // A_a = E2_a psi, B_a = conj(E1_a) psi; S[(n NA + a) N + i] and F likewise. grid (blocks, nvec).
-__global__ __launch_bounds__(kScanRows) void xscan_adjoint_kernel(int na, int ncv, const double2* __restrict__ e1,
-                                                                  const double2* __restrict__ e2,
-                                                                  const double2* __restrict__ X, int64_t N, int nvec,
-                                                                  const double2* __restrict__ part,
-                                                                  const double2* __restrict__ total,
-                                                                  double2* __restrict__ S, double2* __restrict__ F) {
-    __shared__ double2 s[kScanRows];
-    const int n = blockIdx.y;
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kScanRows + threadIdx.x;
+__global__ __launch_bounds__(64 * kScanWaves) void xscan_adjoint_kernel(int na, int ncv, const double2* __restrict__ e1,
+                                                                        const double2* __restrict__ e2,
+                                                                        const double2* __restrict__ X, int64_t N,
+                                                                        int nblk, const double2* __restrict__ part,
+                                                                        const double2* __restrict__ total,
+                                                                        double2* __restrict__ S, double2* __restrict__ F) {
+    const int n = blockIdx.y, lane = threadIdx.x & 63;
+    const int64_t blk = static_cast<int64_t>(blockIdx.x) * kScanWaves + (threadIdx.x >> 6);
+    const int64_t i = blk * kScanRows + lane;
+    if (blk * kScanRows >= N) return;
     const bool ok = i < N;
     const double2 x = ok ? X[i + n * N] : mk(0.0, 0.0);
     const int64_t k = ok ? i / ncv : 0;
     const int cv = ok ? static_cast<int>(i % ncv) : 0;
-    const int nseries = na * 2 * nvec;
+    const double2* before = part + (static_cast<size_t>(n) * nblk + blk) * 2 * na;
+    const double2* tot = total + static_cast<size_t>(n) * 2 * na;
     for (int a = 0; a < na; ++a) {
         const size_t off = (static_cast<size_t>(k) * na + a) * ncv + cv;
-        for (int sidx = 0; sidx < 2; ++sidx) {
-            const double2 e = ok ? (sidx == 0 ? e2[off] : cconj(e1[off])) : mk(0.0, 0.0);
-            const double2 v = cmul(e, x);
-            s[threadIdx.x] = v;
-            __syncthreads();
-            for (int st = 1; st < kScanRows; st <<= 1) {
-                const double2 add = threadIdx.x >= st ? s[threadIdx.x - st] : mk(0.0, 0.0);
-                __syncthreads();
-                s[threadIdx.x] = cadd(s[threadIdx.x], add);
-                __syncthreads();
-            }
-            const size_t ser = (static_cast<size_t>(a) * 2 + sidx) * nvec + n;
-            const double2 incl = cadd(part[static_cast<size_t>(blockIdx.x) * nseries + ser], s[threadIdx.x]);
-            if (ok) {
-                const size_t out = (static_cast<size_t>(n) * na + a) * N + i;
-                if (sidx == 0) {
-                    const double2 after = csub(total[ser], incl);
-                    S[out] = mk(2.0 * after.x + v.x, 2.0 * after.y + v.y);
-                } else {
-                    const double2 before = csub(incl, v);
-                    F[out] = mk(2.0 * before.x + v.x, -(2.0 * before.y + v.y));
-                }
-            }
-            __syncthreads();
+        const double2 va = cmul(e2[off], x), vb = cmul(cconj(e1[off]), x);
+        const double2 A = cadd(before[2 * a], mk(wave_scan(va.x), wave_scan(va.y)));
+        const double2 B = cadd(before[2 * a + 1], mk(wave_scan(vb.x), wave_scan(vb.y)));
+        if (ok) {
+            const size_t out = (static_cast<size_t>(n) * na + a) * N + i;
+            const double2 after = csub(tot[2 * a], A), prior = csub(B, vb);
+            S[out] = mk(2.0 * after.x + va.x, 2.0 * after.y + va.y);
+            F[out] = mk(2.0 * prior.x + vb.x, -(2.0 * prior.y + vb.y));
         }
     }
 }
@@ -1068,19 +1056,21 @@ int rows_vectors(const Context& c, const ConvState& cs, int nvec) {
     return (nvec + passes - 1) / passes;
 }
 
+int scan_blocks(int64_t N) { return static_cast<int>((N + kScanRows - 1) / kScanRows); }
+
 // Block sums of the exchange scans of nv vectors, as offsets (cs.part) and totals; returns the
-// number of blocks.
+// number of workgroups for the blocks.
 int exchange_scans(Context& c, ConvState& cs, const double2* X, int nv, hipStream_t s) {
-    const int nblk = static_cast<int>((c.N + kScanRows - 1) / kScanRows);
+    const int nblk = scan_blocks(c.N), wgs = (nblk + kScanWaves - 1) / kScanWaves;
     const int nseries = c.lat.natoms * 2 * nv;
     cs.part.reserve(static_cast<size_t>(nblk) * nseries);
     cs.total.reserve(static_cast<size_t>(nseries));
-    hipLaunchKernelGGL(xscan_partial_kernel, dim3(nblk, nv), dim3(kScanRows), 0, s, c.lat.natoms, c.nc * c.nv, c.d_e1.p,
-                       c.d_e2.p, X, c.N, nv, cs.part.p);
-    hipLaunchKernelGGL(xscan_offsets_kernel, dim3((nseries + 255) / 256), dim3(256), 0, s, nblk, nseries, cs.part.p,
-                       cs.total.p);
+    hipLaunchKernelGGL(xscan_partial_kernel, dim3(wgs, nv), dim3(64 * kScanWaves), 0, s, c.lat.natoms, c.nc * c.nv,
+                       c.d_e1.p, c.d_e2.p, X, c.N, nblk, cs.part.p);
+    hipLaunchKernelGGL(xscan_offsets_kernel, dim3((nseries + kOffSeries - 1) / kOffSeries), dim3(kOffSeries * kOffRuns), 0,
+                       s, nblk, nseries, 2 * c.lat.natoms, cs.part.p, cs.total.p);
     XATU_HIP(hipGetLastError());
-    return nblk;
+    return wgs;
 }
 
 template <typename R>
@@ -1103,9 +1093,9 @@ void conv_product(Context& c, const double2* X, double2* Y, int nvec, hipStream_
         double2* Yb = Y + static_cast<int64_t>(v0) * N;
         const int na = c.lat.natoms;
         const int ncv = c.nc * c.nv;
-        const int nblk = exchange_scans(c, cs, Xb, nv, s);
-        hipLaunchKernelGGL(xscan_apply_kernel, dim3(nblk, nv), dim3(kScanRows), 0, s, na, ncv, c.d_e1.p, c.d_e2.p, Xb, N,
-                           nv, cs.part.p, cs.total.p, Yb);
+        const int wgs = exchange_scans(c, cs, Xb, nv, s);
+        hipLaunchKernelGGL(xscan_apply_kernel, dim3(wgs, nv), dim3(64 * kScanWaves), 0, s, na, ncv, c.d_e1.p, c.d_e2.p, Xb, N,
+                           scan_blocks(N), cs.part.p, cs.total.p, Yb);
         XATU_HIP(hipGetLastError());
     }
 }
@@ -1173,11 +1163,11 @@ void conv_band_adjoint(Context& c, const double2* psi, int ns, double2* g) {
         launch_rows_out<double>(a1, c.nc, parts, cs.d_kmap.p, c.d_twiddle.p, b.Ct, b.G.p, b.T.p, s);
         launch_rows_out<double>(a2, c.nv, parts, cs.d_kmap.p, c.d_twiddle.p, b.Vt, b.G.p, cs.T64b.p, s);
         if (c.inter.exchange) {
-            const int nblk = exchange_scans(c, cs, X, nv, s);
+            const int wgs = exchange_scans(c, cs, X, nv, s);
             cs.S.reserve(static_cast<size_t>(nv) * na * c.N);
             cs.F.reserve(static_cast<size_t>(nv) * na * c.N);
-            hipLaunchKernelGGL(xscan_adjoint_kernel, dim3(nblk, nv), dim3(kScanRows), 0, s, na, c.nc * c.nv, c.d_e1.p,
-                               c.d_e2.p, X, c.N, nv, cs.part.p, cs.total.p, cs.S.p, cs.F.p);
+            hipLaunchKernelGGL(xscan_adjoint_kernel, dim3(wgs, nv), dim3(64 * kScanWaves), 0, s, na, c.nc * c.nv, c.d_e1.p,
+                               c.d_e2.p, X, c.N, scan_blocks(c.N), cs.part.p, cs.total.p, cs.S.p, cs.F.p);
         }
         hipLaunchKernelGGL(band_adjoint_kernel, dim3((static_cast<size_t>(c.nk) * norb + 255) / 256, nv), dim3(256), 0, s,
                            c.lat, c.nk, c.nv, c.nc, nv, parts, parts, b.Ct, b.Vt, X, c.N, b.T.p, cs.T64b.p,

@@ -59,4 +59,16 @@ __device__ inline T wave_sum_groups8(T x) {
 template <typename T>
 __device__ inline T wave_sum(T x) { return wave_sum_groups8(sum8(x)); }
 
+// Inclusive prefix sum over the lanes of the wave (shifts by 1, 2, 4 and 8 within the rows of 16, then
+// the rows' ends broadcast).
+__device__ inline double wave_scan(double x) {
+    x += dpp<0x111>(x);
+    x += dpp<0x112>(x);
+    x += dpp<0x114>(x);
+    x += dpp<0x118>(x);
+    x += dpp<kDppBcast15, 0xA>(x);
+    x += dpp<kDppBcast31, 0xC>(x);
+    return x;
+}
+
 }  // namespace xatu_dev

@@ -530,43 +530,43 @@ __global__ __launch_bounds__(col_group(A, B) * B) void conv_columns_kernel(Latti
         }
         return;
     } else {
-    C v[B];
-    if (s < A) {
-#pragma unroll
-        for (int i = 0; i < B; ++i) v[i] = ex[(i * A + s) * T + c];
-        dft_len<R, B, -1>(v);
-        if constexpr (SPECTRUM) {
-            const R* p = spectrum_of(lat, W, nvec, live ? u : count - 1, n, P);
-#pragma unroll
-            for (int k = 0; k < B; ++k) {
-                const R q = p[static_cast<int64_t>(s + A * k) * W];
-                v[k].x *= q;
-                v[k].y *= q;
-            }
-            dft_len<R, B, 1>(v);
-#pragma unroll
-            for (int i = 1; i < B; ++i) v[i] = cmul(v[i], cconj(tw[i * s]));
-        } else if (live) {
-#pragma unroll
-            for (int k = 0; k < B; ++k) g[static_cast<int64_t>(s + A * k) * count] = v[k];
-        }
-    }
-    if constexpr (SPECTRUM) {
-        // a lane writes the slots that it read itself
+        C v[B];
         if (s < A) {
 #pragma unroll
-            for (int i = 0; i < B; ++i) ex[(i * A + s) * T + c] = v[i];
-        }
-        __syncthreads();
-        C w[A];
+            for (int i = 0; i < B; ++i) v[i] = ex[(i * A + s) * T + c];
+            dft_len<R, B, -1>(v);
+            if constexpr (SPECTRUM) {
+                const R* p = spectrum_of(lat, W, nvec, live ? u : count - 1, n, P);
 #pragma unroll
-        for (int k = 0; k < A; ++k) w[k] = ex[(s * A + k) * T + c];
-        dft_len<R, A, 1>(w);
-        if (live) {
+                for (int k = 0; k < B; ++k) {
+                    const R q = p[static_cast<int64_t>(s + A * k) * W];
+                    v[k].x *= q;
+                    v[k].y *= q;
+                }
+                dft_len<R, B, 1>(v);
 #pragma unroll
-            for (int j = 0; j < A; ++j) g[static_cast<int64_t>(B * j + s) * count] = w[j];
+                for (int i = 1; i < B; ++i) v[i] = cmul(v[i], cconj(tw[i * s]));
+            } else if (live) {
+#pragma unroll
+                for (int k = 0; k < B; ++k) g[static_cast<int64_t>(s + A * k) * count] = v[k];
+            }
         }
-    }
+        if constexpr (SPECTRUM) {
+            // a lane writes the slots that it read itself
+            if (s < A) {
+#pragma unroll
+                for (int i = 0; i < B; ++i) ex[(i * A + s) * T + c] = v[i];
+            }
+            __syncthreads();
+            C w[A];
+#pragma unroll
+            for (int k = 0; k < A; ++k) w[k] = ex[(s * A + k) * T + c];
+            dft_len<R, A, 1>(w);
+            if (live) {
+#pragma unroll
+                for (int j = 0; j < A; ++j) g[static_cast<int64_t>(B * j + s) * count] = w[j];
+            }
+        }
     }
 }
 

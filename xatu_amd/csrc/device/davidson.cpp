@@ -90,10 +90,6 @@ public:
         ws_.Y.reserve(static_cast<size_t>(mmax_) * b_);
         ws_.theta.reserve(b_);
         T_.assign(static_cast<size_t>(mmax_) * mmax_, cd(0.0, 0.0));
-        c_.h_proj.reserve(static_cast<size_t>(mmax_) * b_);
-        c_.h_coef.reserve(static_cast<size_t>(mmax_) * b_);
-        c_.h_whiten.reserve_mapped(static_cast<size_t>(b_) * b_);
-        c_.h_theta.reserve(b_);
         dev_rr_ = mmax_ <= projected_eigen_max_dim() && b_ <= projected_eigen_max_want();
         if (dev_rr_) {
             const int md = projected_eigen_max_dim();
@@ -114,6 +110,9 @@ public:
             ws_.R.reserve(static_cast<size_t>(N_) * b_);
             ws_.partial.reserve(static_cast<size_t>(b_) * ((N_ + 255) / 256));
             c_.h_part.reserve(static_cast<size_t>(b_) * ((N_ + 255) / 256));
+            c_.h_coef.reserve(static_cast<size_t>(mmax_) * b_);
+            c_.h_theta.reserve(b_);
+            reserve_pinned();
         }
     }
 
@@ -179,6 +178,14 @@ public:
     double projections_ms() const { return proj_ms_; }
 
 private:
+    // Pinned staging of the block's Gram matrix and its whitening on the host: the host
+    // Rayleigh-Ritz path and blocks that the device could not whiten (allocating pinned memory
+    // at every new context cost its first solve up to a millisecond).
+    void reserve_pinned() {
+        c_.h_proj.reserve(static_cast<size_t>(mmax_) * b_);
+        c_.h_whiten.reserve_mapped(static_cast<size_t>(b_) * b_);
+    }
+
     // One wait per iteration: Rayleigh-Ritz on the device, Ritz block, residuals,
     // preconditioned corrections (restart when the basis is full), their orthogonalisation and
     // whitening; the residual norms, the Ritz values and the times of the phases arrive from the
@@ -252,6 +259,7 @@ private:
             if (nb <= 0) return false;
             int kept = nb;
             if (!got[2 * kStepMaxBlock + kStamps]) {
+                reserve_pinned();
                 XATU_HIP(hipMemcpyAsync(c_.h_proj.p, ws_.P.p, static_cast<size_t>(mn) * nb * sizeof(cd),
                                         hipMemcpyDeviceToHost, c_.stream));
                 XATU_HIP(hipStreamSynchronize(c_.stream));
@@ -414,6 +422,7 @@ private:
     // dropping dependent directions. An ill-conditioned block (kept eigenvalues spanning
     // more than 1e8) repeats the whole procedure once on the whitened vectors.
     int orthonormalise_slot(int nb, int round = 0) {
+        reserve_pinned();
         const int n = static_cast<int>(N_);
         const int mn = m_ + nb;
         double2* T = ws_.V.p + static_cast<size_t>(m_) * N_;

@@ -746,14 +746,17 @@ struct ConvState {
         void* work = nullptr;
     };
     std::map<std::tuple<int, int, int>, Plan> plans;  // (bytes per real, batch, row-interleaved)
-    ~ConvState() {
+    int plan_ndim = 0, plan_side = 0;  // the mesh that the plans are for
+    void drop_plans() {
         for (auto& kv : plans) {
             for (rocfft_plan q : {kv.second.fwd, kv.second.bwd, kv.second.fwd2, kv.second.bwd2})
                 if (q) rocfft_plan_destroy(q);
             if (kv.second.info) rocfft_execution_info_destroy(kv.second.info);
             if (kv.second.work) (void)hipFree(kv.second.work);
         }
+        plans.clear();
     }
+    ~ConvState() { drop_plans(); }
 };
 
 void destroy_conv_state(ConvState* s) { delete s; }
@@ -839,6 +842,13 @@ void ensure_conv(Context& c) {
     const int64_t M = c.lat.nmesh;
     cs.M = M;
     const int m = c.lat.mesh_n;
+    if (cs.plan_ndim != c.lat.ndim || cs.plan_side != m) {
+        // the lattice was set again: plans of another mesh have other lengths
+        if (!cs.plans.empty()) XATU_HIP(hipStreamSynchronize(c.stream));
+        cs.drop_plans();
+        cs.plan_ndim = c.lat.ndim;
+        cs.plan_side = m;
+    }
     const int norb = c.lat.norb;
     const int na2 = c.lat.natoms * c.lat.natoms;
     std::vector<int> gk(c.nk), kmap(M, -1);

@@ -335,10 +335,10 @@ __global__ void reciprocal_table_kernel(LatticeDesc lat, const double* __restric
     if (a != b) ft[base + b + static_cast<size_t>(lat.natoms) * a] = make_double2(m.x, -m.y);
 }
 
-// M_ab(Q) for the exchange term. grid: 1; block: 64 (npairs <= 36)
+// M_ab(Q) for the exchange term, a thread per pair. grid: ceil(npairs / 64); block: 64
 __global__ void reciprocal_q_kernel(LatticeDesc lat, const double* __restrict__ gvec, int ng, RecipDesc rd, int npairs,
                                     double qx, double qy, double qz, double2* __restrict__ ftq) {
-    const int p = threadIdx.x;
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= npairs) return;
     int a, b;
     pair_of(p, lat.natoms, a, b);
@@ -361,7 +361,7 @@ void launch_reciprocal_table(const Context& c, const double* d_gvec, int ng, dou
     hipLaunchKernelGGL(reciprocal_table_kernel, grid, dim3(256), 0, s, c.lat, d_gvec, ng, rd, npairs, c.d_ft.p);
     XATU_HIP(hipGetLastError());
     if (c.inter.exchange) {
-        hipLaunchKernelGGL(reciprocal_q_kernel, dim3(1), dim3(64), 0, s, c.lat, d_gvec, ng, rd, npairs, c.inter.Q[0],
+        hipLaunchKernelGGL(reciprocal_q_kernel, dim3((npairs + 63) / 64), dim3(64), 0, s, c.lat, d_gvec, ng, rd, npairs, c.inter.Q[0],
                            c.inter.Q[1], c.inter.Q[2], c.d_ftq.p);
         XATU_HIP(hipGetLastError());
     }

@@ -39,6 +39,7 @@
 
 #include "../common/heev.hpp"
 #include "context.hpp"
+#include "refinement.hpp"
 #include "solver_step.hpp"
 
 namespace xatu_dev {
@@ -648,24 +649,14 @@ void solve_davidson(Context& c, const xatu_solve_options& opt, double* eigval_ou
         const int it32 = rep->iterations;
         // ... then FP64 refinement from the lowest Ritz vectors, with FP64 products
         // (matrix-free when no FP64 matrix is resident), until the FP64 residuals meet tol.
-        // Block: nev and some guard vectors, because the highest state wanted converges with its
-        // distance from the first state outside the block, which may be next to nothing (a block
-        // of nev took 64 iterations, 99 ms, where two guard vectors took 14, 47 ms: N = 36864, nev
-        // = 16; the whole FP32 block, twice nev, 53 ms). max(2, nev / 4) against none, N = 1875 to 36864, nev = 2 to
-        // 16, several spectra each: 0.38 to 1.05 of the time. None where the product recomputes tiles or takes the slower
-        // transforms over the whole mesh (sides without a factor pair), which cost up to 1.4 with them
-        // when the spectrum has its gap (142 x 142, nev = 5: 44 -> 63 ms). A resident FP64 matrix is multiplied by whole tiles of
-        // 16 vectors: the guard fills the last one. Basis 6 blocks up to the device
-        // Rayleigh-Ritz limit (4 blocks: up to 1.2 of the time).
+        // Block and basis: refinement.hpp.
         const int form = opt.matrix_free ? opt.matrix_free : (c.built64 ? 0 : XATU_MATRIX_FREE_CONV);
         const bool resident = form == 0;
         const bool rows = !resident && form != XATU_MATRIX_FREE_TILES && !c.lat.recip && c.lat.ndim == 2 &&
                           conv_rows_available(c);
-        const int guard = resident || rows ? std::max(2, nev / 4) : 0;
-        const int bref = std::min({b, nev + guard, resident ? (nev + 15) / 16 * 16 : b});
-        const int mref = static_cast<int>(std::min<int64_t>(
-            N, std::max({4 * bref, std::min(6 * bref, projected_eigen_max_dim()), bref + 1})));
-        dav = std::make_unique<Davidson>(c, c.solver_ws[0], XATU_FP64, form, nev, bref, mref, rep);
+        const RefinementShape ref =
+            refinement_shape(N, nev, b, resident, rows, projected_eigen_max_want(), projected_eigen_max_dim());
+        dav = std::make_unique<Davidson>(c, c.solver_ws[0], XATU_FP64, form, nev, ref.block, ref.basis, rep);
         dav->init_from(d32->ritz_vectors());
         ok = dav->run(tol, maxit);
         rep->refine_iterations = rep->iterations - it32;

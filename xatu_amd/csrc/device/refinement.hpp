@@ -19,9 +19,9 @@ struct RefinementShape {
 // against none, N = 1875 to 36864, nev = 2 to 16, several spectra each: 0.38 to 1.05 of the time. None where the
 // product recomputes tiles or takes the slower transforms over the whole mesh (sides without a factor pair),
 // which cost up to 1.4 with them when the spectrum has its gap (142 x 142, nev = 5: 44 -> 63 ms). A resident FP64
-matrix is multiplied by whole tiles of 16 vectors: the guard fills the last one and does not begin another
-// (four guard vectors at nev = 16, N = 2500 to 36864, four spectra each: 0.42 to 1.12 of the time, most often
-// longer; three at nev = 15 instead of one 0.94 to 1.21). Never so many that a block which fits the device
+// matrix is multiplied by whole tiles of 16 vectors: the guard fills the last one and does not begin another
+// (four guard vectors at nev = 16, N = 2500 to 36864, four spectra each: 0.42 to 1.12 of the time, longer in
+// half of them; three at nev = 15 instead of one 0.94 to 1.21). Never so many that a block which fits the device
 // Rayleigh-Ritz kernel no longer does: past it an iteration waits for the host three times (nev = 27 to 32, N =
 // 2500 and 9216, two spectra each: 1.02 to 1.39 times as long with all the guard vectors).
 // Basis: 6 blocks up to that kernel's limit (4 blocks: up to 1.2 of the time).

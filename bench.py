@@ -296,7 +296,7 @@ def main():
                              "projections": round(rep.ms_projections, 2),
                              "iterations": rep.iterations, "refine_iterations": rep.refine_iterations}
     # Roofline of the dominant kernel of the mixed step: the product with the FP32 matrix
-    # (staging, product and reduction kernels, timed by the device clock values the kernels around them leave).
+    # (staging, product and reduction kernels, from the device clock at the start of the first to that at the start of the next).
     # With N even it runs on the FP16 matrix cores with split operands and reads only the
     # block-lower half of the Hermitian matrix; its algorithmic bytes are the N(N+1)/2
     # distinct complex entries (8 bytes each). Otherwise the full matrix on the FP32 matrix

@@ -965,7 +965,7 @@ struct Shape {
         yp.alloc(std::max<size_t>(yp.n, static_cast<size_t>(splits) * c.N * kBlockVectors));
         for (int v0 = 0; v0 < nvec; v0 += kBlockVectors) {
             const int nv = std::min(kBlockVectors, nvec - v0);
-            launch_stage_vectors(X + static_cast<int64_t>(v0) * c.N, c.N, nv, xt.p, s);
+            launch_stage_vectors(X + static_cast<int64_t>(v0) * c.N, c.N, nv, xt.p, c.take_product_stamp(), s);
             hipLaunchKernelGGL((bse_matfree_kernel<R, NA, NC, NV, TK>), dim3(nT * splits), dim3(matfree_threads(TK)),
                                lds, s, c.lat, c.nk, c.d_evec_k.p, c.d_evec_kq.p, c.d_eval_k.p, c.d_eval_kq.p,
                                c.d_kcoord.p, c.d_ft.p, c.d_e1.p, c.d_e2.p, c.inter.exchange, c.scissor, xt.p, nv,
@@ -1054,7 +1054,7 @@ void matfree_generic(Context& c, const double2* X, double2* Y, int nvec, hipStre
     yp.alloc(std::max<size_t>(yp.n, static_cast<size_t>(splits) * c.N * kBlockVectors));
     for (int v0 = 0; v0 < nvec; v0 += kBlockVectors) {
         const int nv = std::min(kBlockVectors, nvec - v0);
-        launch_stage_vectors(X + static_cast<int64_t>(v0) * c.N, c.N, nv, xt.p, s);
+        launch_stage_vectors(X + static_cast<int64_t>(v0) * c.N, c.N, nv, xt.p, c.take_product_stamp(), s);
         hipLaunchKernelGGL((bse_matfree_generic_kernel<R>), dim3(nT * splits), dim3(256), 0, s, c.lat, c.nk, c.nv,
                            c.nc, c.d_evec_k.p, c.d_evec_kq.p, c.d_eval_k.p, c.d_eval_kq.p, c.d_kcoord.p, c.d_ft.p,
                            c.d_e1.p, c.d_e2.p, c.inter.exchange, c.scissor, xt.p, nv, splits, tiles_per_split, yp.p);

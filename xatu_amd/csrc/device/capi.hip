@@ -240,8 +240,10 @@ void prepare_operator(Context& c) {
 namespace xatu_dev {
 
 // Product with the resident matrix of the given precision (or matrix-free), launched
-// on the context stream without waiting.
-void launch_operator(Context& c, int precision, int matrix_free, const double2* X, double2* Y, int nvec) {
+// on the context stream without waiting; stamp: the device clock when its first kernel starts.
+void launch_operator(Context& c, int precision, int matrix_free, const double2* X, double2* Y, int nvec,
+                     unsigned long long* stamp) {
+    c.product_stamp = stamp;
     if (matrix_free) {
         if (!c.prepared) throw Error(XATU_ERR_LOGIC, "operator not prepared (call xatu_build_bse)");
         // the convolution form needs a table periodic on the mesh: the reciprocal-space

@@ -8,6 +8,7 @@
 #include <stdexcept>
 #include <memory>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../../include/xatu_bse.h"
@@ -241,6 +242,9 @@ struct Context {
     HostBuf<double> h_theta, h_part;
     HostBuf<StepReport> h_step;  // mapped: the per-iteration results of the device solver
     unsigned long long step_sequence = 0;  // of the last report asked for
+    // where the next product leaves the device clock at its start (null: nowhere); its first kernel takes it
+    unsigned long long* product_stamp = nullptr;
+    unsigned long long* take_product_stamp() { return std::exchange(product_stamp, nullptr); }
     // solver workspaces, kept (grow only) between solves: [0] the FP64 solve or refinement,
     // [1] the FP32 phase of the mixed form, which both exist during a mixed solve
     SolverWorkspace solver_ws[2];
@@ -369,8 +373,8 @@ void launch_matfree64(Context& c, const double2* X, double2* Y, int nvec, hipStr
 void launch_matfree32(Context& c, const double2* X, double2* Y, int nvec, hipStream_t s);
 // Vector blocks of the products: Xt[row][32] (zero padded beyond nvec <= 32) in the
 // product's precision, and the fixed-order sum Y[row + n N] = sum_s Yp[s][row][n].
-void launch_stage_vectors(const double2* X, int64_t N, int nvec, double2* Xt, hipStream_t s);
-void launch_stage_vectors(const double2* X, int64_t N, int nvec, float2* Xt, hipStream_t s);
+void launch_stage_vectors(const double2* X, int64_t N, int nvec, double2* Xt, unsigned long long* stamp, hipStream_t s);
+void launch_stage_vectors(const double2* X, int64_t N, int nvec, float2* Xt, unsigned long long* stamp, hipStream_t s);
 // C (N x nb) = alpha A B + beta C, A: N x m (lda), B: m x nb (ldb), FP64 complex, in
 // launches of 32 columns; beta = 0 does not read C. C must not overlap A or B.
 void launch_block_gemm(const double2* A, int lda, const double2* B, int ldb, int64_t N, int m, int nb, double alpha,
@@ -384,7 +388,8 @@ void solve_davidson(Context& c, const xatu_solve_options& opt, double* eigval_ou
                     xatu_solve_report* rep);
 void apply_operator(Context& c, int precision, int matrix_free, const double2* X, double2* Y, int nvec,
                     double* ms_kernel);
-void launch_operator(Context& c, int precision, int matrix_free, const double2* X, double2* Y, int nvec);
+void launch_operator(Context& c, int precision, int matrix_free, const double2* X, double2* Y, int nvec,
+                     unsigned long long* stamp = nullptr);
 void record_product(Context& c, int matrix_free, double ms, int nvec);
 
 // Hellmann-Feynman gradients (hf.hip / capi.cpp).

@@ -175,10 +175,12 @@ template <typename R>
 constexpr int conv_y_be_block() { return sizeof(R) == 8 ? 6 : 12; }
 
 // u[((n NC + c) norb + be) nk + k] = sum_v conj(V_k[be, v]) x[k NCV + c NV + v, n]
-// thread per k, blockIdx.y = group of vectors
+// thread per k, blockIdx.y = group of vectors; the device clock to stamp, if any
 template <typename R, int NC, int NV>
 __global__ __launch_bounds__(256) void conv_u_kernel(int nk, int norb, int nvec, const cx_t<R>* __restrict__ Vt,
-                                                     const double2* __restrict__ X, int64_t N, cx_t<R>* __restrict__ U) {
+                                                     const double2* __restrict__ X, int64_t N, cx_t<R>* __restrict__ U,
+                                                     unsigned long long* __restrict__ stamp) {
+    if (stamp && blockIdx.x + blockIdx.y == 0 && threadIdx.x == 0) *stamp = wall_clock64();
     constexpr int VG = conv_vec_group<R>();
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     const int n0 = blockIdx.y * VG;
@@ -959,9 +961,11 @@ void conv_bands_in(Context& c, ConvBuffers<R>& b, const double2* X, int nv, hipS
     b.U.reserve(static_cast<size_t>(nv) * c.nc * norb * c.nk);
     const unsigned kb = (c.nk + 255) / 256;
     const int vg = (nv + conv_vec_group<R>() - 1) / conv_vec_group<R>();
+    unsigned long long* stamp = c.take_product_stamp();
     with_bands<R>(c, [&](auto ncc, auto nvc) {
         constexpr int NC = decltype(ncc)::value, NV = decltype(nvc)::value;
-        hipLaunchKernelGGL((conv_u_kernel<R, NC, NV>), dim3(kb, vg), dim3(256), 0, s, c.nk, norb, nv, b.Vt, X, c.N, b.U.p);
+        hipLaunchKernelGGL((conv_u_kernel<R, NC, NV>), dim3(kb, vg), dim3(256), 0, s, c.nk, norb, nv, b.Vt, X, c.N, b.U.p,
+                           stamp);
     });
     XATU_HIP(hipGetLastError());
 }
@@ -1029,8 +1033,8 @@ void conv_mesh_product(Context& c, ConvState& cs, ConvBuffers<R>& b, const doubl
     const GLayout lay = inter ? GLayout{c.lat.mesh_n, c.lat.mesh_n, static_cast<int64_t>(batch) * c.lat.mesh_n}
                               : GLayout{M, 0, 0};
     b.G.reserve(static_cast<size_t>(batch) * M);
-    if (!cs.full) XATU_HIP(hipMemsetAsync(b.G.p, 0, static_cast<size_t>(batch) * M * sizeof(cx_t<R>), s));
     conv_bands_in<R>(c, b, X, nv, s);
+    if (!cs.full) XATU_HIP(hipMemsetAsync(b.G.p, 0, static_cast<size_t>(batch) * M * sizeof(cx_t<R>), s));
     const dim3 kb((c.nk + 255) / 256);
     with_bands<R>(c, [&](auto ncc, auto nvc) {
         constexpr int NC = decltype(ncc)::value, NV = decltype(nvc)::value;
@@ -1210,7 +1214,7 @@ void conv_pair_density(Context& c, const double2* psi, int ns, double2* S) {
         constexpr int NC = decltype(ncc)::value, NV = decltype(nvc)::value;
         constexpr int VG = conv_vec_group<double>();
         hipLaunchKernelGGL((conv_u_kernel<double, NC, NV>), dim3(kb.x, (ns + VG - 1) / VG), dim3(256), 0, s, c.nk, norb,
-                           ns, cs.Vt64.p, psi, N, cs.U64.p);
+                           ns, cs.Vt64.p, psi, N, cs.U64.p, nullptr);
         hipLaunchKernelGGL((conv_z_kernel<double, NC>), dim3(kb.x, (norb + conv_orb_group<double>() - 1) / conv_orb_group<double>(), ns),
                            dim3(256), 0, s, c.nk, norb, ns, GLayout{M, 0, 0}, cs.d_gk.p, cs.Ct64.p, cs.U64.p,
                            cs.G64.p);

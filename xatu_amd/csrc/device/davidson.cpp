@@ -132,7 +132,6 @@ public:
         XATU_HIP(hipMemsetAsync(ws_.V.p, 0, static_cast<size_t>(N_) * b_ * sizeof(double2), c_.stream));
         launch_unit_vectors(d_idx.p, N_, b_, ws_.V.p, c_.stream);
         m_ = 0;
-        if (dev_rr_) launch_stamp(ws_.stamps.p + kStampProduct, c_.stream);
         append_block(b_);
         XATU_HIP(hipStreamSynchronize(c_.stream));
     }
@@ -145,7 +144,6 @@ public:
         m_ = 0;
         const int kept = orthonormalise_slot(b_);
         if (kept < b_) throw Error(XATU_ERR_NOT_CONVERGED, "Davidson: the refinement's starting block is rank deficient");
-        if (dev_rr_) launch_stamp(ws_.stamps.p + kStampProduct, c_.stream);
         append_block(b_);
     }
 
@@ -241,7 +239,6 @@ private:
             w.theta = ws_.theta.p;
             w.norm2 = ws_.norm2.p;
             w.stamps = ws_.stamps.p;
-            w.product_stamp = ws_.stamps.p + kStampProduct;
             w.host = c_.h_step.dev;
             w.sequence = ++c_.step_sequence;
             launch_whiten(w, c_.stream);
@@ -266,7 +263,6 @@ private:
                 XATU_HIP(hipStreamSynchronize(c_.stream));
                 kept = ortho_whiten(nb, 0);
                 if (kept == 0) return false;
-                launch_stamp(ws_.stamps.p + kStampProduct, c_.stream);
             }
             append_block(kept);
         }
@@ -328,7 +324,7 @@ private:
         double2* Vn = ws_.V.p + static_cast<size_t>(m_) * N_;
         double2* Wn = ws_.W.p + static_cast<size_t>(m_) * N_;
         if (dev_rr_) {
-            launch_operator(c_, prec_, mf_, Vn, Wn, nb);
+            launch_operator(c_, prec_, mf_, Vn, Wn, nb, ws_.stamps.p + kStampProduct);
             rep_->products += nb;
             launch_gram_extend(c_, ws_.V.p, Wn, N_, m_, nb, ws_.Tm.p, mmax_, ws_.stamps.p, c_.stream);
             last_nb_ = nb;

@@ -26,9 +26,11 @@ namespace {
 
 constexpr int kVec = kBlockVectors;
 
-// Xt[j][n] = X[j + n N] for n < nvec, 0 otherwise (j < N, n < VT).
+// Xt[j][n] = X[j + n N] for n < nvec, 0 otherwise (j < N, n < VT); the device clock to stamp, if any.
 template <typename Rin, typename R, int VT>
-__global__ void stage_vectors_kernel(const cx_t<Rin>* __restrict__ X, int64_t N, int nvec, cx_t<R>* __restrict__ Xt) {
+__global__ void stage_vectors_kernel(const cx_t<Rin>* __restrict__ X, int64_t N, int nvec, cx_t<R>* __restrict__ Xt,
+                                     unsigned long long* __restrict__ stamp) {
+    if (stamp && blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
     const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (idx >= N * VT) return;
     const int64_t j = idx / VT;
@@ -495,7 +497,7 @@ int product_splits(int64_t N, int vt, int max_splits) {
 // sums yp (splits x N x 16 UT).
 template <typename Rin, typename R, typename Rout, int UT>
 void dense_product_tile(int64_t N, const cx_t<R>* H, const cx_t<Rin>* X, cx_t<Rout>* Y, int nv, hipStream_t s,
-                        cx_t<R>* xt, cx_t<R>* yp, int splits) {
+                        cx_t<R>* xt, cx_t<R>* yp, int splits, unsigned long long* stamp) {
     using T = ProductTiling<R>;
     constexpr int VT = 16 * UT;
     const int rows_wg = 64 * T::TW;
@@ -504,7 +506,8 @@ void dense_product_tile(int64_t N, const cx_t<R>* H, const cx_t<Rin>* X, cx_t<Ro
     const int64_t kchunk = ((N + splits - 1) / splits + step - 1) / step * step;
     // every split owns a (possibly empty) column range and writes its partial rows
     const int64_t tot = N * VT;
-    hipLaunchKernelGGL((stage_vectors_kernel<Rin, R, VT>), dim3((tot + 255) / 256), dim3(256), 0, s, X, N, nv, xt);
+    hipLaunchKernelGGL((stage_vectors_kernel<Rin, R, VT>), dim3((tot + 255) / 256), dim3(256), 0, s, X, N, nv, xt,
+                       stamp);
     hipLaunchKernelGGL((dense_product_kernel<R, UT>), dim3(row_blocks * splits), dim3(256), 0, s, H, xt, N, kchunk,
                        splits, yp);
     hipLaunchKernelGGL((reduce_product_kernel<R, Rout, VT>), dim3((tot + 255) / 256), dim3(256), 0, s, yp, N, nv,
@@ -514,21 +517,22 @@ void dense_product_tile(int64_t N, const cx_t<R>* H, const cx_t<Rin>* X, cx_t<Ro
 // max_splits: what the partial-sum buffer holds for 32 vectors per row.
 template <typename Rin, typename R, typename Rout>
 void dense_product_into(int64_t N, const cx_t<R>* H, const cx_t<Rin>* X, cx_t<Rout>* Y, int nvec, hipStream_t s,
-                        cx_t<R>* xt, cx_t<R>* yp, int max_splits) {
+                        cx_t<R>* xt, cx_t<R>* yp, int max_splits, unsigned long long* stamp) {
     for (int v0 = 0; v0 < nvec; v0 += kVec) {
         const int nv = std::min(kVec, nvec - v0);
         const int vt = vector_tile(nv);
         const int splits = product_splits<R>(N, vt, max_splits);
         if (vt == 16)
-            dense_product_tile<Rin, R, Rout, 1>(N, H, X + v0 * N, Y + v0 * N, nv, s, xt, yp, splits);
+            dense_product_tile<Rin, R, Rout, 1>(N, H, X + v0 * N, Y + v0 * N, nv, s, xt, yp, splits, stamp);
         else
-            dense_product_tile<Rin, R, Rout, 2>(N, H, X + v0 * N, Y + v0 * N, nv, s, xt, yp, splits);
+            dense_product_tile<Rin, R, Rout, 2>(N, H, X + v0 * N, Y + v0 * N, nv, s, xt, yp, splits, stamp);
+        stamp = nullptr;
     }
     XATU_HIP(hipGetLastError());
 }
 
 template <typename Rin, typename R, typename Rout>
-void dense_product(const Context& c, const cx_t<R>* H, const cx_t<Rin>* X, cx_t<Rout>* Y, int nvec, hipStream_t s,
+void dense_product(Context& c, const cx_t<R>* H, const cx_t<Rin>* X, cx_t<Rout>* Y, int nvec, hipStream_t s,
                    DevBuf<cx_t<R>>& xt, DevBuf<cx_t<R>>& yp) {
     const int64_t N = c.N;
     size_t room = 0;  // partial sums of the largest vector block of the call
@@ -538,7 +542,7 @@ void dense_product(const Context& c, const cx_t<R>* H, const cx_t<Rin>* X, cx_t<
     }
     xt.reserve(static_cast<size_t>(N) * kVec);
     yp.reserve(room);
-    dense_product_into<Rin, R, Rout>(N, H, X, Y, nvec, s, xt.p, yp.p, 64);
+    dense_product_into<Rin, R, Rout>(N, H, X, Y, nvec, s, xt.p, yp.p, 64, c.take_product_stamp());
 }
 
 }  // namespace
@@ -554,7 +558,7 @@ void launch_matvec64_scratch(const Context& c, const double2* X, double2* Y, int
     // kernels and, when they fit, the same splits as the allocating product)
     const int max_splits = static_cast<int>(std::min<int64_t>(64, scratch_elems / (N * kVec) - 1));
     if (max_splits < 1) throw Error(XATU_ERR_INVALID_ARGUMENT, "scratch too small for the product");
-    dense_product_into<double, double, double>(N, c.d_H64.p, X, Y, nvec, s, scratch, scratch + N * kVec, max_splits);
+    dense_product_into<double, double, double>(N, c.d_H64.p, X, Y, nvec, s, scratch, scratch + N * kVec, max_splits, nullptr);
 }
 
 // Product with the FP32 matrix: on the FP16 matrix cores with split operands where the
@@ -569,13 +573,13 @@ void launch_matvec32(Context& c, const double2* X, double2* Y, int nvec, hipStre
     dense_product<double, float, double>(c, c.d_H32.p, X, Y, nvec, s, c.s_xt32, c.s_yp32);
 }
 
-void launch_stage_vectors(const double2* X, int64_t N, int nvec, double2* Xt, hipStream_t s) {
+void launch_stage_vectors(const double2* X, int64_t N, int nvec, double2* Xt, unsigned long long* stamp, hipStream_t s) {
     hipLaunchKernelGGL((stage_vectors_kernel<double, double, kVec>), dim3((N * kVec + 255) / 256), dim3(256), 0, s, X, N,
-                       nvec, Xt);
+                       nvec, Xt, stamp);
 }
-void launch_stage_vectors(const double2* X, int64_t N, int nvec, float2* Xt, hipStream_t s) {
+void launch_stage_vectors(const double2* X, int64_t N, int nvec, float2* Xt, unsigned long long* stamp, hipStream_t s) {
     hipLaunchKernelGGL((stage_vectors_kernel<double, float, kVec>), dim3((N * kVec + 255) / 256), dim3(256), 0, s, X, N,
-                       nvec, Xt);
+                       nvec, Xt, stamp);
 }
 void launch_reduce_partials(const double2* Yp, int64_t N, int nvec, int splits, double2* Y, hipStream_t s) {
     hipLaunchKernelGGL((reduce_product_kernel<double, double, kVec>), dim3((N * kVec + 255) / 256), dim3(256), 0, s, Yp, N, nvec,

@@ -253,10 +253,7 @@ __global__ __launch_bounds__(64 * kStepMaxBlock / kCols) void whiten_apply_kerne
                 if (j < jn) a.T[i + static_cast<int64_t>(j0 + j) * a.N] = acc[j];
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.product_stamp[0] = device_clock();
 }
-
-__global__ void stamp_kernel(unsigned long long* stamp) { *stamp = device_clock(); }
 
 unsigned step_blocks(int64_t N) { return static_cast<unsigned>((N + kRows - 1) / kRows); }
 unsigned step_threads(int b) { return 64 * ((b + kCols - 1) / kCols); }
@@ -279,11 +276,6 @@ void launch_whiten(const WhitenArgs& a, hipStream_t s) {
     // without a block only the report's workgroup
     hipLaunchKernelGGL(whiten_apply_kernel, dim3(a.nb > 0 ? step_blocks(a.N) + 1 : 1), dim3(step_threads(std::max(a.nb, 1))),
                        0, s, a, a.S);
-    XATU_HIP(hipGetLastError());
-}
-
-void launch_stamp(unsigned long long* stamp, hipStream_t s) {
-    hipLaunchKernelGGL(stamp_kernel, dim3(1), dim3(1), 0, s, stamp);
     XATU_HIP(hipGetLastError());
 }
 

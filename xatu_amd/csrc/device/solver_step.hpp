@@ -7,8 +7,9 @@ namespace xatu_dev {
 
 constexpr int kStepMaxBlock = 32;  // columns of a Ritz or correction block
 
-// Device clock values: start of the Rayleigh-Ritz kernel, of the Ritz block, of the whitening;
-// end of the whitening product (start of the operator's), start of the projections after it.
+// Device clock values: start of the Rayleigh-Ritz kernel, of the Ritz block, of the whitening, of the
+// operator's product (left by its first kernel: the host waits for the iteration's report before it
+// launches the product) and of the projections after it.
 enum { kStampEigen, kStampRitz, kStampWhiten, kStampProduct, kStampExtend, kStamps };
 
 // Report of an iteration in mapped host memory: Ritz values, squared residual norms, stamps, whether
@@ -45,13 +46,11 @@ struct WhitenArgs {
     int* flag;
     const double *theta, *norm2;
     unsigned long long* stamps;
-    unsigned long long* product_stamp;
     StepReport* host;
     unsigned long long sequence;
 };
 // Whitening of the block and its application; the report to the host.
 void launch_whiten(const WhitenArgs& a, hipStream_t s);
-void launch_stamp(unsigned long long* stamp, hipStream_t s);
 
 // P = A^H B (m x n), and norm2[j] = the sum of column j's residual partials (n = 0: these only)
 void launch_gram_norms(Context& c, const double2* A, int lda, const double2* B, int ldb, int m, int n, double2* P, int ldp,

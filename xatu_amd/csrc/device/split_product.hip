@@ -87,8 +87,9 @@ __global__ void operator_bounds_kernel(const double2* __restrict__ ft, int64_t n
 
 // partial[n kMaxChunks + chunk] = max |Re|, |Im| of X[rows of chunk, n]; grid (chunks, 32).
 __global__ void column_max_kernel(const double2* __restrict__ X, int64_t N, int nvec, int64_t rows,
-                                  float* __restrict__ partial) {
+                                  float* __restrict__ partial, unsigned long long* __restrict__ stamp) {
     __shared__ double red[256];
+    if (stamp && blockIdx.x + blockIdx.y == 0 && threadIdx.x == 0) *stamp = wall_clock64();
     const int chunk = blockIdx.x, n = blockIdx.y;
     double m = 0.0;
     if (n < nvec) {
@@ -967,7 +968,8 @@ void launch_matvec_split16(Context& c, const double2* X, double2* Y, int nvec, h
     for (int v0 = 0; v0 < nvec; v0 += kVec) {
         const int nv = std::min(kVec, nvec - v0);
         const double2* Xb = X + static_cast<int64_t>(v0) * N;
-        hipLaunchKernelGGL(column_max_kernel, dim3(chunks, kVec), dim3(256), 0, s, Xb, N, nv, rows, c.s_colmax.p);
+        hipLaunchKernelGGL(column_max_kernel, dim3(chunks, kVec), dim3(256), 0, s, Xb, N, nv, rows, c.s_colmax.p,
+                           c.take_product_stamp());
         hipLaunchKernelGGL(vector_scale_kernel, dim3(1), dim3(64), 0, s, c.s_colmax.p, chunks, sH, c.s_xscale.p,
                            c.s_xinv.p);
         hipLaunchKernelGGL(stage_split_kernel, dim3((nstage + 255) / 256), dim3(256), 0, s, Xb, N, nv, nsteps, ngroups,

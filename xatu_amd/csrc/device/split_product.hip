@@ -33,13 +33,12 @@
 // (32 zero entries of padding after the matrix, zeroed heads of the unbuilt columns).
 #include <algorithm>
 #include <cmath>
-#include <functional>
-#include <queue>
 #include <vector>
 
 #include "context.hpp"
 #include "cplx.hpp"
 #include "mfma.hpp"
+#include "split_items.hpp"
 
 namespace xatu_dev {
 
@@ -860,59 +859,17 @@ void split_product_scale(Context& c) {
     if (c.h16_scale > 0.0f) lay_out_items(c);
 }
 
-// Work items (row block, column chunk) of the split product, the longest first, laid out once
-// per matrix dimension. The chunk is the multiple of the row block with the shortest schedule
-// of its items on the CUs (one workgroup each; about 22 us per 256 x 256 block and 8 us to
-// start and end an item, both measured) plus the direct partial sums an item writes and the
-// reduction reads back: at small N short chunks, so that every CU has work (a fixed 4096
-// left 84 items, the longest 16 blocks, at N = 9216), at N = 36864 chunks of 1536. Products
-// with staging and reduction, 4096 -> now: N = 2304 217 -> 58 us, 5184 361 -> 67, 9216
-// 387 -> 136, 14400 414 -> 280, 20736 517 -> 517, 36864 1572 -> 1571.
+// Work items of the split product (split_items.hpp), laid out once per matrix dimension.
 static void lay_out_items(Context& c) {
     const int64_t N = c.N;
     if (c.herm_n == N && c.herm_items > 0) return;
-    const int64_t B = (N + kHermRows - 1) / kHermRows;
-    constexpr int kCus = 256, kMaxItems = 2048;
-    struct Item {
-        int2 at;
-        int64_t len;
-    };
-    std::vector<Item> best;
-    double best_us = 1e300;
-    for (int blocks : {1, 2, 3, 4, 6, 8, 12, 16}) {
-        const int64_t chunk = static_cast<int64_t>(blocks) * kHermRows;
-        // skip layouts of far more items than CUs while a longer chunk remains
-        if (blocks < 16 && B * B / (2 * blocks) > kMaxItems) continue;
-        std::vector<Item> it;
-        for (int64_t ch = 0; ch * chunk < N; ++ch)
-            for (int64_t b = 0; b < B; ++b) {
-                const int64_t rb0 = b * kHermRows, cb = ch * chunk;
-                if (rb0 >= cb + chunk) continue;
-                it.push_back({make_int2(static_cast<int>(b), static_cast<int>(ch)), std::min(N, cb + chunk) - std::max(rb0, cb)});
-            }
-        std::stable_sort(it.begin(), it.end(), [](const Item& x, const Item& y) { return x.len > y.len; });
-        std::priority_queue<double, std::vector<double>, std::greater<double>> cu(std::greater<double>(),
-                                                                                 std::vector<double>(kCus, 0.0));
-        double last = 0.0;
-        for (const Item& i : it) {
-            const double t = cu.top() + 8.0 + 22.0 * static_cast<double>(i.len) / kHermRows;
-            cu.pop();
-            cu.push(t);
-            last = std::max(last, t);
-        }
-        // microseconds for the direct partial sums, 64 KB per item written and read
-        const double us = last + it.size() * 2.0 * kHermRows * kVec * sizeof(float2) / 5e6;
-        if (us < best_us) {
-            best_us = us;
-            best.swap(it);
-            c.herm_chunk = static_cast<int>(chunk);
-        }
-    }
-    std::vector<int2> sorted(best.size());
-    for (size_t i = 0; i < best.size(); ++i) sorted[i] = best[i].at;
-    c.d_herm_items.alloc(sorted.size());
-    XATU_HIP(hipMemcpy(c.d_herm_items.p, sorted.data(), sorted.size() * sizeof(int2), hipMemcpyHostToDevice));
-    c.herm_items = static_cast<int>(sorted.size());
+    const SplitLayout l = split_layout(N, kHermRows, 2.0 * kHermRows * kVec * sizeof(float2));
+    std::vector<int2> at(l.items.size());
+    for (size_t i = 0; i < at.size(); ++i) at[i] = make_int2(l.items[i].block, l.items[i].chunk);
+    c.d_herm_items.alloc(at.size());
+    XATU_HIP(hipMemcpy(c.d_herm_items.p, at.data(), at.size() * sizeof(int2), hipMemcpyHostToDevice));
+    c.herm_items = static_cast<int>(at.size());
+    c.herm_chunk = static_cast<int>(l.chunk);
     c.herm_n = N;
 }
 

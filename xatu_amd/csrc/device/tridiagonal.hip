@@ -117,7 +117,45 @@ __global__ __launch_bounds__(64 * WAVES) void tridiagonal_step_kernel(double2* _
     norm = 0.0;
 #pragma unroll
     for (int k = 0; k < WAVES; ++k) norm += s_red[1][k][0];
-    const double2 alpha = s_alpha;
+    double2 alpha = s_alpha;
+    double back = 1.0;  // from the units of the reflector's scalars to the matrix's
+    const double sum = alpha.x * alpha.x + alpha.y * alpha.y + norm;
+    if (__builtin_expect(!(sum > 1e-280 && sum < 1e280), 0)) {
+        // squares that left the normal numbers (or nothing but zeros): the column in units of a power of two
+        // near its largest entry. The whole workgroup comes here or none of it.
+        double most = fmax(fabs(alpha.x), fabs(alpha.y));
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int r = threadIdx.x + kThreads * k;
+            if (r >= j + 2 && r < n) most = fmax(most, fmax(fabs(a[k].x), fabs(a[k].y)));
+        }
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) most = fmax(most, __shfl_xor(most, d));
+        if (lane == 0) s_red[0][wave][0] = most;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < WAVES; ++k) most = fmax(most, s_red[0][k][0]);
+        double unit = 1.0;
+        if (most > 0.0) {
+            const int ex = max(-1000, min(1000, ilogb(most)));
+            unit = ldexp(1.0, -ex);
+            back = ldexp(1.0, ex);
+        }
+        norm = 0.0;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int r = threadIdx.x + kThreads * k;
+            a[k] = mk(a[k].x * unit, a[k].y * unit);
+            if (r >= j + 2 && r < n) norm += a[k].x * a[k].x + a[k].y * a[k].y;
+        }
+        norm = wave_sum(norm);
+        if (lane == 0) s_red[1][wave][0] = norm;
+        __syncthreads();
+        norm = 0.0;
+#pragma unroll
+        for (int k = 0; k < WAVES; ++k) norm += s_red[1][k][0];
+        alpha = mk(alpha.x * unit, alpha.y * unit);
+    }
     double beta = alpha.x;
     double2 t = mk(0.0, 0.0), scale = mk(0.0, 0.0);
     if (norm > 0.0 || alpha.y != 0.0) {
@@ -139,7 +177,7 @@ __global__ __launch_bounds__(64 * WAVES) void tridiagonal_step_kernel(double2* _
     }
     if (last && threadIdx.x == 0) {
         tau[j] = t;
-        E[j] = beta;
+        E[j] = beta * back;
     }
     __syncthreads();
     if (!mine) return;

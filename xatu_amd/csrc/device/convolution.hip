@@ -1127,18 +1127,23 @@ bool conv_rows_available(Context& c) {
 // with S_ab(q) the pair densities of conv_pair_density. Their transform is the power spectrum of
 // z, so Shat_p(R) = sum_{al in a, be in b} |Z_{al be}(-R)|^2 + sum_{al in b, be in a} |Z_{al be}(R)|^2
 // (a = b: one sum, at R), Z the forward transform of z on the window that holds every cell.
-// shat[(s npairs + p) nR + R] for the ns <= 32 states of psi (N x ns).
+// shat[(s npairs + p) nR + R] for the ns <= 32 states of psi (N x ns), taken in passes that keep the buffer
+// within kRowsBufferBytes.
 void conv_cell_density(Context& c, const double2* psi, int ns, double* shat) {
     ensure_conv(c);
     ConvState& cs = *c.conv;
     ConvBuffers<double> b(cs);
     hipStream_t s = c.stream;
     const int npairs = c.lat.natoms * (c.lat.natoms + 1) / 2;
-    conv_bands_in<double>(c, b, psi, ns, s);
-    conv_rows_forward<double>(c, cs, b, ns, false, s);
-    hipLaunchKernelGGL(cell_power_kernel, dim3((c.nR + 255) / 256, npairs, ns), dim3(256), 0, s, c.lat, cs.W, cs.w0,
-                       c.d_cells.p, c.nR, npairs, ns, b.G.p, shat);
-    XATU_HIP(hipGetLastError());
+    const int step = rows_vectors<double>(c, cs, ns);
+    for (int v0 = 0; v0 < ns; v0 += step) {
+        const int nv = std::min(step, ns - v0);
+        conv_bands_in<double>(c, b, psi + static_cast<int64_t>(v0) * c.N, nv, s);
+        conv_rows_forward<double>(c, cs, b, nv, false, s);
+        hipLaunchKernelGGL(cell_power_kernel, dim3((c.nR + 255) / 256, npairs, nv), dim3(256), 0, s, c.lat, cs.W, cs.w0,
+                           c.d_cells.p, c.nR, npairs, nv, b.G.p, shat + static_cast<size_t>(v0) * npairs * c.nR);
+        XATU_HIP(hipGetLastError());
+    }
 }
 
 // Adjoint of the assembly with respect to the band vectors by the same transforms: with

@@ -72,8 +72,9 @@ struct DevBuf {
 
 // Owning pinned host allocation, grown on demand: small transfers to and from it need no
 // staging copy. reserve_mapped: fine-grained (coherent) memory mapped into the device's
-// address space at dev, which kernels store into directly (visible to the host once the
-// kernel has completed, with no copy).
+// address space at dev, which kernels store into directly, with no copy: all of it is there once the
+// kernel has completed; what the host reads while it runs needs a check of its own, as each value of
+// the solver's report has (solver_step.hpp).
 template <typename T>
 struct HostBuf {
     T* p = nullptr;

@@ -29,7 +29,7 @@
 // (A and P enter F conjugated, so their derivative is -1/2 p dF/d conj; B and Q enter
 // holomorphically, so theirs is -1/2 conj(p dF/dB)). Where the operator is a convolution on a
 // 2-D mesh with row and column transforms the same sums come from those (conv_band_adjoint);
-// otherwise (1-D and 3-D meshes, the reciprocal-space table, other mesh sides) every
+// otherwise (1-D and 3-D meshes, the reciprocal-space table, other mesh sides, a state or two on a small mesh) every
 // canonical pair is handled by one thread, which adds its contributions to the four
 // coefficient vectors with hardware FP64 atomics. Conduction vectors belong to the k+Q stack, valence vectors
 // to the k stack, as in the assembly.
@@ -343,6 +343,17 @@ PairsLauncher pairs_launcher(const Context& c) {
     return f;
 }
 
+// One or two states on a small mesh: the ten launches of the transforms take longer than a pass over the pairs per
+// state. One state, 2 orbitals, 8 x 8: 54 us by pairs, 83 by the transforms, equal at 17 x 17; 8 orbitals 63 and 115,
+// equal at 14 x 14; 12 orbitals and four bands 98 and 136, equal at 10 x 10; 36 orbitals and four bands 2 x 2 88 and 127, equal
+// at 3 x 3; with six bands 205 and 132. Two states, 8 orbitals, 2 x 2: 89 and 107, equal at 4 x 4. From three
+// states on the transforms always. The line lies below the equal points: the transforms' sums do not depend on the order
+// of atomic adds.
+bool pairs_are_faster(const Context& c, int nstates) {
+    const int64_t size = static_cast<int64_t>(c.nk) * c.lat.norb;
+    return c.lat.norb * c.nc * c.nv <= 144 && size <= (nstates == 1 ? 512 : nstates == 2 ? 32 : 0);
+}
+
 // w[((n 2 + stack) nk + k) nb + b]: dE/dE_c(k+Q) = sum_v |psi|^2, dE/dE_v(k) = -sum_c |psi|^2, zero for
 // the other columns of each stack. grid (ceil(nk / 256), states)
 __global__ void band_energy_kernel(int nk, int nv, int nc, const double2* __restrict__ psi, int64_t N,
@@ -375,27 +386,26 @@ void band_gradients(Context& c, int nstates, const double2* d_vec, double* w_out
     const size_t stack = static_cast<size_t>(c.lat.norb) * c.nb * c.nk;  // complex entries per stack
     const int64_t N = c.N;
     hipStream_t s = c.stream;
-    DevBuf<double> w;
-    w.alloc(static_cast<size_t>(nstates) * 2 * c.nb * c.nk);
-    hipLaunchKernelGGL(band_energy_kernel, dim3((c.nk + 255) / 256, nstates), dim3(256), 0, s, c.nk, c.nv, c.nc, d_vec, N,
-                       w.p);
-    XATU_HIP(hipGetLastError());
-    const bool direct = c.lat.ndim == 2 && !c.lat.recip && conv_rows_available(c);
+    const bool direct = c.lat.ndim == 2 && !c.lat.recip && !pairs_are_faster(c, nstates) && conv_rows_available(c);
     const int step = direct ? std::min(nstates, kBandStates) : 1;
-    DevBuf<double2> g;
-    g.alloc(2 * stack * step);
+    const size_t nw = static_cast<size_t>(nstates) * 2 * c.nb * c.nk;
+    DevBuf<double2> g;  // and the energies' derivatives, a pair in an entry
+    g.alloc(2 * stack * step + (nw + 1) / 2);
+    double* w = reinterpret_cast<double*>(g.p + 2 * stack * step);
+    hipLaunchKernelGGL(band_energy_kernel, dim3((c.nk + 255) / 256, nstates), dim3(256), 0, s, c.nk, c.nv, c.nc, d_vec, N, w);
+    XATU_HIP(hipGetLastError());
     for (int st = 0; st < nstates; st += step) {
         const int ns = std::min(step, nstates - st);
         const double2* psi = d_vec + static_cast<int64_t>(st) * N;
         if (direct) {
             conv_band_adjoint(c, psi, ns, g.p);
         } else {
-            XATU_HIP(hipMemsetAsync(g.p, 0, g.bytes(), s));
+            XATU_HIP(hipMemsetAsync(g.p, 0, 2 * stack * sizeof(double2), s));
             pairs(c, psi, g.p, g.p + stack, s);
         }
         XATU_HIP(hipMemcpyAsync(g_out + 4 * stack * st, g.p, 2 * stack * ns * sizeof(double2), hipMemcpyDeviceToHost, s));
     }
-    XATU_HIP(hipMemcpyAsync(w_out, w.p, w.bytes(), hipMemcpyDeviceToHost, s));
+    XATU_HIP(hipMemcpyAsync(w_out, w, nw * sizeof(double), hipMemcpyDeviceToHost, s));
     XATU_HIP(hipStreamSynchronize(s));
 }
 

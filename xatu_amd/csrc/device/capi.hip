@@ -433,12 +433,11 @@ int xatu_fourier_sums(xatu_ctx* ctx, const xatu_interaction* inter) {
         c.h_cells = truncate_supercell(c.lat.bravais, c.lat.ndim, inter->ncell, c.a1norm * inter->cutoff);
         c.nR = static_cast<int>(c.h_cells.size() / c.lat.ndim);
         if (c.nR == 0) throw Error(XATU_ERR_INVALID_ARGUMENT, "no lattice vectors inside the cutoff");
-        std::vector<int> padded(static_cast<size_t>(c.nR) * 3, 0);
+        // the cells, and in two dimensions as rows of cells behind them
+        c.rows_at = (static_cast<size_t>(c.nR) * 3 + 3) / 4 * 4;
+        std::vector<int> padded(c.rows_at, 0);
         for (int r = 0; r < c.nR; ++r)
             for (int j = 0; j < c.lat.ndim; ++j) padded[3 * r + j] = c.h_cells[r * c.lat.ndim + j];
-        c.d_cells.alloc(padded.size());
-        XATU_HIP(hipMemcpyAsync(c.d_cells.p, padded.data(), padded.size() * sizeof(int), hipMemcpyHostToDevice,
-                                c.stream));
         std::vector<int4> rows;
         if (c.lat.ndim == 2) {
             // consecutive cells of one second coefficient, the first one counting up
@@ -447,9 +446,11 @@ int xatu_fourier_sums(xatu_ctx* ctx, const xatu_interaction* inter) {
                 if (!rows.empty() && rows.back().x == m2 && rows.back().y + rows.back().w == m1) ++rows.back().w;
                 else rows.push_back(make_int4(m2, m1, r, 1));
             }
-            c.d_rows.reserve(rows.size());
-            XATU_HIP(hipMemcpyAsync(c.d_rows.p, rows.data(), rows.size() * sizeof(int4), hipMemcpyHostToDevice, c.stream));
         }
+        for (const int4& r : rows) padded.insert(padded.end(), {r.x, r.y, r.z, r.w});
+        c.d_cells.alloc(padded.size());
+        XATU_HIP(hipMemcpyAsync(c.d_cells.p, padded.data(), padded.size() * sizeof(int), hipMemcpyHostToDevice,
+                                c.stream));
         c.n_rows = static_cast<int>(rows.size());
         const int npairs = c.lat.natoms * (c.lat.natoms + 1) / 2;
         const int na2 = c.lat.natoms * c.lat.natoms;
@@ -459,12 +460,11 @@ int xatu_fourier_sums(xatu_ctx* ctx, const xatu_interaction* inter) {
         c.d_ftq.alloc(na2);
         EventTimer ev(c.stream);
         ev.start();
-        launch_potential_table(c, c.pot_d, c.d_vtab.p, c.stream);
-        launch_twiddles(c.lat.mesh_n, c.d_twiddle.p, c.stream);
+        launch_potential_table(c, c.pot_d, c.d_vtab.p, c.d_twiddle.p, c.stream);
         launch_fourier_mesh(c, c.stream);
         if (inter->exchange) {
             c.d_vtabx.alloc(static_cast<size_t>(npairs) * c.nR);
-            launch_potential_table(c, c.pot_x, c.d_vtabx.p, c.stream);
+            launch_potential_table(c, c.pot_x, c.d_vtabx.p, nullptr, c.stream);
             launch_fourier_q(c, c.stream);
         } else {
             XATU_HIP(hipMemsetAsync(c.d_ftq.p, 0, na2 * sizeof(double2), c.stream));

@@ -185,9 +185,10 @@ struct Context {
     PotDesc pot_d{}, pot_x{};
     int nR = 0;
     std::vector<int> h_cells;   // nR x ndim integer coefficients
-    DevBuf<int> d_cells;        // nR x 3 (padded)
+    DevBuf<int> d_cells;        // nR x 3 (padded), then the rows from rows_at on
     int n_rows = 0;
-    DevBuf<int4> d_rows;        // 2-D: the cells as rows {m_2, first m_1, first cell, count}
+    size_t rows_at = 0;         // 2-D: the cells as rows {m_2, first m_1, first cell, count}
+    const int4* rows() const { return reinterpret_cast<const int4*>(d_cells.p + rows_at); }
     DevBuf<double2> d_rowsum;   // sums along the rows and their remainders
     DevBuf<double> d_vtab;      // npairs x nR direct potential table
     DevBuf<double> d_vtabx;     // npairs x nR exchange potential table
@@ -307,8 +308,8 @@ struct EventTimer {
 };
 
 // Kernel launchers implemented in the .hip translation units.
-void launch_potential_table(const Context& c, const PotDesc& pot, double* out, hipStream_t s);
-void launch_twiddles(int mesh_n, double2* out, hipStream_t s);
+// twiddle: the table of 2 mesh_n roots of unity, written by the same launch (null: not)
+void launch_potential_table(const Context& c, const PotDesc& pot, double* out, double2* twiddle, hipStream_t s);
 void launch_fourier_mesh(Context& c, hipStream_t s);
 void launch_fourier_q(const Context& c, hipStream_t s);
 // Reciprocal-mode tables: M_ab(q) over the raw mesh differences into d_ft and, with

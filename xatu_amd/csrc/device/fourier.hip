@@ -32,11 +32,21 @@ constexpr int kFtPairs = 10;  // pairs handled per workgroup (natoms <= 4 -> one
 constexpr int kRowThreads = 128;
 constexpr size_t kRowSums = size_t(1) << 22;  // row sums (32 bytes each) held at a time
 
+// The potential per (pair, R), and in the workgroups after the pairs tw[p] = e^{i pi p / mesh_n}, p < 2 mesh_n: a
+// launch of its own for these roots costs as much as the whole table at small sizes.
+// grid: (ceil(max(nR, 2 mesh_n) / 256), npairs + (tw ? 1 : 0)); block: 256
 __global__ void potential_table_kernel(LatticeDesc lat, PotDesc pot, const int* __restrict__ cells, int nR,
-                                       int npairs, double* __restrict__ out) {
+                                       int npairs, double* __restrict__ out, double2* __restrict__ tw) {
     const int R = blockIdx.x * blockDim.x + threadIdx.x;
     const int p = blockIdx.y;
-    if (R >= nR || p >= npairs) return;
+    if (p == npairs) {
+        if (R >= 2 * lat.mesh_n) return;
+        double s, c;
+        sincospi(static_cast<double>(R) / static_cast<double>(lat.mesh_n), &s, &c);
+        tw[R] = make_double2(c, s);
+        return;
+    }
+    if (R >= nR) return;
     // pair index -> (a, b), a <= b, enumerated row by row
     int a = 0, rem = p;
     while (rem >= lat.natoms - a) {
@@ -45,14 +55,6 @@ __global__ void potential_table_kernel(LatticeDesc lat, PotDesc pot, const int* 
     }
     const int b = a + rem;
     out[static_cast<size_t>(p) * nR + R] = potential(cell_distance(lat, cells + 3 * R, a, b), pot);
-}
-
-__global__ void twiddle_kernel(int n, double2* __restrict__ tw) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= 2 * n) return;
-    double s, c;
-    sincospi(static_cast<double>(p) / static_cast<double>(n), &s, &c);
-    tw[p] = make_double2(c, s);
 }
 
 __device__ inline void neumaier_add(double& sum, double& comp, double x) {
@@ -367,15 +369,10 @@ void launch_reciprocal_table(const Context& c, const double* d_gvec, int ng, dou
     }
 }
 
-void launch_potential_table(const Context& c, const PotDesc& pot, double* out, hipStream_t s) {
+void launch_potential_table(const Context& c, const PotDesc& pot, double* out, double2* twiddle, hipStream_t s) {
     const int npairs = c.lat.natoms * (c.lat.natoms + 1) / 2;
-    dim3 grid((c.nR + 255) / 256, npairs);
-    hipLaunchKernelGGL(potential_table_kernel, grid, dim3(256), 0, s, c.lat, pot, c.d_cells.p, c.nR, npairs, out);
-    XATU_HIP(hipGetLastError());
-}
-
-void launch_twiddles(int mesh_n, double2* out, hipStream_t s) {
-    hipLaunchKernelGGL(twiddle_kernel, dim3((2 * mesh_n + 255) / 256), dim3(256), 0, s, mesh_n, out);
+    dim3 grid((std::max(c.nR, 2 * c.lat.mesh_n) + 255) / 256, npairs + (twiddle ? 1 : 0));
+    hipLaunchKernelGGL(potential_table_kernel, grid, dim3(256), 0, s, c.lat, pot, c.d_cells.p, c.nR, npairs, out, twiddle);
     XATU_HIP(hipGetLastError());
 }
 
@@ -393,10 +390,10 @@ void launch_fourier_mesh(Context& c, hipStream_t s) {
         for (int p0 = 0; p0 < npairs; p0 += chunk) {
             const unsigned np = std::min(chunk, npairs - p0);
             hipLaunchKernelGGL(fourier_rows_kernel, dim3(np, c.n_rows, g), dim3(kRowThreads), 0, s, n, c.n_rows,
-                               c.d_rows.p, c.nR, c.d_vtab.p + static_cast<size_t>(p0) * c.nR, c.d_twiddle.p,
+                               c.rows(), c.nR, c.d_vtab.p + static_cast<size_t>(p0) * c.nR, c.d_twiddle.p,
                                c.d_rowsum.p, lo);
             hipLaunchKernelGGL(fourier_mesh2_kernel, dim3(np, n, g), dim3(kRowThreads), 0, s, c.lat, p0, c.n_rows,
-                               c.d_rows.p, c.d_rowsum.p, lo, c.d_twiddle.p, inv_total, c.d_ft.p);
+                               c.rows(), c.d_rowsum.p, lo, c.d_twiddle.p, inv_total, c.d_ft.p);
         }
         XATU_HIP(hipGetLastError());
         return;

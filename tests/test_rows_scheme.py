@@ -15,7 +15,7 @@ PAIRS = [(int(a), int(b)) for a, b in re.findall(r"X\((\d+), (\d+)\)", SOURCE)]
 
 def test_pairs():
     sides = [a * b for a, b in PAIRS]
-    assert len(sides) == len(set(sides)) == 99 and min(sides) == 2 and max(sides) <= 128
+    assert len(sides) == len(set(sides)) == 100 and min(sides) == 1 and max(sides) <= 128
     for a, b in PAIRS:
         assert a <= b and a in LENGTHS and b in LENGTHS
         assert b <= 31 or a == 1

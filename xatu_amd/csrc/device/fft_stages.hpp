@@ -2,7 +2,7 @@
 // convolution product's row and column transforms. A mesh side n = A B with A and B among these
 // lengths, or 37 and 41 themselves, is transformed in two steps: x[B j2 + s] -> A-point DFTs over j2
 // (one per s), the twiddles e^{-2 pi i s k1 / n}, B-point DFTs over s, giving X[k1 + A k2]
-// (a prime B much longer than A spread over lanes, conv_rows.hpp). That covers 99 of the 127 sides up to
+// (a prime B much longer than A spread over lanes, conv_rows.hpp). That covers 100 of the 128 sides up to
 // 128, all but 125 and those with a longer prime factor; pairs of factors 2, 3 and 5 alone cover 36, and
 // the others took the library's transforms over whole meshes (products of 16 vectors, 12 orbitals, with
 // their copies from and to the host: FP64 23 x 23 0.45 -> 0.30 ms, 49 x 49 0.96 -> 0.69, 77 x 77 1.72 -> 1.36,
@@ -18,15 +18,15 @@ constexpr int kFftMaxSide = 128;  // largest mesh side of the two-step transform
 
 // Factor pairs (A, B), A <= B, of the supported mesh sides.
 #define XATU_FFT_PAIRS(X)                                                                                     \
-    X(1, 2) X(1, 3) X(1, 5) X(1, 7) X(1, 11) X(1, 13) X(1, 17) X(1, 19) X(1, 23) X(1, 29) X(1, 31) X(1, 37)   \
-    X(1, 41) X(2, 2) X(2, 3) X(2, 4) X(2, 5) X(2, 7) X(2, 11) X(2, 13) X(2, 17) X(2, 19) X(2, 23) X(2, 29)    \
-    X(2, 31) X(3, 3) X(3, 4) X(3, 5) X(3, 6) X(3, 7) X(3, 9) X(3, 11) X(3, 13) X(3, 17) X(3, 19) X(3, 23)     \
-    X(3, 29) X(3, 31) X(4, 4) X(4, 5) X(4, 6) X(4, 7) X(4, 8) X(4, 11) X(4, 13) X(4, 17) X(4, 19) X(4, 23)    \
-    X(4, 29) X(4, 31) X(5, 5) X(5, 6) X(5, 7) X(5, 8) X(5, 9) X(5, 10) X(5, 11) X(5, 13) X(5, 15) X(5, 17)    \
-    X(5, 19) X(5, 23) X(6, 6) X(6, 7) X(6, 8) X(6, 9) X(6, 10) X(6, 11) X(6, 13) X(6, 17) X(6, 19) X(7, 7)    \
-    X(7, 8) X(7, 9) X(7, 10) X(7, 11) X(7, 12) X(7, 13) X(7, 14) X(7, 15) X(7, 17) X(8, 8) X(8, 9) X(8, 10)   \
-    X(8, 11) X(8, 12) X(8, 13) X(8, 14) X(8, 16) X(9, 9) X(9, 10) X(9, 11) X(9, 12) X(9, 13) X(9, 14)         \
-    X(10, 10) X(10, 11) X(10, 12) X(11, 11)
+    X(1, 1) X(1, 2) X(1, 3) X(1, 5) X(1, 7) X(1, 11) X(1, 13) X(1, 17) X(1, 19) X(1, 23) X(1, 29) X(1, 31)    \
+    X(1, 37) X(1, 41) X(2, 2) X(2, 3) X(2, 4) X(2, 5) X(2, 7) X(2, 11) X(2, 13) X(2, 17) X(2, 19) X(2, 23)    \
+    X(2, 29) X(2, 31) X(3, 3) X(3, 4) X(3, 5) X(3, 6) X(3, 7) X(3, 9) X(3, 11) X(3, 13) X(3, 17) X(3, 19)     \
+    X(3, 23) X(3, 29) X(3, 31) X(4, 4) X(4, 5) X(4, 6) X(4, 7) X(4, 8) X(4, 11) X(4, 13) X(4, 17) X(4, 19)    \
+    X(4, 23) X(4, 29) X(4, 31) X(5, 5) X(5, 6) X(5, 7) X(5, 8) X(5, 9) X(5, 10) X(5, 11) X(5, 13) X(5, 15)    \
+    X(5, 17) X(5, 19) X(5, 23) X(6, 6) X(6, 7) X(6, 8) X(6, 9) X(6, 10) X(6, 11) X(6, 13) X(6, 17) X(6, 19)   \
+    X(7, 7) X(7, 8) X(7, 9) X(7, 10) X(7, 11) X(7, 12) X(7, 13) X(7, 14) X(7, 15) X(7, 17) X(8, 8) X(8, 9)    \
+    X(8, 10) X(8, 11) X(8, 12) X(8, 13) X(8, 14) X(8, 16) X(9, 9) X(9, 10) X(9, 11) X(9, 12) X(9, 13)         \
+    X(9, 14) X(10, 10) X(10, 11) X(10, 12) X(11, 11)
 
 // (A, B) of a mesh side; A = 0: the side is not one of the supported products.
 inline void fft_factors(int n, int& A, int& B) {
